@@ -28,11 +28,12 @@ struct MeshView {
 // Patch work lists.  Bucket b holds patches whose row count m = q*|set|
 // fits rows_of_bucket(b); larger sets, up to BIG_MMAX rows, go to the big
 // list.
-enum { NBUCKET = 6 };
+enum { NBUCKET = 7 };
+constexpr int NSMALL = 3;  // the buckets k_qr_small fits (up to 32 rows)
 constexpr int BIG_MMAX = 512;
 __host__ __device__ inline int bucket_rows(int b)
 {
-  const int r[NBUCKET] = {16, 32, 64, 96, 128, 192};
+  const int r[NBUCKET] = {16, 24, 32, 64, 96, 128, 192};
   return r[b];
 }
 __host__ __device__ inline int bucket_of(int m)
@@ -52,7 +53,11 @@ enum {
 };
 
 struct Lists {
-  int32_t* items[NBUCKET];   // regular: patch ids; expanded: item ids
+  // FP64 form: the regular patches of each bucket, one after the other in
+  // one array (the mesh's set sizes give the bucket sizes beforehand); fast
+  // forms: the refits of each bucket (list 0 that same array, the others the
+  // xitems the fast forms do not use)
+  int32_t* items[NBUCKET];
   int32_t* count;            // [NBUCKET] regular, [NBUCKET] expanded, [1] expand-queue
   int32_t* xitems[NBUCKET];
   int32_t* xq;               // patches queued for the exact rank test /
@@ -83,7 +88,7 @@ struct Lists {
 struct LaunchShape {
   int fast_threads = 256;   // k_fast block size (64, 128 or 256)
   int fast_blocks = 8192;   // k_fast persistent grid cap
-  int exact_blocks = 8192;  // k_exact_fit grid per bucket (a quarter for 192 rows)
+  int exact_blocks = 8192;  // grid cap of the exact fits, per bucket
   int expand_blocks = 4096; // k_expand grid
   int tile_blocks = 8192;   // k_tile persistent grid cap; 0: the regular pass
                             // runs thread per patch (k_fast) instead
@@ -175,9 +180,17 @@ int launch_csr(const MeshView& m, int dim, int32_t* off, int32_t* idx,
 int launch_scan_i32(int32_t* a, int64_t n, int32_t* work, hipStream_t s);
 int launch_copy_i32(int32_t* dst, const int32_t* src, int64_t n, hipStream_t s);
 int launch_classify(const FitArgs& a, int nterms, hipStream_t s);
-// mode 0: regular patches, 1: expanded sets, 2: the fast forms' refits
-// (items[] lists holding patch ids or, with bit 31, expanded-set ids).
-int launch_exact_fit(const FitArgs& a, int nterms, int mode, hipStream_t s);
+// The exact fits of the lists (k_qr.hip).  launch_qr_regular: the classified
+// regular patches, count[b] of them in bucket b; ws: workspace for the
+// reflectors of sets above 32 rows (any size that holds one set; qr_ws_bytes
+// gives the useful maximum).  launch_qr_lists: mode 1: expanded sets, 2: the
+// fast forms' refits (items[] lists holding patch ids or, with bit 31,
+// expanded-set ids), whose counts only the device knows.
+size_t qr_ws_bytes(int nterms, const int64_t* count);
+int launch_qr_regular(const FitArgs& a, int nterms, const int64_t* count, void* ws, size_t ws_bytes, hipStream_t s);
+int launch_qr_lists(const FitArgs& a, int nterms, int mode, hipStream_t s);
+// Buckets of more than 32 rows of the same lists (k_exact.hip).
+int launch_exact_lists(const FitArgs& a, int nterms, int mode, hipStream_t s);
 int launch_expand(const FitArgs& a, int nterms, hipStream_t s);
 // The exact fits of the big list (one wave per set, workspace ws of
 // big_ws_bytes(grid) bytes); grid 0 launches nothing.

@@ -1,41 +1,21 @@
-// k_exact.hip -- the FP64 patch recovery of spr::recoverField, reproducing the
-// reference's arithmetic operation for operation.
+// k_exact.hip -- patch construction of spr::recoverField with the reference's
+// rank decisions (spr/sprRecoverField.cc:155-393), and the exact fits that
+// k_qr.hip does not take: expanded sets and refits of more than 32 rows, and
+// sets of more than 192.
 //
-// The reference fits each patch with mth::decomposeQR / solveFromQR
-// (mth/mthQR.cc:19-163): Householder reflectors from R with sequential
-// column sums, an EXPLICIT m x m Q formed by reflect_rows, y = Q^T b as a
-// sequential dot product, back substitution, and evaluation of the monomials
-// at the entity's node (spr/sprRecoverField.cc:283-353).  Because the size
-// field downstream amplifies a 1-ulp change of the recovered field by ~1e4
-// or more, this form keeps every rounding of that sequence: sums in the same
-// order, no fused multiply-add (the library is built with -ffp-contract=off),
-// correctly rounded sqrt and division.
-//
-// Work mapping (one 64-lane wavefront per block):
-//  - a patch is owned by a group of LANES lanes (16, 32 or 64); a wave runs
-//    64/LANES patches in lock step;
-//  - the R recurrence keeps R (m x NT) and the reflectors V (NT x m) in LDS;
-//    its sequential sums run on one lane per group, its updates on all;
-//  - Q is never stored: every row of Q evolves independently under the
-//    reflectors, so lane j keeps row j in registers (MMAX doubles, static
-//    indexing) and only its first NT entries are kept (all that Q^T b needs
-//    for the back substitution);
-//  - rows of the patch matrix are recomputed from the mesh: sample points
-//    are the mesh-order rule points mapped by the coordinate field.
-#include "device.h"
+// k_exact_fit, one wave per patch: the R recurrence keeps R (m x NT) and the
+// reflectors V (NT x m) in LDS, its sequential sums on one lane, its updates
+// on all; lane j keeps row j of Q in registers and only its first NT entries
+// survive to the solve.  (The arithmetic is k_qr.hip's, whose mapping is the
+// faster one; these lists are short and their lengths known to the device
+// alone.)
+#include "exact_common.h"
 #include "fit_common.h"
-#include "spr_math.h"
+
+#include <algorithm>
 
 namespace sprg {
 namespace {
-
-__device__ __forceinline__ double sgn(double x) { return (x < 0) ? -1 : 1; }
-
-__device__ __forceinline__ int64_t node_of(const MeshView& m, int32_t t, int n)
-{
-  return n < 4 ? (int64_t)m.tv[4 * (int64_t)t + n]
-               : m.nv + (int64_t)m.te[6 * (int64_t)t + (n - 4)];
-}
 
 // getSamplePoints (spr/sprRecoverField.cc:193-211): the rule of the MESH
 // order, point l (the N1 rule ignores l), mapped by the coordinate field
@@ -194,72 +174,87 @@ __device__ __forceinline__ bool r_recurrence(double* R, double* V, double* sDot,
   return ok;
 }
 
-__device__ __forceinline__ void patch_set(const FitArgs& a, int64_t p,
-                                          const int32_t** set, int* ns)
-{
-  const MeshView& m = a.m;
-  if (p < m.nv) {
-    *set = m.v2t + m.v2t_off[p];
-    *ns = m.v2t_off[p + 1] - m.v2t_off[p];
-  } else {
-    int64_t e = p - m.nv;
-    *set = m.e2t + m.e2t_off[e];
-    *ns = m.e2t_off[e + 1] - m.e2t_off[e];
-  }
-}
-
 // Sorts patches into row-count buckets; patches with fewer rows than terms
-// go straight to the expansion queue (hasEnoughPoints, :355-363).  With
-// a.fast set, every regular patch goes to list 0.
-__global__ __launch_bounds__(256) void k_classify(FitArgs a, int nterms)
+// go straight to the expansion queue (hasEnoughPoints, :355-363).  A block
+// counts its CL_B patches per list in LDS and reserves each list's places
+// with one atomic (one per wave and list made the launch 2.85 ms for 14.0M
+// patches: the lists' counters are a handful of addresses).
+constexpr int CL_T = 256, CL_V = 16, CL_B = CL_T * CL_V;
+
+__global__ __launch_bounds__(CL_T) void k_classify(FitArgs a, int nterms)
 {
-  int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  // -1 none, 0..NBUCKET-1 bucket, NBUCKET expansion queue, NBUCKET + 1 the
-  // big list (the rank is decided there)
-  int target = -1;
-  if (p < a.npatch) {
-    const int32_t* set;
-    int ns;
-    patch_set(a, p, &set, &ns);
-    int m = ns * a.q;
-    if (m < nterms) {
-      target = NBUCKET;
-    } else if (a.fast) {
-      target = 0;
-    } else {
-      target = bucket_of(m);
-      if (target >= NBUCKET) {
-        target = m <= BIG_MMAX ? NBUCKET + 1 : -1;
-        if (target < 0) atomicOr(a.L.status, ST_TOO_LARGE);
+  // lists: 0..NBUCKET-1 bucket, NBUCKET expansion queue, NBUCKET + 1 the big
+  // list (the rank is decided there)
+  constexpr int NL = NBUCKET + 2;
+  __shared__ int sCount[NL];
+  __shared__ int sBase[NL];
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x < NL) sCount[threadIdx.x] = 0;
+  __syncthreads();
+  const int64_t p0 = blockIdx.x * (int64_t)CL_B + threadIdx.x;
+  int target[CL_V], pos[CL_V];
+#pragma unroll
+  for (int u = 0; u < CL_V; ++u) {
+    const int64_t p = p0 + u * CL_T;
+    target[u] = -1;
+    if (p < a.npatch) {
+      const int32_t* set;
+      int ns;
+      patch_set(a, p, &set, &ns);
+      const int m = ns * a.q;
+      if (m < nterms) {
+        target[u] = NBUCKET;
+      } else {
+        target[u] = bucket_of(m);
+        if (target[u] >= NBUCKET) {
+          target[u] = m <= BIG_MMAX ? NBUCKET + 1 : -1;
+          if (target[u] < 0) atomicOr(a.L.status, ST_TOO_LARGE);
+        }
       }
     }
   }
-  for (int b = 0; b < NBUCKET; ++b)
-    wave_append(b, target, a.L.count + b, a.L.items[b], (int32_t)p);
-  wave_append(NBUCKET, target, a.L.count + 2 * NBUCKET, a.L.xq, (int32_t)p);
-  big_append(target == NBUCKET + 1, a.L, (int32_t)(p | 0x40000000));
+  // places within the block, one LDS atomic per wave and list present
+#pragma unroll
+  for (int u = 0; u < CL_V; ++u) {
+    pos[u] = 0;
+    for (int b = 0; b < NL; ++b) {
+      const uint64_t mask = __ballot(target[u] == b);
+      if (!mask) continue;
+      const int leader = __ffsll((unsigned long long)mask) - 1;
+      int base = 0;
+      if (lane == leader) base = atomicAdd(&sCount[b], __popcll(mask));
+      base = __builtin_amdgcn_readlane(base, leader);
+      if (target[u] == b) pos[u] = base + __popcll(mask & ((1ull << lane) - 1));
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < NL) {
+    const int b = threadIdx.x, n = sCount[b];
+    int32_t* const counter = b < NBUCKET ? a.L.count + b : b == NBUCKET ? a.L.count + 2 * NBUCKET : a.L.status + 3;
+    sBase[b] = n ? atomicAdd(counter, n) : 0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < CL_V; ++u) {
+    const int b = target[u];
+    if (b < 0) continue;
+    const int32_t p = (int32_t)(p0 + u * CL_T);
+    int32_t* list = a.L.xq;
+#pragma unroll
+    for (int k = 0; k < NBUCKET; ++k)
+      if (b == k) list = a.L.items[k];
+    if (b == NBUCKET + 1) list = a.L.big;
+    list[sBase[b] + pos[u]] = b == NBUCKET + 1 ? (p | 0x40000000) : p;
+  }
 }
 
-// MODE: FIT_REGULAR walks items[bucket] (patch ids), FIT_EXPANDED walks
-// xitems[bucket] (expanded-set ids), FIT_MIXED walks items[bucket] holding
-// either (bit 31 set: an expanded-set id) -- the fast forms' refits.
-enum { FIT_REGULAR = 0, FIT_EXPANDED = 1, FIT_MIXED = 2 };
-
-// Waves per SIMD the fit of a bucket is compiled for: the kernel is bound by
-// the latency of its sequential sums, so the buckets that hold most patches
-// ask for two resident waves (the LDS of the 16- and 32-row buckets allows
-// no more); the Q row of MMAX doubles per lane sets the floor of the
-// register budget.
-// (Only targets that compile without scratch spills are requested.)
-constexpr int exact_waves(int nt, int mmax)
-{
-  return nt == 4 ? (mmax == 32 ? 2 : 1) : (mmax <= 32 || mmax == 96 ? 2 : 1);
-}
+// The Q row of MMAX doubles per lane sets the floor of the register budget:
+// two waves per SIMD where that compiles without scratch spills.
+constexpr int exact_waves(int nt, int mmax) { return nt == 10 && mmax == 96 ? 2 : 1; }
 
 template <int NT, int MMAX, int LANES, int MODE>
 __global__ __launch_bounds__(64, exact_waves(NT, MMAX)) void k_exact_fit(FitArgs a, int bucket)
 {
-  constexpr bool EXP = MODE == FIT_EXPANDED;
   constexpr int G = 64 / LANES;
   __shared__ double sR[G][MMAX * NT];
   __shared__ double sV[G][NT * MMAX];
@@ -271,40 +266,23 @@ __global__ __launch_bounds__(64, exact_waves(NT, MMAX)) void k_exact_fit(FitArgs
   const int g = threadIdx.x / LANES, gl = threadIdx.x % LANES;
   const MeshView& m = a.m;
   const int q = a.q, nc = a.nc;
-  const int32_t* list = EXP ? a.L.xitems[bucket] : a.L.items[bucket];
-  const int nitems = a.L.count[(EXP ? NBUCKET : 0) + bucket];
+  int nitems;
+  const int32_t* const list = fit_list<MODE>(a, bucket, &nitems);
   for (int base = blockIdx.x * G; base < nitems; base += gridDim.x * G) {
     const int item = base + g;
     const bool act = item < nitems;
     int64_t p = 0;
     int ns = 0;
     const int32_t* set = nullptr;
-    if (act) {
-      const int32_t entry = list[item];
-      if (EXP || (MODE == FIT_MIXED && entry < 0)) {
-        const int32_t it = entry & 0x7fffffff;
-        p = a.L.x_patch[it];
-        set = a.L.x_set + a.L.x_off[it];
-        ns = a.L.x_len[it];
-      } else {
-        p = entry;
-        patch_set(a, p, &set, &ns);
-      }
-    }
+    if (act) fit_item<MODE>(a, list[item], &p, &set, &ns);
     const int mrows = ns * q;
     for (int i = gl; i < ns; i += LANES) sS[g][i] = set[i];
     __syncthreads();
     build_rows<NT, LANES>(m, q, sS[g], mrows, sR[g], gl);
     __syncthreads();
     bool ok = r_recurrence<NT, LANES, MMAX>(sR[g], sV[g], sDot[g], sNorm[g], mrows, gl, act);
-    if (act && !ok && gl == 0) {
-      if (MODE != FIT_REGULAR) {  // sets whose rank was already decided
-        atomicOr(a.L.status, ST_INTERNAL);
-      } else {
-        int k = atomicAdd(a.L.count + 2 * NBUCKET, 1);
-        a.L.xq[k] = (int32_t)p;
-      }
-    }
+    // these sets' rank was already decided
+    if (act && !ok && gl == 0) atomicOr(a.L.status, ST_INTERNAL);
     // keep the top NT x NT of R for the back substitution, reuse sR for Q
     for (int i = gl; i < NT * NT; i += LANES) sRt[g][i] = sR[g][i];
     __syncthreads();
@@ -858,19 +836,18 @@ __global__ __launch_bounds__(64) void k_exact_big(FitArgs a, double* ws)
 
 inline unsigned grid_for(int64_t n, int per) { return (unsigned)((n + per - 1) / per); }
 
-template <int NT, int EXP>
-int fit_all(const FitArgs& a, hipStream_t s)
+template <int NT, int MODE>
+int fit_lists(const FitArgs& a, hipStream_t s)
 {
   // Persistent grids: each block loops over its share of the bucket's
   // device-side item count.
-  const unsigned blocks = (unsigned)a.shape.exact_blocks;
+  const unsigned blocks = (unsigned)std::min<int64_t>(a.shape.exact_blocks, a.npatch);
   const unsigned quarter = blocks / 4 > 0 ? blocks / 4 : 1;  // the 192-row bucket is rare
-  k_exact_fit<NT, 16, 16, EXP><<<blocks, 64, 0, s>>>(a, 0);
-  k_exact_fit<NT, 32, 32, EXP><<<blocks, 64, 0, s>>>(a, 1);
-  k_exact_fit<NT, 64, 64, EXP><<<blocks, 64, 0, s>>>(a, 2);
-  k_exact_fit<NT, 96, 64, EXP><<<blocks, 64, 0, s>>>(a, 3);
-  k_exact_fit<NT, 128, 64, EXP><<<blocks, 64, 0, s>>>(a, 4);
-  k_exact_fit<NT, 192, 64, EXP><<<quarter, 64, 0, s>>>(a, 5);
+  static_assert(NSMALL == 3 && NBUCKET == 7, "the buckets below");
+  k_exact_fit<NT, 64, 64, MODE><<<blocks, 64, 0, s>>>(a, 3);
+  k_exact_fit<NT, 96, 64, MODE><<<blocks, 64, 0, s>>>(a, 4);
+  k_exact_fit<NT, 128, 64, MODE><<<blocks, 64, 0, s>>>(a, 5);
+  k_exact_fit<NT, 192, 64, MODE><<<quarter, 64, 0, s>>>(a, 6);
   return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "exact fit launch failed");
 }
 
@@ -879,17 +856,15 @@ int fit_all(const FitArgs& a, hipStream_t s)
 int launch_classify(const FitArgs& a, int nterms, hipStream_t s)
 {
   if (a.npatch == 0) return 0;
-  k_classify<<<grid_for(a.npatch, 256), 256, 0, s>>>(a, nterms);
+  k_classify<<<grid_for(a.npatch, CL_B), CL_T, 0, s>>>(a, nterms);
   return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "classify launch failed");
 }
 
-int launch_exact_fit(const FitArgs& a, int nterms, int mode, hipStream_t s)
+int launch_exact_lists(const FitArgs& a, int nterms, int mode, hipStream_t s)
 {
-  switch (mode) {
-    case FIT_REGULAR: return nterms == 4 ? fit_all<4, FIT_REGULAR>(a, s) : fit_all<10, FIT_REGULAR>(a, s);
-    case FIT_EXPANDED: return nterms == 4 ? fit_all<4, FIT_EXPANDED>(a, s) : fit_all<10, FIT_EXPANDED>(a, s);
-    default: return nterms == 4 ? fit_all<4, FIT_MIXED>(a, s) : fit_all<10, FIT_MIXED>(a, s);
-  }
+  if (a.npatch == 0) return 0;
+  if (mode == FIT_EXPANDED) return nterms == 4 ? fit_lists<4, FIT_EXPANDED>(a, s) : fit_lists<10, FIT_EXPANDED>(a, s);
+  return nterms == 4 ? fit_lists<4, FIT_MIXED>(a, s) : fit_lists<10, FIT_MIXED>(a, s);
 }
 
 size_t big_ws_bytes(int grid) { return sizeof(double) * BIG_WS_DOUBLES * (size_t)grid; }

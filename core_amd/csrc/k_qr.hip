@@ -1,0 +1,786 @@
+// k_qr.hip -- the exact patch fits (SPRG_FP64, and the fast forms' refits):
+// mth::decomposeQR / solveFromQR (mth/mthQR.cc:19-163) operation for
+// operation -- Householder reflectors from sequential column sums, an
+// EXPLICIT Q formed by reflect_rows, y = Q^T b as a sequential dot product,
+// back substitution, evaluation at the entity's node
+// (spr/sprRecoverField.cc:283-353).  The size field downstream amplifies an
+// ulp of the recovered field by 1e4 and more, so every rounding of that
+// sequence is kept: sums in the same order, no fused multiply-add (the
+// library is built with -ffp-contract=off), correctly rounded square root
+// and division.
+//
+// The sums are sequential, so the work is spread over independent sums, not
+// inside one:
+//   R       a lane owns a COLUMN of the patch matrix, in registers: the NT
+//           columns' sums and updates run side by side, and a wave holds
+//           64 / NT patches (6 of the 10-term fit);
+//   Q       a lane owns ROWS of Q (every row evolves independently under the
+//           reflectors; only its first NT entries survive to the solve);
+//   Q^T b   a lane owns a component.
+// What is left of the reference's work: the first reflector's dot products
+// are its own entries (q_j starts as e_j), and the last reflector changes
+// only entry NT-1 of the NT that are kept.  (The sums' zero terms are left
+// out or in as it suits: adding +-0 changes no value but the sign of a zero.)
+//
+// Up to 32 rows one launch does it all, the reflectors in LDS.  Above, Q is
+// nearly all the work (m x m x 9 x 4 operations), and a row of Q fills the
+// registers, so there are three launches: k_qr_reflect leaves the reflectors
+// in memory, k_qr_rows reads them as scalars (VALU operands that take no
+// vector registers) and leaves Q's columns, k_qr_solve finishes.
+//
+// Measured, 14.0M patches of a 10.4M-tet mesh, 9 components: 225 ms with one
+// lane group per patch running the sums, 87.5 ms so; sets of 16 rows (6.1M)
+// 24.8 -> 9.2 ms, of 24 rows (6.1M) 69.8 -> 18.2 ms, of 65 to 96 rows (1.7M)
+// 123.6 -> 60.4 ms (reflectors 12.1, Q 40.1, solve 8.2).  Bounds: the FP64
+// issue of the separate multiplies and adds (no fused ones exist here): VALU
+// busy 66% in the small fits, 61% in Q, whose two waves per SIMD (96 doubles a
+// lane) wait for the scalar loads.  Q with the reflectors in LDS, a wave's
+// lanes filled with the rows of two sets: 1.39 ms per 36,864 sets instead of
+// 0.87.
+#include <algorithm>
+
+#include "exact_common.h"
+#include "fit_common.h"
+
+namespace sprg {
+namespace {
+
+// The two factors of monomial k among (1, x, y, z): poly_terms' products.
+__device__ __forceinline__ void term_pair(int k, int* a, int* b)
+{
+  // 1, x, y, z, xy, yz, zx, xx, yy, zz
+  *a = k < 4 ? k : k < 7 ? k - 3 : k - 6;
+  *b = k < 4 ? 0 : k == 4 ? 2 : k == 5 ? 3 : k == 6 ? 1 : k - 6;
+}
+
+// Samples of tet t (getSamplePoints, spr/sprRecoverField.cc:193-211): point
+// l < q of the MESH order's rule (the order-1 rule ignores l), mapped by the
+// coordinate field in the summation order of apf/apfElement.cc:106-114; each
+// node is loaded once for the tet's points.  Row l goes to X[4 l ..] as
+// (1, x, y, z).
+template <int ORDER>
+__device__ __forceinline__ void sample_tet(const MeshView& m, int32_t t, int q, double* X)
+{
+  constexpr int NN = ORDER == 1 ? 4 : 10;
+  constexpr int NQ = ORDER == 1 ? 1 : 4;  // distinct points
+  const int64_t tt = t;
+  int64_t node[NN];
+  const int4 v = *reinterpret_cast<const int4*>(m.tv + 4 * tt);
+  node[0] = v.x; node[1] = v.y; node[2] = v.z; node[3] = v.w;
+#pragma unroll
+  for (int k = 4; k < NN; ++k) node[k] = m.nv + (int64_t)m.te[6 * tt + (k - 4)];
+  double x[NQ][3];
+#pragma unroll
+  for (int l = 0; l < NQ; ++l) x[l][0] = x[l][1] = x[l][2] = 0;
+#pragma unroll
+  for (int n = 0; n < NN; ++n) {
+    const double* p = m.xyz + 3 * node[n];
+    const double p0 = p[0], p1 = p[1], p2 = p[2];
+#pragma unroll
+    for (int l = 0; l < NQ; ++l) {
+      double xi[3], N[10];
+      rule_point(ORDER, l, xi);
+      tet_values(ORDER, xi, N);
+      x[l][0] += p0 * N[n];
+      x[l][1] += p1 * N[n];
+      x[l][2] += p2 * N[n];
+    }
+  }
+  if constexpr (ORDER == 1) {
+    for (int l = 0; l < q; ++l) {
+      X[4 * l] = 1;
+      X[4 * l + 1] = x[0][0];
+      X[4 * l + 2] = x[0][1];
+      X[4 * l + 3] = x[0][2];
+    }
+  } else {
+#pragma unroll
+    for (int l = 0; l < NQ; ++l)
+      if (l < q) {
+        X[4 * l] = 1;
+        X[4 * l + 1] = x[l][0];
+        X[4 * l + 2] = x[l][1];
+        X[4 * l + 3] = x[l][2];
+      }
+  }
+}
+
+// A patch whose R lost rank: regular sets go to the expansion queue; sets
+// whose rank was already decided are inconsistent.  Every lane of the wave
+// calls it.
+template <int MODE>
+__device__ __forceinline__ void rank_failed(const FitArgs& a, bool failed, int64_t p)
+{
+  if (MODE == FIT_REGULAR) {
+    wave_append(1, failed ? 1 : 0, a.L.count + 2 * NBUCKET, a.L.xq, (int32_t)p);
+  } else if (failed) {
+    atomicOr(a.L.status, ST_INTERNAL);
+  }
+}
+
+// Back substitution (backsubUT, mth/mthQR.cc:131-148) with the packed upper
+// triangle rt(i, j), j >= i, and the polynomial at the node.
+template <int NT, class RT>
+__device__ __forceinline__ double backsub_eval(const double* y, RT rt, const double* node)
+{
+  double t[10], x[NT];
+  poly_terms(NT == 4 ? 1 : 2, node, t);
+#pragma unroll
+  for (int ii = 0; ii < NT; ++ii) {
+    const int i = NT - ii - 1;
+    x[i] = y[i];
+#pragma unroll
+    for (int j = i + 1; j < NT; ++j) x[i] -= rt(i, j) * x[j];
+    x[i] /= rt(i, i);
+  }
+  double v = 0;
+#pragma unroll
+  for (int i = 0; i < NT; ++i) v += x[i] * t[i];
+  return v;
+}
+
+// ---------------------------------------------------------------------------
+// up to 32 rows
+
+// Rows of Q a lane holds at once, and the passes that cover MMAX rows: as
+// many rows as the registers take (each reflector entry read from LDS then
+// serves several rows, and the rows' independent sums hide each other's
+// latency).
+constexpr int small_rpl(int nt, int mmax)
+{
+  return nt == 4 ? (mmax == 16 ? 4 : mmax == 24 ? 3 : 2) : mmax == 24 ? 3 : 2;
+}
+constexpr int small_waves(int nt, int mmax) { return mmax == 16 ? 3 : 2; }
+
+template <int NT, int MMAX, int MODE>
+__global__ __launch_bounds__(64, small_waves(NT, MMAX)) void k_qr_small(FitArgs a, int bucket)
+{
+  constexpr int ORDER = NT == 4 ? 1 : 2;
+  constexpr int G = NT, P = 64 / G;  // lanes per patch, patches per wave
+  constexpr int RPL = small_rpl(NT, MMAX);
+  constexpr int NPASS = (MMAX + G * RPL - 1) / (G * RPL);
+  constexpr int DIVS = (MMAX + G - 1) / G;
+  constexpr int VS = NT * MMAX, NRT = NT * (NT + 1) / 2;
+  // a patch's LDS: samples, then the reflectors V [NT][MMAX], then Q's
+  // columns [MMAX][NT]; R's triangle; two norms.  The stride keeps the
+  // patches' equal offsets 16 bytes apart modulo the banks.
+  constexpr int S = (VS + NRT + 2 + 31) / 32 * 32 + 2;
+  __shared__ double sm[P * S];
+  __shared__ int32_t sSet[P * MMAX];
+  const int lane = threadIdx.x;
+  const int g = lane / G < P ? lane / G : P - 1;
+  int gl = lane - g * G;
+  const bool on = gl < G;  // the lanes past P * G own nothing
+  const int col = on ? gl : G - 1;
+  double* const sV = sm + g * S;
+  double* const sRt = sV + VS;
+  double* const sN = sRt + NRT;
+  int32_t* const sS = sSet + g * MMAX;
+  int fa, fb;
+  term_pair(col, &fa, &fb);
+  const MeshView& m = a.m;
+  const int q = a.q, nc = a.nc;
+  int nitems;
+  const int32_t* const list = fit_list<MODE>(a, bucket, &nitems);
+  for (int base = blockIdx.x * P; base < nitems; base += gridDim.x * P) {
+    asm volatile("" : "+v"(gl));  // its many comparisons stay inside the loop (hoisted, they spill)
+    const bool act = base + g < nitems;
+    int64_t p = 0;
+    int ns = 0;
+    const int32_t* set = nullptr;
+    if (act) fit_item<MODE>(a, list[base + g], &p, &set, &ns);
+    const int rows = ns * q;  // <= MMAX
+    if (on)
+      for (int s = gl; s < ns; s += G) {
+        const int32_t t = set[s];
+        sS[s] = t;
+        sample_tet<ORDER>(m, t, q, sV + 4 * s * q);
+      }
+    __syncthreads();
+    // R: this lane's column
+    double r[MMAX];
+#pragma unroll
+    for (int i = 0; i < MMAX; ++i) {
+      const double v = sV[4 * i + fa] * sV[4 * i + fb];
+      r[i] = i < rows ? v : 0.0;
+    }
+    __syncthreads();
+    bool ok = act;
+    double s = 0;  // the squares of the column, rows k on
+#pragma unroll
+    for (int i = 0; i < MMAX; ++i) s += r[i] * r[i];
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+      // get_reflector on every lane's column; column k's is the one kept
+      const double cn = sqrt(s);
+      const double vk = r[k] + sgn(r[k]) * cn;
+      s = vk * vk;
+#pragma unroll
+      for (int i = k + 1; i < MMAX; ++i) s += r[i] * r[i];
+      if (on && gl == k) {
+        sN[0] = cn;
+        sN[1] = sqrt(s);
+        sV[k * MMAX + k] = vk;
+#pragma unroll
+        for (int i = k + 1; i < MMAX; ++i) sV[k * MMAX + i] = r[i];
+      }
+      __syncthreads();
+      ok = ok && !(sN[0] < 1e-10);
+      const double rn = sN[1];
+      // the lanes' divisions side by side (rows before k, whatever they
+      // hold, are not stored)
+      double w[DIVS];
+#pragma unroll
+      for (int u = 0; u < DIVS; ++u) {
+        const int i = gl + u * G;
+        w[u] = sV[k * MMAX + (i < MMAX ? i : MMAX - 1)] / rn;
+        asm volatile("" : "+v"(w[u]));  // formed here, not under the stores' conditions
+      }
+#pragma unroll
+      for (int u = 0; u < DIVS; ++u) {
+        const int i = gl + u * G;
+        if (on && i >= k && i < MMAX) sV[k * MMAX + i] = w[u];
+      }
+      __syncthreads();
+      double v[MMAX];
+#pragma unroll
+      for (int i = k; i < MMAX; ++i) v[i] = sV[k * MMAX + i];
+      double dot = 0;
+#pragma unroll
+      for (int i = k; i < MMAX; ++i) dot += r[i] * v[i];
+      const double d2 = 2 * dot;
+      // the update, and the squares the next reflector starts from
+      s = 0;
+#pragma unroll
+      for (int i = k; i < MMAX; ++i) {
+        r[i] -= d2 * v[i];
+        if (i > k) s += r[i] * r[i];
+      }
+      // row k is final (columns before k hold leftovers there)
+      if (on && gl >= k) sRt[tri(gl, k)] = r[k];
+    }
+    rank_failed<MODE>(a, act && !ok && gl == 0, p);
+    // Q: rows gl, gl + G, ... of each pass
+    double Qr[NPASS][RPL][NT];
+#pragma unroll
+    for (int ps = 0; ps < NPASS; ++ps) {
+      double x[RPL][MMAX], t2[RPL];
+#pragma unroll
+      for (int u = 0; u < RPL; ++u) {
+        const int j = (ps * RPL + u) * G + gl;
+        t2[u] = 2 * (j < MMAX ? sV[j] : 0.0);  // 2 e_j . v_0
+      }
+#pragma unroll
+      for (int l = 0; l < MMAX; ++l) {
+        const double v = sV[l];
+#pragma unroll
+        for (int u = 0; u < RPL; ++u) {
+          constexpr int G_ = G;
+          const int j0 = (ps * RPL + u) * G_;  // the lane's row is j0 + gl
+          const double pr = t2[u] * v;
+          x[u][l] = (l >= j0 && l < j0 + G_) ? (gl == l - j0 ? 1.0 : 0.0) - pr : -pr;
+        }
+      }
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int k = 1; k < NT; ++k) {
+        double dot[RPL];
+#pragma unroll
+        for (int u = 0; u < RPL; ++u) dot[u] = 0;
+#pragma unroll
+        for (int l = k; l < MMAX; ++l) {
+          const double v = sV[k * MMAX + l];
+#pragma unroll
+          for (int u = 0; u < RPL; ++u) dot[u] += x[u][l] * v;
+        }
+#pragma unroll
+        for (int u = 0; u < RPL; ++u) {
+          t2[u] = 2 * dot[u];
+          asm volatile("" : "+v"(t2[u]));  // formed here, not where Q is stored
+        }
+        // the reflector is read again for the update: held, it would cost
+        // MMAX more registers
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int l = k; l < (k == NT - 1 ? NT : MMAX); ++l) {
+          const double v = sV[k * MMAX + l];
+#pragma unroll
+          for (int u = 0; u < RPL; ++u) x[u][l] -= t2[u] * v;
+        }
+        asm volatile("" ::: "memory");
+      }
+#pragma unroll
+      for (int u = 0; u < RPL; ++u)
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+          Qr[ps][u][i] = x[u][i];
+          asm volatile("" : "+v"(Qr[ps][u][i]));
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int ps = 0; ps < NPASS; ++ps)
+#pragma unroll
+      for (int u = 0; u < RPL; ++u) {
+        const int j = (ps * RPL + u) * G + gl;
+        if (on && j < rows)
+#pragma unroll
+          for (int i = 0; i < NT; ++i) sV[j * NT + i] = Qr[ps][u][i];
+      }
+    __syncthreads();
+    // y = Q^T b (mth/mth_def.h:221-232), sequential over the rows; a lane
+    // per component reads its own values and solves for them
+    if (on && ok) {
+      const double node[3] = {m.xyz[3 * p], m.xyz[3 * p + 1], m.xyz[3 * p + 2]};
+      for (int c = gl; c < nc; c += G) {
+        double y[NT];
+#pragma unroll
+        for (int i = 0; i < NT; ++i) y[i] = 0;
+        auto add_row = [&](int r_, double b) {
+#pragma unroll
+          for (int i = 0; i < NT; ++i) y[i] += sV[r_ * NT + i] * b;
+        };
+        if (q == 4) {
+          // the next tet's four values in flight while one is summed
+          double b[4], bn[4];
+          const double* src = a.ip + (int64_t)sS[0] * 4 * nc + c;
+#pragma unroll
+          for (int l = 0; l < 4; ++l) bn[l] = src[l * nc];
+          for (int s = 0; s < ns; ++s) {
+#pragma unroll
+            for (int l = 0; l < 4; ++l) b[l] = bn[l];
+            src = a.ip + (int64_t)sS[s + 1 < ns ? s + 1 : s] * 4 * nc + c;
+#pragma unroll
+            for (int l = 0; l < 4; ++l) bn[l] = src[l * nc];
+#pragma unroll
+            for (int l = 0; l < 4; ++l) add_row(4 * s + l, b[l]);
+          }
+        } else {
+          for (int s = 0; s < ns; ++s)
+            for (int l = 0; l < q; ++l) add_row(s * q + l, a.ip[((int64_t)sS[s] * q + l) * nc + c]);
+        }
+        a.out[p * nc + c] = backsub_eval<NT>(y, [&](int i, int j) { return sRt[tri(j, i)]; }, node);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 33 to 192 rows: the regular sets of a bucket, a chunk at a time
+
+// Workspace of one set: the reflectors [NT][MMAX] (zero outside rows
+// k..m-1, up to the next multiple of 8 rows), then R's top [NT][NT], whose
+// last row's first entry says whether R kept full rank.
+constexpr int qr_ws_doubles(int nt, int mmax) { return nt * mmax + nt * nt; }
+constexpr int qr_waves(int mmax) { return (mmax + 63) / 64; }
+// with Q's first NT columns [MMAX][NT]
+constexpr size_t qr_set_bytes(int nt, int mmax) { return sizeof(double) * (qr_ws_doubles(nt, mmax) + (size_t)mmax * nt); }
+
+// Lanes per patch: one per column (of the 4-term fit, whose patches would
+// take too much LDS sixteen to a wave, twice that).
+constexpr int reflect_lanes(int nt) { return nt == 4 ? 8 : nt; }
+
+// The reflectors of the sets items[first, first + cap) of the bucket.  The
+// row loop runs over a column that shifts up by one entry per reflector, so
+// that every register index is fixed and the reflector loop stays rolled;
+// blocks of rows past the wave's longest set are skipped.
+template <int NT, int MMAX>
+__global__ __launch_bounds__(64, MMAX <= 96 ? 2 : 1) void k_qr_reflect(FitArgs a, int bucket, int first, int cap,
+                                                                       double* __restrict__ ws)
+{
+  constexpr int ORDER = NT == 4 ? 1 : 2;
+  constexpr int G = reflect_lanes(NT), P = 64 / G, B = 16, D = 5, E = 8;
+  constexpr int WS = qr_ws_doubles(NT, MMAX);
+  constexpr int S = 4 * MMAX + 2;  // samples, then the current reflector
+  static_assert(MMAX % B == 0, "whole blocks of rows");
+  __shared__ double sm[P * S];
+  __shared__ double sNorm[P][2];
+  const int lane = threadIdx.x;
+  const int g = lane / G < P ? lane / G : P - 1;
+  int gl = lane - g * G;
+  const bool on = gl < G;
+  const int col = gl < NT ? gl : NT - 1;
+  double* const sV = sm + g * S;
+  double* const sN = sNorm[g];
+  int fa, fb;
+  term_pair(col, &fa, &fb);
+  const MeshView& m = a.m;
+  const int q = a.q;
+  int nitems;
+  const int32_t* const list = fit_list<FIT_REGULAR>(a, bucket, &nitems);
+  const int left = nitems - first, n = left < cap ? left : cap;
+  for (int base = blockIdx.x * P; base < n; base += gridDim.x * P) {
+    asm volatile("" : "+v"(gl));
+    const bool act = base + g < n;
+    int64_t p = 0;
+    int ns = 0;
+    const int32_t* set = nullptr;
+    if (act) fit_item<FIT_REGULAR>(a, list[first + base + g], &p, &set, &ns);
+    const int rows = ns * q;
+    int mw = rows;  // the wave's longest set
+    for (int o = 32; o > 0; o >>= 1) {
+      const int y = __shfl(mw, lane ^ o);
+      mw = y > mw ? y : mw;
+    }
+    mw = __builtin_amdgcn_readlane(mw, 0);
+    double* const W = ws + (int64_t)(base + g) * WS;  // touched by active patches only
+    if (on)
+      for (int s = gl; s < ns; s += G) sample_tet<ORDER>(m, set[s], q, sV + 4 * s * q);
+    __syncthreads();
+    double r[MMAX];
+#pragma unroll
+    for (int i0 = 0; i0 < MMAX; i0 += B) {
+#pragma unroll
+      for (int i = i0; i < i0 + B; ++i) r[i] = 0;
+      if (i0 < mw) {
+#pragma unroll
+        for (int i = i0; i < i0 + B; ++i) {
+          const double v = sV[4 * i + fa] * sV[4 * i + fb];
+          r[i] = i < rows ? v : 0.0;
+        }
+      }
+    }
+    __syncthreads();
+    bool ok = act;
+    double s = 0;  // the squares of the column, rows k on
+#pragma unroll
+    for (int i0 = 0; i0 < MMAX; i0 += B)
+      if (i0 < mw) {
+#pragma unroll
+        for (int i = i0; i < i0 + B; ++i) {
+          s += r[i] * r[i];
+          asm volatile("" : "+v"(r[i]));  // the squares are formed again below: MMAX of them would not fit
+        }
+      }
+#pragma unroll 1
+    for (int k = 0; k < NT; ++k) {
+      const int mk = mw - k;  // r[i] is row k + i
+      const double cn = sqrt(s);
+      const double vk = r[0] + sgn(r[0]) * cn;
+      s = vk * vk;
+#pragma unroll
+      for (int i0 = 0; i0 < MMAX; i0 += B)
+        if (i0 < mk) {
+#pragma unroll
+          for (int i = i0; i < i0 + B; ++i)
+            if (i > 0) s += r[i] * r[i];
+        }
+      if (on && gl == k) {
+        sN[0] = cn;
+        sN[1] = sqrt(s);
+#pragma unroll
+        for (int i0 = 0; i0 < MMAX; i0 += B)
+          if (i0 <= mk) {
+#pragma unroll
+            for (int i = i0; i < i0 + B; ++i) sV[i] = i == 0 ? vk : r[i];
+          }
+      }
+      __syncthreads();
+      ok = ok && !(sN[0] < 1e-10);
+      const double rn = sN[1];
+      {
+        // the normalised reflector, D divisions of a lane side by side
+        const int end = rows - k, pad = ((rows + 7) & ~7) - k;
+        double* const Vk = W + k * MMAX;
+        if (on && act && gl < k) Vk[gl] = 0;
+#pragma unroll 1
+        for (int i0 = 0; i0 < mk + 7; i0 += D * G) {
+          double w[D];
+#pragma unroll
+          for (int u = 0; u < D; ++u) {
+            const int i = i0 + u * G + gl;
+            w[u] = sV[i < MMAX ? i : MMAX - 1] / rn;
+            asm volatile("" : "+v"(w[u]));  // formed here, not under the stores' conditions
+          }
+#pragma unroll
+          for (int u = 0; u < D; ++u) {
+            const int i = i0 + u * G + gl;
+            if (on && act && i < pad) {
+              if (i < end) sV[i] = w[u];
+              Vk[k + i] = i < end ? w[u] : 0.0;
+            }
+          }
+        }
+      }
+      __syncthreads();
+      // the reflector is read from LDS eight entries ahead of their use,
+      // twice (the column leaves no room to hold it)
+      double v[E], vn[E];
+      auto fetch = [&](int i0) {
+#pragma unroll
+        for (int u = 0; u < E; ++u) vn[u] = sV[i0 + u];
+      };
+      auto arrive = [&]() {
+#pragma unroll
+        for (int u = 0; u < E; ++u) v[u] = vn[u];
+        asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+        asm volatile("" ::: "memory");
+      };
+      fetch(0);
+      double dot = 0;
+#pragma unroll
+      for (int i0 = 0; i0 < MMAX; i0 += E)
+        if (i0 < mk) {
+          arrive();
+          fetch(i0 + E);
+#pragma unroll
+          for (int u = 0; u < E; ++u) dot += r[i0 + u] * v[u];
+          asm volatile("" : "+v"(dot));
+        }
+      const double d2 = 2 * dot;
+      fetch(0);
+      const double top = r[0] - d2 * sV[0];
+      if (on && act && gl >= k && gl < NT) W[NT * MMAX + k * NT + gl] = top;
+      // the update, each row one place up, and the squares the next
+      // reflector starts from; a block starting at mk still hands its (zero)
+      // first row to the block before
+      s = 0;
+#pragma unroll
+      for (int i0 = 0; i0 < MMAX; i0 += E)
+        if (i0 <= mk) {
+          arrive();
+          fetch(i0 + E);
+#pragma unroll
+          for (int u = 0; u < E; ++u)
+            if (i0 + u > 0) {
+              r[i0 + u - 1] = r[i0 + u] - d2 * v[u];
+              s += r[i0 + u - 1] * r[i0 + u - 1];
+              asm volatile("" : "+v"(r[i0 + u - 1]));
+            }
+          asm volatile("" : "+v"(s));
+        }
+      r[MMAX - 1] = 0;
+      __syncthreads();
+    }
+    if (act && gl == 0) W[NT * MMAX + (NT - 1) * NT] = ok ? 1.0 : 0.0;
+    rank_failed<FIT_REGULAR>(a, act && !ok && gl == 0, p);
+    __syncthreads();
+  }
+}
+
+// Q of the same sets: a block per set, a wave per 64 rows, a row per lane; the
+// first NT entries of each row are kept.  The reflectors are read at addresses
+// that are the same for the whole wave, as scalars; the block's waves read the
+// same ones at about the same time, and the four sets that a CU holds then
+// keep two reflectors each in the scalar cache, so a sweep finds the reflector
+// of the sweep before it there.
+template <int NT, int MMAX>
+__global__ __launch_bounds__(64 * qr_waves(MMAX), MMAX <= 96 ? 2 : 1) void k_qr_rows(
+    FitArgs a, int bucket, int first, int cap, const double* __restrict__ ws, double* __restrict__ qs)
+{
+  constexpr int WS = qr_ws_doubles(NT, MMAX), B = 8;
+  int tid = threadIdx.x;
+  const int r0 = 64 * __builtin_amdgcn_readlane(tid >> 6, 0);  // the wave's first row
+  int nitems;
+  const int32_t* const list = fit_list<FIT_REGULAR>(a, bucket, &nitems);
+  const int left = nitems - first, n = left < cap ? left : cap;
+  for (int it = blockIdx.x; it < n; it += gridDim.x) {
+    asm volatile("" : "+v"(tid));  // what depends on it stays inside the loop (hoisted, it costs the row its registers)
+    const int lane = tid & 63;
+    const double* __restrict__ V = ws + (int64_t)it * WS;
+    if (V[NT * MMAX + (NT - 1) * NT] == 0) continue;  // R lost rank: queued for the expansion
+    int64_t p;
+    int ns;
+    const int32_t* set;
+    fit_item<FIT_REGULAR>(a, list[first + it], &p, &set, &ns);
+    const int rows = ns * a.q;
+    if (r0 >= rows) continue;
+    const int j = r0 + lane;  // this lane's row
+    double x[MMAX];
+    double t2 = 2 * (j < rows ? V[j] : 0.0);  // 2 e_j . v_0
+    double dot = 0;
+    // Reflector k's update and reflector k + 1's dot product in one sweep,
+    // eight rows at a time; the next eight rows' entries of both are in
+    // flight meanwhile.  (Scalar loads return in any order, so a wait is a
+    // wait for all: the loads are issued once the first row has used the
+    // current entries.)
+    auto sweep = [&](const double* __restrict__ v, auto first_sweep) {
+      double a0[B], a1[B], n0[B], n1[B];
+      auto load = [&](int l0) {
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+          n0[u] = v[l0 + u];
+          n1[u] = v[MMAX + l0 + u];
+        }
+      };
+      load(0);
+#pragma unroll
+      for (int l0 = 0; l0 < MMAX; l0 += B)
+        if (l0 < rows) {
+#pragma unroll
+          for (int u = 0; u < B; ++u) {
+            a0[u] = n0[u];
+            a1[u] = n1[u];
+          }
+#pragma unroll
+          for (int u = 0; u < B; ++u) {
+            const int l = l0 + u;
+            x[l] = (first_sweep ? (l == j ? 1.0 : 0.0) : x[l]) - t2 * a0[u];
+            if (u == 0) {
+              asm volatile("" : "+v"(x[l]));
+              asm volatile("" ::: "memory");
+              load(l0 + B < MMAX ? l0 + B : l0);
+            }
+            dot += x[l] * a1[u];
+          }
+          // keeps the loads in this block (sunk to the next, they would be
+          // waited for at once)
+          asm volatile("" : "+v"(dot) : "s"(n0[0]), "s"(n1[0]));
+        }
+    };
+    // the reflector after next into this XCD's L2 meanwhile (it was
+    // written through another's: its first read would wait for memory)
+    double ahead = V[2 * MMAX + (lane < MMAX / 8 ? 8 * lane : 0)];
+    sweep(V, std::true_type());
+    asm volatile("" : "+v"(ahead));
+#pragma unroll 1
+    for (int k = 1; k < NT - 1; ++k) {
+      t2 = 2 * dot;
+      dot = 0;
+      ahead = V[(k + 2 < NT ? k + 2 : k) * MMAX + (lane < MMAX / 8 ? 8 * lane : 0)];
+      sweep(V + k * MMAX, std::false_type());
+      asm volatile("" : "+v"(ahead));
+    }
+    x[NT - 1] -= (2 * dot) * V[(NT - 1) * MMAX + NT - 1];
+    if (j < rows) {
+      double* const Q = qs + (int64_t)it * (MMAX * NT) + j * NT;
+#pragma unroll
+      for (int i = 0; i < NT; ++i) Q[i] = x[i];
+    }
+  }
+}
+
+// y = Q^T b (mth/mth_def.h:221-232), sequential over the rows, back
+// substitution and the value at the node, a thread per set and component:
+// latency-bound chains, so many waves, apart from k_qr_rows' two per SIMD.
+template <int NT, int MMAX>
+__global__ __launch_bounds__(256) void k_qr_solve(FitArgs a, int bucket, int first, int cap,
+                                                  const double* __restrict__ ws, const double* __restrict__ qs)
+{
+  constexpr int WS = qr_ws_doubles(NT, MMAX), L = 4;
+  int nitems;
+  const int32_t* const list = fit_list<FIT_REGULAR>(a, bucket, &nitems);
+  const int left = nitems - first, n = left < cap ? left : cap;
+  const int64_t id = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (id >= (int64_t)n * a.nc) return;
+  const int it = (int)(id / a.nc), c = (int)(id % a.nc);
+  const double* const Rt = ws + (int64_t)it * WS + NT * MMAX;
+  if (Rt[(NT - 1) * NT] == 0) return;
+  int64_t p;
+  int ns;
+  const int32_t* set;
+  fit_item<FIT_REGULAR>(a, list[first + it], &p, &set, &ns);
+  const int q = a.q;
+  const double* Q = qs + (int64_t)it * (MMAX * NT);
+  double y[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) y[i] = 0;
+  auto add_row = [&](double b) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) y[i] += Q[i] * b;
+    Q += NT;
+  };
+  if (q == 4) {
+    // the next tet's values in flight while one is summed
+    double b[L], bn[L];
+    auto load = [&](int32_t t) {
+#pragma unroll
+      for (int l = 0; l < L; ++l) bn[l] = a.ip[((int64_t)t * 4 + l) * a.nc + c];
+    };
+    load(set[0]);
+    int32_t tn = set[ns > 1 ? 1 : 0];
+    for (int s = 0; s < ns; ++s) {
+#pragma unroll
+      for (int l = 0; l < L; ++l) b[l] = bn[l];
+      load(tn);
+      tn = set[s + 2 < ns ? s + 2 : ns - 1];
+#pragma unroll
+      for (int l = 0; l < L; ++l) add_row(b[l]);
+    }
+  } else {
+    for (int s = 0; s < ns; ++s)
+      for (int l = 0; l < q; ++l) add_row(a.ip[((int64_t)set[s] * q + l) * a.nc + c]);
+  }
+  const double node[3] = {a.m.xyz[3 * p], a.m.xyz[3 * p + 1], a.m.xyz[3 * p + 2]};
+  a.out[p * a.nc + c] = backsub_eval<NT>(y, [&](int i, int j) { return Rt[i * NT + j]; }, node);
+}
+
+// Sets per k_qr_reflect / k_qr_rows / k_qr_solve sequence: enough to keep
+// every SIMD's waves busy through several rounds of each launch, and no more
+// (the reflectors and Q of 36,864 96-row sets take 596 MB).
+constexpr int64_t QR_CHUNK = 36864;
+
+template <int NT, int MODE>
+void small_fits(const FitArgs& a, const int64_t* count, hipStream_t s)
+{
+  constexpr int P = 64 / NT;
+  auto blocks = [&](int b) {
+    const int64_t n = count ? count[b] : a.npatch;
+    return (unsigned)std::max<int64_t>(1, std::min<int64_t>(a.shape.exact_blocks, (n + P - 1) / P));
+  };
+  if (!count || count[0]) k_qr_small<NT, 16, MODE><<<blocks(0), 64, 0, s>>>(a, 0);
+  if (!count || count[1]) k_qr_small<NT, 24, MODE><<<blocks(1), 64, 0, s>>>(a, 1);
+  if (!count || count[2]) k_qr_small<NT, 32, MODE><<<blocks(2), 64, 0, s>>>(a, 2);
+}
+
+template <int NT, int MMAX>
+void large_fits(const FitArgs& a, int bucket, int64_t count, double* ws, size_t ws_bytes, hipStream_t s)
+{
+  constexpr int P = 64 / reflect_lanes(NT);
+  const int cap = (int)std::min<int64_t>(QR_CHUNK, (int64_t)(ws_bytes / qr_set_bytes(NT, MMAX)));
+  double* const qs = ws + (int64_t)cap * qr_ws_doubles(NT, MMAX);
+  for (int64_t first = 0; first < count; first += cap) {
+    const int64_t n = std::min<int64_t>(cap, count - first);
+    const int64_t most = a.shape.exact_blocks;
+    k_qr_reflect<NT, MMAX><<<(unsigned)std::min(most, (n + P - 1) / P), 64, 0, s>>>(a, bucket, (int)first, cap, ws);
+    if (a.nc == 0) continue;  // the rank decisions alone
+    k_qr_rows<NT, MMAX><<<(unsigned)std::min(most, n), 64 * qr_waves(MMAX), 0, s>>>(a, bucket, (int)first, cap, ws, qs);
+    k_qr_solve<NT, MMAX><<<(unsigned)((n * a.nc + 255) / 256), 256, 0, s>>>(a, bucket, (int)first, cap, ws, qs);
+  }
+}
+
+template <int NT>
+int regular_fits(const FitArgs& a, const int64_t* count, double* ws, size_t ws_bytes, hipStream_t s)
+{
+  static_assert(NSMALL == 3 && NBUCKET == 7, "the buckets below");
+  for (int b = NSMALL; b < NBUCKET; ++b)
+    if (count[b] && ws_bytes < qr_set_bytes(NT, bucket_rows(b)))
+      return sprg_fail(SPRG_ENOMEM, "exact fit: no workspace for a set of %d rows", bucket_rows(b));
+  small_fits<NT, FIT_REGULAR>(a, count, s);
+  large_fits<NT, 64>(a, 3, count[3], ws, ws_bytes, s);
+  large_fits<NT, 96>(a, 4, count[4], ws, ws_bytes, s);
+  large_fits<NT, 128>(a, 5, count[5], ws, ws_bytes, s);
+  large_fits<NT, 192>(a, 6, count[6], ws, ws_bytes, s);
+  return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "exact fit launch failed");
+}
+
+}  // namespace
+
+size_t qr_ws_bytes(int nterms, const int64_t* count)
+{
+  size_t most = 0;
+  for (int b = NSMALL; b < NBUCKET; ++b)
+    most = std::max(most, qr_set_bytes(nterms, bucket_rows(b)) * (size_t)std::min<int64_t>(count[b], QR_CHUNK));
+  return most;
+}
+
+int launch_qr_regular(const FitArgs& a, int nterms, const int64_t* count, void* ws, size_t ws_bytes, hipStream_t s)
+{
+  double* const w = static_cast<double*>(ws);
+  return nterms == 4 ? regular_fits<4>(a, count, w, ws_bytes, s) : regular_fits<10>(a, count, w, ws_bytes, s);
+}
+
+int launch_qr_lists(const FitArgs& a, int nterms, int mode, hipStream_t s)
+{
+  if (a.npatch == 0) return 0;
+  if (mode == FIT_EXPANDED) {
+    if (nterms == 4) small_fits<4, FIT_EXPANDED>(a, nullptr, s); else small_fits<10, FIT_EXPANDED>(a, nullptr, s);
+  } else {
+    if (nterms == 4) small_fits<4, FIT_MIXED>(a, nullptr, s); else small_fits<10, FIT_MIXED>(a, nullptr, s);
+  }
+  if (hipGetLastError() != hipSuccess) return sprg_fail(SPRG_EHIP, "exact fit launch failed");
+  return launch_exact_lists(a, nterms, mode, s);
+}
+
+}  // namespace sprg

@@ -20,12 +20,6 @@ using namespace sprg;
 // vertex average.
 constexpr int NPHASE = 5;
 
-struct sprg_ctx {
-  int device = 0;
-  hipStream_t stream = nullptr;
-  void* scratch = nullptr;  // this device's address of `scratch` (below)
-};
-
 namespace {
 
 // Grow-only device buffer.
@@ -57,6 +51,15 @@ struct DBuf {
 
 }  // namespace
 
+struct sprg_ctx {
+  int device = 0;
+  hipStream_t stream = nullptr;
+  void* scratch = nullptr;  // this device's address of `scratch` (below)
+  // reflectors of the exact fits (k_qr.hip): the context's calls run one
+  // after the other on its stream, so its meshes share it
+  DBuf qr_ws;
+};
+
 struct sprg_mesh {
   sprg_ctx* ctx = nullptr;
   int64_t nv = 0, nt = 0, ne = 0, nnodes = 0;
@@ -70,6 +73,7 @@ struct sprg_mesh {
   // per-call workspace
   DBuf lists, xset, rec, elem, partial, scalars, status, setlen, big_ws;
   int max_set = 0;    // tets in the largest initial patch set
+  std::vector<int64_t> set_count;  // initial sets by their number of tets
   int64_t list_cap = 0, xset_cap = 0;
   // phase timing of the last call: events on the context stream
   hipEvent_t ev[NPHASE + 1] = {};
@@ -188,6 +192,7 @@ extern "C" int sprg_ctx_destroy(sprg_ctx* ctx)
   if (!ctx) return 0;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
+  ctx->qr_ws.release();
   (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return 0;
@@ -277,6 +282,16 @@ int build_tiles(sprg_mesh* m, const int32_t* tet_verts, const int32_t* tet_edges
   m->max_set = 0;
   for (int32_t c : vcount) m->max_set = std::max(m->max_set, (int)c);
   for (int32_t c : ecount) m->max_set = std::max(m->max_set, (int)c);
+  {
+    // four counters per size in turn: neighbours' sizes repeat, and an
+    // increment waits for the one before it
+    const size_t ns = (size_t)m->max_set + 1;
+    std::vector<int64_t> n(4 * ns, 0);
+    for (const std::vector<int32_t>* v : {&vcount, &ecount})
+      for (size_t i = 0; i < v->size(); ++i) ++n[(i & 3) * ns + (*v)[i]];
+    m->set_count.resize(ns);
+    for (size_t k = 0; k < ns; ++k) m->set_count[k] = n[k] + n[ns + k] + n[2 * ns + k] + n[3 * ns + k];
+  }
   if (nv + ne >= (1 << 27)) return 0;  // the slot encoding holds 27-bit patch ids
   if (10 * nt >= INT32_MAX) return 0;  // loc offsets are int32
   std::vector<int32_t> own_off(nv + 1, 0), own_e(ne);
@@ -627,19 +642,31 @@ void collect_phases(sprg_mesh* m)
 // set of this mesh has that many rows at q points per tet.
 int big_grid(const sprg_mesh* m, int q) { return (int64_t)m->max_set * q > bucket_rows(NBUCKET - 1) ? 128 : 0; }
 
-// Bytes of the work lists of np patches: items and xitems per bucket, xq,
-// xq_exact, fbq, x_patch, x_len (int32 each), x_off (int64), counters,
+// Regular patches of each row bucket at q points per tet.
+void bucket_counts(const sprg_mesh* m, int q, int64_t* count)
+{
+  const int nterms = m->order == 1 ? 4 : 10;
+  for (int b = 0; b < NBUCKET; ++b) count[b] = 0;
+  for (size_t ns = 0; ns < m->set_count.size(); ++ns) {
+    const int rows = (int)ns * q, b = bucket_of(rows);
+    if (rows >= nterms && b < NBUCKET) count[b] += m->set_count[ns];
+  }
+}
+
+// Bytes of the work lists of np patches: items, xitems per bucket, xq,
+// xq_exact, fbq, big, x_patch, x_len (int32 each), x_off (int64), counters,
 // cursors and the status words.
 size_t list_bytes(int64_t np)
 {
-  const size_t n32 = (size_t)np * (2 * NBUCKET + 6) + 2 * NBUCKET + 8;
+  const size_t n32 = (size_t)np * (NBUCKET + 7) + 2 * NBUCKET + 8;
   return n32 * 4 + (size_t)np * 8 + 64;
 }
 
 // Lays the work lists of cap patches out from base (8-byte aligned); the
 // expanded sets live in x_set[0, x_cap).
-void carve_lists(char* base, int64_t cap, int32_t* x_set, int64_t x_cap, Lists& L)
+void carve_lists(const sprg_mesh* m, char* base, int64_t cap, int32_t* x_set, int64_t x_cap, FitArgs& a)
 {
+  Lists& L = a.L;
   int64_t* x_off = (int64_t*)base;  // 8-byte aligned first
   int64_t* x_cursor = x_off + cap;
   int32_t* p = (int32_t*)(x_cursor + 2);
@@ -649,8 +676,20 @@ void carve_lists(char* base, int64_t cap, int32_t* x_set, int64_t x_cap, Lists& 
   p += 2 * NBUCKET + 2;
   L.status = p;  // [0] status bits, [1] exact-expansion count, [2] fallback entries taken before the expansion
   p += 4;
-  for (int b = 0; b < NBUCKET; ++b) { L.items[b] = p; p += cap; }
+  int32_t* const items = p;
+  p += cap;
   for (int b = 0; b < NBUCKET; ++b) { L.xitems[b] = p; p += cap; }
+  if (a.fast) {
+    // a patch is refitted at most once, by any bucket
+    for (int b = 0; b < NBUCKET; ++b) L.items[b] = b == 0 ? items : L.xitems[b];
+  } else {
+    int64_t count[NBUCKET], first = 0;
+    bucket_counts(m, a.q, count);
+    for (int b = 0; b < NBUCKET; ++b) {
+      L.items[b] = items + first;
+      first += count[b];
+    }
+  }
   L.xq = p; p += cap;
   L.xq_exact = p; p += cap;
   L.fbq = p; p += cap;
@@ -660,6 +699,19 @@ void carve_lists(char* base, int64_t cap, int32_t* x_set, int64_t x_cap, Lists& 
   L.x_set = x_set;
   L.x_cap = x_cap;
   L.cap = cap;
+}
+
+// The exact fits' workspace of the context, for the mesh's sets at q points
+// per tet: the useful maximum, or as much of it as the device grants.
+int ensure_qr_ws(sprg_mesh* m, int q)
+{
+  int64_t count[NBUCKET];
+  bucket_counts(m, q, count);
+  DBuf& ws = m->ctx->qr_ws;
+  int rc = 0;
+  for (size_t want = qr_ws_bytes(m->order == 1 ? 4 : 10, count), k = 0; k < 6 && ws.bytes < want >> k; ++k)
+    if (!(rc = ws.ensure(want >> k))) break;
+  return rc;
 }
 
 // Lays the work lists out in the mesh's own workspaces (grown as needed).
@@ -677,7 +729,9 @@ int setup_lists(sprg_mesh* m, FitArgs& a)
     if (rc) return rc;
     m->xset_cap = cap;
   }
-  carve_lists(m->lists.as<char>(), m->list_cap, m->xset.as<int32_t>(), m->xset_cap, a.L);
+  carve_lists(m, m->lists.as<char>(), m->list_cap, m->xset.as<int32_t>(), m->xset_cap, a);
+  if (!a.fast)
+    if (int rc = ensure_qr_ws(m, a.q)) return rc;
   if (big_grid(m, a.q) > 0) {
     int rc = m->big_ws.ensure(big_ws_bytes(big_grid(m, a.q)));
     if (rc) return rc;
@@ -714,7 +768,8 @@ bool valid_form(int form) { return form == SPRG_FP64 || form == SPRG_FP32R || fo
 // exact fit of the initial sets -> expansion -> exact fit of the expanded
 // sets.  Fast forms: fit of every patch -> expansion -> fit of the expanded
 // sets -> FP64 fallback -> exact refits.  marks: record the phase events.
-int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, hipStream_t s, bool marks)
+// qr_ws: the exact fits' workspace (FP64 form).
+int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, void* qr_ws, size_t qr_bytes, hipStream_t s, bool marks)
 {
   const bool fast = form != SPRG_FP64;
   const int nterms = m->order == 1 ? 4 : 10;
@@ -744,7 +799,9 @@ int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, hipStream_t s, boo
     }
   } else {
     if ((rc = launch_classify(a, nterms, s))) return rc;
-    if ((rc = launch_exact_fit(a, nterms, 0, s))) return rc;
+    int64_t count[NBUCKET];
+    bucket_counts(m, a.q, count);
+    if ((rc = launch_qr_regular(a, nterms, count, qr_ws, qr_bytes, s))) return rc;
   }
   if (marks) m->mark(1);
   if ((rc = launch_expand(a, nterms, s))) return rc;
@@ -753,9 +810,9 @@ int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, hipStream_t s, boo
     if ((rc = launch_fast_fit(a, nterms, form, 1, s))) return rc;
     if ((rc = launch_fast_fit(a, nterms, form, 2, s))) return rc;
     // poorly conditioned sets: the reference's arithmetic
-    if ((rc = launch_exact_fit(a, nterms, 2, s))) return rc;
+    if ((rc = launch_qr_lists(a, nterms, 2, s))) return rc;
   } else {
-    if ((rc = launch_exact_fit(a, nterms, 1, s))) return rc;
+    if ((rc = launch_qr_lists(a, nterms, 1, s))) return rc;
   }
   // sets above 192 rows, from every pass above
   if ((rc = launch_exact_big(a, nterms, m->big_ws.as<double>(), big_grid(m, a.q), s))) return rc;
@@ -813,7 +870,8 @@ int run_recover(sprg_mesh* m, int q, int nc, const double* ip, double* out, int 
     FitArgs a = fit_args(m, q, nc, ip, out, form);
     int rc = setup_lists(m, a);
     if (rc) return rc;
-    if ((rc = enqueue_recover(m, a, form, s, true))) return rc;
+    const DBuf& ws = m->ctx->qr_ws;
+    if ((rc = enqueue_recover(m, a, form, ws.p, ws.bytes, s, true))) return rc;
     int32_t st = 0;
     if ((rc = read_status(m, a, &st))) return rc;
     collect_phases(m);
@@ -835,7 +893,10 @@ int run_recover_noalloc(sprg_mesh* m, int q, int nc, const double* ip, double* o
   char* base = static_cast<char*>(m->ctx->scratch);
   if (!base) return sprg_fail(SPRG_EHIP, "recover_noalloc: no scratch on this context's device");
   const int64_t np = m->npatch();
-  const size_t lists = (list_bytes(np) + 255) / 256 * 256;
+  // 80 bytes a patch (the lists take less): this decides which meshes the
+  // entry point accepts and how many expanded sets it holds
+  const size_t lists = ((size_t)np * 80 + 144 + 255) / 256 * 256;
+  if (list_bytes(np) > lists) return sprg_fail(SPRG_EINTERNAL, "recover_noalloc: work lists above their share");
   // at least one expanded-set entry per patch plus slack beyond the lists
   const size_t need = lists + sizeof(int32_t) * ((size_t)np + (1 << 18));
   if (need > SPRG_NOALLOC_SCRATCH_BYTES)
@@ -849,9 +910,11 @@ int run_recover_noalloc(sprg_mesh* m, int q, int nc, const double* ip, double* o
                      bucket_rows(NBUCKET - 1));
   FitArgs a = fit_args(m, q, nc, ip, out, form);
   const int64_t x_cap = (int64_t)((SPRG_NOALLOC_SCRATCH_BYTES - lists) / sizeof(int32_t));
-  carve_lists(base, np, reinterpret_cast<int32_t*>(base + lists), x_cap, a.L);
+  carve_lists(m, base, np, reinterpret_cast<int32_t*>(base + lists), x_cap, a);
   hipStream_t s = m->ctx->stream;
-  int rc = enqueue_recover(m, a, form, s, true);
+  // the exact fits of the regular sets are done before the first expanded
+  // set is stored, so their reflectors take that storage
+  int rc = enqueue_recover(m, a, form, a.L.x_set, sizeof(int32_t) * (size_t)x_cap, s, true);
   if (rc) return rc;
   int32_t st = 0;
   if ((rc = read_status(m, a, &st))) return rc;
@@ -1282,7 +1345,7 @@ int record_batch(sprg_batch* b, int ip_order, int nc, const double* const* ip,
   int rc = 0;
   for (int i = 0; i < n && !rc; ++i) {
     sprg_mesh* m = b->meshes[i];
-    rc = enqueue_recover(m, fa[i], form, s, false);
+    rc = enqueue_recover(m, fa[i], form, b->ctx->qr_ws.p, b->ctx->qr_ws.bytes, s, false);
     if (!rc) {
       const bool tgt = target != nullptr;
       EstArgs e = est_args(m, ip_order, nc, ip[i], tgt ? 1 : 0, ar, tgt ? (double)target[i] : 0,
@@ -1330,6 +1393,8 @@ int workspace_key(sprg_batch* b, int q, int nc, int form, std::vector<uint64_t>&
     key.push_back((uint64_t)m->shape.expand_blocks);
     key.push_back((uint64_t)m->shape.tile_blocks);
   }
+  key.push_back((uint64_t)(uintptr_t)b->ctx->qr_ws.p);
+  key.push_back((uint64_t)b->ctx->qr_ws.bytes);
   return 0;
 }
 
