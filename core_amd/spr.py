@@ -347,8 +347,9 @@ def averageToVertex(element_values, mesh, name="size"):
 
 
 class Batch:
-    """Several meshes whose size-field pipelines run as one recorded HIP
-    graph (sprg_batch_*): the first call records, identical calls replay."""
+    """Several meshes whose size-field pipelines run as recorded HIP graphs
+    side by side (sprg_batch_*): the first call records, identical calls
+    replay."""
 
     def __init__(self, meshes):
         meshes = list(meshes)
@@ -378,7 +379,7 @@ class Batch:
         """For every mesh i: getSPRSizeField(fields[i], adapt_ratio) when
         targets is None, else getTargetSPRSizeField(fields[i], targets[i],
         alpha, beta).  Returns the "size" tensors; pass the previous
-        `outputs` back to replay the recorded graph."""
+        `outputs` back to replay the recorded graphs."""
         n = len(self.meshes)
         if len(fields) != n:
             raise SPRError(_lib.SPRG_EINVAL, "one field per mesh")

@@ -189,11 +189,11 @@ int sprg_average_to_vertex(sprg_mesh* mesh, const double* elem, double* vert);
  * runs, for every mesh i, spr::getSPRSizeField(ip[i], adapt_ratio) when
  * target is NULL, else spr::getTargetSPRSizeField(ip[i], target[i], alpha,
  * beta) (every target[i] > 0), writing size[i] [nv_i] (device pointers).
- * The first call records all pipelines into one HIP graph; later calls
- * replay it when the fields, parameters, launch shapes and every mesh's
- * workspace are unchanged (otherwise they record again: an eager call that
- * grows a mesh's workspace invalidates the recorded graph).  ms (optional):
- * wall time of the replay.  Results equal the per-mesh calls bit for bit.
+ * The first call records all pipelines into HIP graphs that run side by
+ * side; later calls replay them when the fields, parameters, launch shapes
+ * and every mesh's workspace are unchanged (otherwise they record again: an
+ * eager call that grows a mesh's workspace invalidates the recorded graphs).
+ * ms (optional): wall time of the replay.  Results equal the per-mesh calls bit for bit.
  * No reference counterpart: the reference estimates one mesh per call. */
 typedef struct sprg_batch sprg_batch;
 int sprg_batch_create(sprg_ctx* ctx, int nmesh, sprg_mesh* const* meshes,
