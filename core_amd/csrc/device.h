@@ -61,7 +61,8 @@ struct Lists {
   int32_t* count;            // [NBUCKET] regular, [NBUCKET] expanded, [1] expand-queue
   int32_t* xitems[NBUCKET];
   int32_t* xq;               // patches queued for the exact rank test /
-                             // expansion; bit 31: test the initial set first
+                             // expansion; bit 31: test the initial set
+                             // first, bit 30: it was tested (k_rank_test)
   int32_t* xq_exact;         // queued patches whose expansion needs the exact
                              // rank test (same encoding as xq); its count
                              // follows the status word
@@ -191,6 +192,9 @@ int launch_qr_regular(const FitArgs& a, int nterms, const int64_t* count, void* 
 int launch_qr_lists(const FitArgs& a, int nterms, int mode, hipStream_t s);
 // Buckets of more than 32 rows of the same lists (k_exact.hip).
 int launch_exact_lists(const FitArgs& a, int nterms, int mode, hipStream_t s);
+// Before launch_expand in the fast forms: the rank test of queued initial sets
+// of up to 32 rows (k_qr.hip).
+int launch_rank_test(const FitArgs& a, int nterms, hipStream_t s);
 int launch_expand(const FitArgs& a, int nterms, hipStream_t s);
 // The exact fits of the big list (one wave per set, workspace ws of
 // big_ws_bytes(grid) bytes); grid 0 launches nothing.

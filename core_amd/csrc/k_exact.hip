@@ -528,12 +528,19 @@ __global__ __launch_bounds__(64) void k_expand(FitArgs a)
   const int64_t chunk_size = share > 1024 ? 1024 : share < XSET ? XSET : share;
   if (lane == 0) { sBase = 0; sLeft = 0; }
   for (int k = blockIdx.x; k < nq; k += gridDim.x) {
-    // the item id of a queued patch is its position in xq; the light pass
-    // marks it empty first (x_len 0) and whichever pass finds the set fills it
+    // the item id of a queued patch is its position in xq; it is marked
+    // empty first (x_len 0: by k_rank_test in the fast forms) and whichever
+    // pass finds the set fills it
     const int32_t it = EXACT ? queue[k] : k;
     const int32_t entry = a.L.xq[it];
-    if (!EXACT && lane == 0) a.L.x_len[it] = 0;
-    const int64_t p = entry & 0x7fffffff;
+    if (!EXACT) {
+      if (a.fast) {
+        if (a.L.x_len[it] > 0) continue;  // k_rank_test kept the initial set
+      } else if (lane == 0) {
+        a.L.x_len[it] = 0;
+      }
+    }
+    const int64_t p = entry & 0x3fffffff;  // bit 30: the initial set's rank is tested
     const bool test_first = entry < 0;
     const int32_t* set0;
     int ns0;
@@ -655,7 +662,10 @@ __global__ __launch_bounds__(64) void k_expand(FitArgs a)
           // a certified full rank needs no exact test; anything else does
           ok = certify_full_rank<NT>(m, q, sCur, mrows, p, lane, sD);
           if (!ok && !EXACT) {
-            if (lane == 0) a.L.xq_exact[atomicAdd(nexact, 1)] = it;
+            if (lane == 0) {
+              a.L.xq_exact[atomicAdd(nexact, 1)] = it;
+              if (entry & 0x40000000) atomicAdd(a.L.status + 4, -1);  // counted once
+            }
             deferred = true;
             break;
           }

@@ -142,6 +142,74 @@ __device__ __forceinline__ double backsub_eval(const double* y, RT rt, const dou
 // ---------------------------------------------------------------------------
 // up to 32 rows
 
+// R of up to MMAX rows, a column per lane (decomposeQR, mth/mthQR.cc:19-63,
+// restricted to what the solve uses): false as soon as a column norm falls
+// below 1e-10 (mth/mthQR.cc:31).  KEEP: reflector k stays in sV[k MMAX + k ..],
+// R's triangle in sRt; else each takes the place of the one before.  Every
+// lane of the wave calls it.
+template <int NT, int MMAX, bool KEEP>
+__device__ __forceinline__ bool small_r(double (&r)[MMAX], double* sV, double* sN, double* sRt, int gl, bool on,
+                                        bool act)
+{
+  constexpr int G = NT, DIVS = (MMAX + G - 1) / G;
+  constexpr int KS = KEEP ? MMAX : 0;  // the reflectors' stride
+  bool ok = act;
+  double s = 0;  // the squares of the column, rows k on
+#pragma unroll
+  for (int i = 0; i < MMAX; ++i) s += r[i] * r[i];
+#pragma unroll
+  for (int k = 0; k < NT; ++k) {
+    // get_reflector on every lane's column; column k's is the one kept
+    const double cn = sqrt(s);
+    const double vk = r[k] + sgn(r[k]) * cn;
+    s = vk * vk;
+#pragma unroll
+    for (int i = k + 1; i < MMAX; ++i) s += r[i] * r[i];
+    if (on && gl == k) {
+      sN[0] = cn;
+      sN[1] = sqrt(s);
+      sV[k * KS + k] = vk;
+#pragma unroll
+      for (int i = k + 1; i < MMAX; ++i) sV[k * KS + i] = r[i];
+    }
+    __syncthreads();
+    ok = ok && !(sN[0] < 1e-10);
+    const double rn = sN[1];
+    // the lanes' divisions side by side (rows before k, whatever they
+    // hold, are not stored)
+    double w[DIVS];
+#pragma unroll
+    for (int u = 0; u < DIVS; ++u) {
+      const int i = gl + u * G;
+      w[u] = sV[k * KS + (i < MMAX ? i : MMAX - 1)] / rn;
+      asm volatile("" : "+v"(w[u]));  // formed here, not under the stores' conditions
+    }
+#pragma unroll
+    for (int u = 0; u < DIVS; ++u) {
+      const int i = gl + u * G;
+      if (on && i >= k && i < MMAX) sV[k * KS + i] = w[u];
+    }
+    __syncthreads();
+    double v[MMAX];
+#pragma unroll
+    for (int i = k; i < MMAX; ++i) v[i] = sV[k * KS + i];
+    double dot = 0;
+#pragma unroll
+    for (int i = k; i < MMAX; ++i) dot += r[i] * v[i];
+    const double d2 = 2 * dot;
+    // the update, and the squares the next reflector starts from
+    s = 0;
+#pragma unroll
+    for (int i = k; i < MMAX; ++i) {
+      r[i] -= d2 * v[i];
+      if (i > k) s += r[i] * r[i];
+    }
+    // row k is final (columns before k hold leftovers there)
+    if (KEEP && on && gl >= k) sRt[tri(gl, k)] = r[k];
+  }
+  return ok;
+}
+
 // Rows of Q a lane holds at once, and the passes that cover MMAX rows: as
 // many rows as the registers take (each reflector entry read from LDS then
 // serves several rows, and the rows' independent sums hide each other's
@@ -159,7 +227,6 @@ __global__ __launch_bounds__(64, small_waves(NT, MMAX)) void k_qr_small(FitArgs 
   constexpr int G = NT, P = 64 / G;  // lanes per patch, patches per wave
   constexpr int RPL = small_rpl(NT, MMAX);
   constexpr int NPASS = (MMAX + G * RPL - 1) / (G * RPL);
-  constexpr int DIVS = (MMAX + G - 1) / G;
   constexpr int VS = NT * MMAX, NRT = NT * (NT + 1) / 2;
   // a patch's LDS: samples, then the reflectors V [NT][MMAX], then Q's
   // columns [MMAX][NT]; R's triangle; two norms.  The stride keeps the
@@ -205,60 +272,7 @@ __global__ __launch_bounds__(64, small_waves(NT, MMAX)) void k_qr_small(FitArgs 
       r[i] = i < rows ? v : 0.0;
     }
     __syncthreads();
-    bool ok = act;
-    double s = 0;  // the squares of the column, rows k on
-#pragma unroll
-    for (int i = 0; i < MMAX; ++i) s += r[i] * r[i];
-#pragma unroll
-    for (int k = 0; k < NT; ++k) {
-      // get_reflector on every lane's column; column k's is the one kept
-      const double cn = sqrt(s);
-      const double vk = r[k] + sgn(r[k]) * cn;
-      s = vk * vk;
-#pragma unroll
-      for (int i = k + 1; i < MMAX; ++i) s += r[i] * r[i];
-      if (on && gl == k) {
-        sN[0] = cn;
-        sN[1] = sqrt(s);
-        sV[k * MMAX + k] = vk;
-#pragma unroll
-        for (int i = k + 1; i < MMAX; ++i) sV[k * MMAX + i] = r[i];
-      }
-      __syncthreads();
-      ok = ok && !(sN[0] < 1e-10);
-      const double rn = sN[1];
-      // the lanes' divisions side by side (rows before k, whatever they
-      // hold, are not stored)
-      double w[DIVS];
-#pragma unroll
-      for (int u = 0; u < DIVS; ++u) {
-        const int i = gl + u * G;
-        w[u] = sV[k * MMAX + (i < MMAX ? i : MMAX - 1)] / rn;
-        asm volatile("" : "+v"(w[u]));  // formed here, not under the stores' conditions
-      }
-#pragma unroll
-      for (int u = 0; u < DIVS; ++u) {
-        const int i = gl + u * G;
-        if (on && i >= k && i < MMAX) sV[k * MMAX + i] = w[u];
-      }
-      __syncthreads();
-      double v[MMAX];
-#pragma unroll
-      for (int i = k; i < MMAX; ++i) v[i] = sV[k * MMAX + i];
-      double dot = 0;
-#pragma unroll
-      for (int i = k; i < MMAX; ++i) dot += r[i] * v[i];
-      const double d2 = 2 * dot;
-      // the update, and the squares the next reflector starts from
-      s = 0;
-#pragma unroll
-      for (int i = k; i < MMAX; ++i) {
-        r[i] -= d2 * v[i];
-        if (i > k) s += r[i] * r[i];
-      }
-      // row k is final (columns before k hold leftovers there)
-      if (on && gl >= k) sRt[tri(gl, k)] = r[k];
-    }
+    const bool ok = small_r<NT, MMAX, true>(r, sV, sN, sRt, gl, on, act);
     rank_failed<MODE>(a, act && !ok && gl == 0, p);
     // Q: rows gl, gl + G, ... of each pass
     double Qr[NPASS][RPL][NT];
@@ -362,6 +376,114 @@ __global__ __launch_bounds__(64, small_waves(NT, MMAX)) void k_qr_small(FitArgs 
         a.out[p * nc + c] = backsub_eval<NT>(y, [&](int i, int j) { return sRt[tri(j, i)]; }, node);
       }
     }
+    __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The reference's rank test of the initial sets that the fast forms could not
+// certify (xq entries with bit 31), before the expansion: six sets a wave.
+// A set of full rank becomes the patch's set; any other goes on to the
+// expansion without the test (bit 30: tested).  Sets above 32 rows and short
+// ones stay as they are.  Every entry's x_len is set (0: no set yet).
+// (The expansion's own test takes a wave per set, its sums on one lane: 15.9
+// ms for the 452,700 edge sets of a lattice box at n = 40, and 4.5 ms more to
+// queue them one by one; 1.08 ms here.)
+constexpr int TEST_ROWS = 32;
+
+template <int NT>
+__global__ __launch_bounds__(64, 2) void k_rank_test(FitArgs a)
+{
+  constexpr int ORDER = NT == 4 ? 1 : 2;
+  constexpr int G = NT, P = 64 / G, MMAX = TEST_ROWS;
+  constexpr int VS = 4 * MMAX;  // samples, then a reflector
+  constexpr int S = (VS + 2 + 31) / 32 * 32 + 2;
+  __shared__ double sm[P * S];
+  const int lane = threadIdx.x;
+  const int g = lane / G < P ? lane / G : P - 1;
+  int gl = lane - g * G;
+  const bool on = gl < G;
+  const int col = on ? gl : G - 1;
+  double* const sV = sm + g * S;
+  double* const sN = sV + VS;
+  int fa, fb;
+  term_pair(col, &fa, &fb);
+  const MeshView& m = a.m;
+  const int q = a.q;
+  const int nq = a.L.count[2 * NBUCKET];
+  for (int base = blockIdx.x * P; base < nq; base += gridDim.x * P) {
+    asm volatile("" : "+v"(gl));
+    const int it = base + g;
+    const int32_t entry = it < nq ? a.L.xq[it] : 0;
+    const int64_t p = entry & 0x7fffffff;
+    int ns = 0;
+    const int32_t* set = nullptr;
+    if (entry < 0) patch_set(a, p, &set, &ns);
+    const bool act = entry < 0 && ns * q >= NT && ns * q <= MMAX;
+    const int rows = act ? ns * q : 0;
+    int mw = rows;  // the wave's longest set
+    for (int o = 32; o > 0; o >>= 1) {
+      const int y = __shfl(mw, lane ^ o);
+      mw = y > mw ? y : mw;
+    }
+    mw = __builtin_amdgcn_readlane(mw, 0);
+    bool ok = false;
+    if (mw > 0) {  // wave-uniform
+      if (on && act)
+        for (int s = gl; s < ns; s += G) sample_tet<ORDER>(m, set[s], q, sV + 4 * s * q);
+      __syncthreads();
+      auto test = [&](auto size) {
+        constexpr int M = decltype(size)::value;
+        double r[M];
+#pragma unroll
+        for (int i = 0; i < M; ++i) {
+          const double v = sV[4 * i + fa] * sV[4 * i + fb];
+          r[i] = i < rows ? v : 0.0;
+        }
+        __syncthreads();
+        ok = small_r<NT, M, false>(r, sV, sN, nullptr, gl, on, act);
+      };
+      if (mw <= 16)
+        test(std::integral_constant<int, 16>());
+      else if (mw <= 24)
+        test(std::integral_constant<int, 24>());
+      else
+        test(std::integral_constant<int, 32>());
+    }
+    // places in x_set for the wave's full-rank sets, one atomic per wave
+    const bool head = on && gl == 0 && it < nq;
+    const int len = head && ok ? ns : 0;
+    int end = len;  // inclusive sum over the lanes
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl(end, lane - o);
+      if (lane >= o) end += y;
+    }
+    const int total = __builtin_amdgcn_readlane(end, 63);
+    int64_t off = 0;
+    if (total > 0) {
+      int lo = 0, hi = 0;
+      if (lane == 0) {
+        const unsigned long long at = atomicAdd((unsigned long long*)a.L.x_cursor, (unsigned long long)total);
+        lo = (int)(uint32_t)at;
+        hi = (int)(uint32_t)(at >> 32);
+      }
+      lo = __builtin_amdgcn_readlane(lo, 0);
+      hi = __builtin_amdgcn_readlane(hi, 0);
+      off = (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo) + end - len;
+    }
+    if (head) {
+      const bool room = off + len <= a.L.x_cap;
+      if (len > 0 && !room) atomicOr(a.L.status, ST_XSET_OVERFLOW);
+      a.L.x_len[it] = room ? len : 0;
+      if (len > 0 && room) {
+        a.L.x_patch[it] = (int32_t)p;
+        a.L.x_off[it] = off;
+        for (int i = 0; i < len; ++i) a.L.x_set[off + i] = set[i];
+      }
+      if (act && !ok) a.L.xq[it] = (int32_t)(p | 0x40000000);
+    }
+    const uint64_t tested = __ballot(head && act);
+    if (lane == 0 && tested) atomicAdd(a.L.status + 4, __popcll(tested));
     __syncthreads();
   }
 }
@@ -769,6 +891,17 @@ int launch_qr_regular(const FitArgs& a, int nterms, const int64_t* count, void* 
 {
   double* const w = static_cast<double*>(ws);
   return nterms == 4 ? regular_fits<4>(a, count, w, ws_bytes, s) : regular_fits<10>(a, count, w, ws_bytes, s);
+}
+
+int launch_rank_test(const FitArgs& a, int nterms, hipStream_t s)
+{
+  const int P = nterms == 4 ? 16 : 6;
+  const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(a.shape.expand_blocks, (a.npatch + P - 1) / P));
+  if (nterms == 4)
+    k_rank_test<4><<<blocks, 64, 0, s>>>(a);
+  else
+    k_rank_test<10><<<blocks, 64, 0, s>>>(a);
+  return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "rank test launch failed");
 }
 
 int launch_qr_lists(const FitArgs& a, int nterms, int mode, hipStream_t s)

@@ -674,8 +674,10 @@ void carve_lists(const sprg_mesh* m, char* base, int64_t cap, int32_t* x_set, in
   L.x_cursor = x_cursor;
   L.count = p;
   p += 2 * NBUCKET + 2;
-  L.status = p;  // [0] status bits, [1] exact-expansion count, [2] fallback entries taken before the expansion
-  p += 4;
+  // [0] status bits, [1] exact-expansion count, [2] fallback entries taken
+  // before the expansion, [3] big-list count, [4] sets k_rank_test tested
+  L.status = p;
+  p += 5;
   int32_t* const items = p;
   p += cap;
   for (int b = 0; b < NBUCKET; ++b) { L.xitems[b] = p; p += cap; }
@@ -744,7 +746,7 @@ int read_status(sprg_mesh* m, const FitArgs& a, int32_t* st)
   hipStream_t s = m->ctx->stream;
   // counts [0, 2 NBUCKET + 2), the status word and the exact-expansion
   // count follow each other
-  int32_t c[2 * NBUCKET + 6];
+  int32_t c[2 * NBUCKET + 7];
   HIP_OK(hipMemcpyAsync(c, a.L.count, sizeof c, hipMemcpyDeviceToHost, s), "status");
   HIP_OK(hipStreamSynchronize(s), "recover sync");
   *st = c[2 * NBUCKET + 2];
@@ -755,7 +757,7 @@ int read_status(sprg_mesh* m, const FitArgs& a, int32_t* st)
   m->last_stats[2] = expanded;
   m->last_stats[3] = c[2 * NBUCKET + 1];
   m->last_stats[4] = *st;
-  m->last_stats[5] = c[2 * NBUCKET + 3];
+  m->last_stats[5] = c[2 * NBUCKET + 3] + c[2 * NBUCKET + 6];
   m->last_stats[6] = c[2 * NBUCKET + 5];
   return 0;
 }
@@ -775,8 +777,9 @@ int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, void* qr_ws, size_
   const int nterms = m->order == 1 ? 4 : 10;
   int rc;
   // counters, status, the exact-expansion count and the fallback start
-  // (the status words follow the counters: bits, exact count, fallback start, big count)
-  if ((rc = launch_copy_i32(a.L.count, nullptr, 2 * NBUCKET + 6, s))) return rc;
+  // (the status words follow the counters: bits, exact count, fallback start,
+  // big count, rank-tested count)
+  if ((rc = launch_copy_i32(a.L.count, nullptr, 2 * NBUCKET + 7, s))) return rc;
   if ((rc = launch_copy_i32(reinterpret_cast<int32_t*>(a.L.x_cursor), nullptr, 4, s))) return rc;
   if (marks) {
     m->phase_last = 0;
@@ -804,6 +807,7 @@ int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, void* qr_ws, size_
     if ((rc = launch_qr_regular(a, nterms, count, qr_ws, qr_bytes, s))) return rc;
   }
   if (marks) m->mark(1);
+  if (fast && (rc = launch_rank_test(a, nterms, s))) return rc;
   if ((rc = launch_expand(a, nterms, s))) return rc;
   if (marks) m->mark(2);
   if (fast) {
