@@ -190,7 +190,7 @@ int launch_classify(const FitArgs& a, int nterms, hipStream_t s);
 size_t qr_ws_bytes(int nterms, const int64_t* count);
 int launch_qr_regular(const FitArgs& a, int nterms, const int64_t* count, void* ws, size_t ws_bytes, hipStream_t s);
 int launch_qr_lists(const FitArgs& a, int nterms, int mode, hipStream_t s);
-// Buckets of more than 32 rows of the same lists (k_exact.hip).
+// The buckets of more than 32 rows of the same lists (k_exact.hip).
 int launch_exact_lists(const FitArgs& a, int nterms, int mode, hipStream_t s);
 // Before launch_expand in the fast forms: the rank test of queued initial sets
 // of up to 32 rows (k_qr.hip).
@@ -229,6 +229,15 @@ struct EstArgs {
   double* scalars;     // [4]: self, errsum|G, size_factor, spare
   double* size;        // [nv]
   int nblocks;
+  // the recovery before: its counters [ncounts], copied to report_counts, and
+  // its status word, copied to report_status if that is not null; report_sc
+  // [3] gets the scalars
+  const int32_t* counts;
+  const int32_t* status;
+  int ncounts;
+  int32_t* report_counts;
+  int32_t* report_status;
+  double* report_sc;
 };
 // mark(i) records phase event i on the stream (3: before the element pass,
 // 4: after it, 5: after the vertex average).

@@ -290,12 +290,12 @@ __global__ __launch_bounds__(EST_T, elem_waves(IPO, NC)) void k_element(EstArgs 
   }
 }
 
-// Fixed-order reduction of the block partials, then the size factor
+// Fixed-order reduction of the block partials by a block, then the size factor
 // (computeSizeFactor, spr/sprEstimateError.cc:205-217;
-// target::computeSizeFactor, spr/sprEstimateTargetError.cc:129-137).
-__global__ __launch_bounds__(EST_T) void k_factor(EstArgs a)
+// target::computeSizeFactor, spr/sprEstimateTargetError.cc:129-137), on
+// thread 0: sc = ||eps*||^2, the error sum, the factor.
+__device__ __forceinline__ void size_factor(const EstArgs& a, double (*red)[EST_T], double* sc)
 {
-  __shared__ double red[2][EST_T];
   double s0 = 0, s1 = 0;
   // each thread's partials in order, eight loads in flight at a time
   int i = threadIdx.x;
@@ -339,20 +339,49 @@ __global__ __launch_bounds__(EST_T) void k_factor(EstArgs a)
       int d = 3;
       sf = pow((glob / a.target_n), (1.0 / d));
     }
-    a.scalars[0] = self;
-    a.scalars[1] = glob;
-    a.scalars[2] = sf;
+    sc[0] = self;
+    sc[1] = glob;
+    sc[2] = sf;
   }
 }
 
+__global__ __launch_bounds__(EST_T) void k_factor(EstArgs a)
+{
+  __shared__ double red[2][EST_T];
+  size_factor(a, red, a.scalars);
+}
+
+// Up to this many block partials every block of the vertex average forms the
+// size factor itself (the same sums in the same order), four loads a thread
+// from the L2, instead of a launch of its own (about 5 us of a small call).
+constexpr int FACTOR_INLINE = 1024;
+
 // averageToVertex / avgToVtx (spr/sprEstimateError.cc:255-265,
 // spr/sprEstimateTargetError.cc:180-190), summing in ascending tet order.
-__global__ void k_average(EstArgs a)
+// FACTOR: the block forms the size factor first.  Block 0 reports: the
+// counters and status of the recovery before, and the scalars.  A recovery
+// that failed leaves the sizes alone.
+template <bool FACTOR>
+__global__ __launch_bounds__(EST_T) void k_average(EstArgs a)
 {
   const MeshView& m = a.m;
+  __shared__ double sc[3];
+  if constexpr (FACTOR) {
+    __shared__ double red[2][EST_T];
+    size_factor(a, red, sc);
+  } else {
+    if (threadIdx.x < 3) sc[threadIdx.x] = a.scalars[threadIdx.x];
+  }
+  __syncthreads();
+  if (blockIdx.x == 0) {
+    if (threadIdx.x < 3) a.report_sc[threadIdx.x] = sc[threadIdx.x];
+    if ((int)threadIdx.x < a.ncounts) a.report_counts[threadIdx.x] = a.counts[threadIdx.x];
+    if (threadIdx.x == 0 && a.report_status) *a.report_status = *a.status;
+  }
+  if (*a.status != 0) return;
   const int64_t v = xcd_block(blockIdx.x, gridDim.x, avg_chunk(gridDim.x)) * blockDim.x + threadIdx.x;
   if (v >= m.nv) return;
-  const double sf = a.scalars[2];
+  const double sf = sc[2];
   const int32_t b = m.v2t_off[v], e = m.v2t_off[v + 1];
   auto elem_size = [&](int32_t t) {
     if (!a.target) return a.elem[t] * sf;
@@ -463,8 +492,13 @@ int launch_estimate(EstArgs& a, hipStream_t s, const std::function<void(int)>& m
   rc = a.m.order == 1 ? launch_element_ipo<1>(a, s) : launch_element_ipo<2>(a, s);
   if (rc) return rc;
   mark(4);
-  k_factor<<<1, EST_T, 0, s>>>(a);
-  k_average<<<(unsigned)((a.m.nv + 255) / 256), 256, 0, s>>>(a);
+  const unsigned blocks = (unsigned)((a.m.nv + EST_T - 1) / EST_T);
+  if (a.nblocks <= FACTOR_INLINE) {
+    k_average<true><<<blocks, EST_T, 0, s>>>(a);
+  } else {
+    k_factor<<<1, EST_T, 0, s>>>(a);
+    k_average<false><<<blocks, EST_T, 0, s>>>(a);
+  }
   mark(5);
   return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "estimate launch failed");
 }

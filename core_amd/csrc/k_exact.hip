@@ -248,21 +248,23 @@ __global__ __launch_bounds__(CL_T) void k_classify(FitArgs a, int nterms)
   }
 }
 
-// The Q row of MMAX doubles per lane sets the floor of the register budget:
-// two waves per SIMD where that compiles without scratch spills.
-constexpr int exact_waves(int nt, int mmax) { return nt == 10 && mmax == 96 ? 2 : 1; }
+// A wave's LDS (doubles) for sets of up to MMAX rows.
+constexpr int exact_lds(int nt, int mmax) { return 2 * nt * mmax + nt * nt + 27 * nt + nt + 3 + mmax / 2; }
 
+// The fits of one bucket's list, the launch's blocks (one wave each) taking
+// sets in turn.
 template <int NT, int MMAX, int LANES, int MODE>
-__global__ __launch_bounds__(64, exact_waves(NT, MMAX)) void k_exact_fit(FitArgs a, int bucket)
+__device__ __forceinline__ void exact_fit(const FitArgs& a, int bucket, double* sm)
 {
   constexpr int G = 64 / LANES;
-  __shared__ double sR[G][MMAX * NT];
-  __shared__ double sV[G][NT * MMAX];
-  __shared__ double sRt[G][NT * NT];
-  __shared__ double sY[G][27 * NT];
-  __shared__ double sDot[G][NT];
-  __shared__ double sNorm[G][3];
-  __shared__ int32_t sS[G][MMAX];
+  static_assert(G == 1, "one set per wave");
+  double (*const sR)[MMAX * NT] = reinterpret_cast<double (*)[MMAX * NT]>(sm);
+  double (*const sV)[MMAX * NT] = reinterpret_cast<double (*)[MMAX * NT]>(sm + MMAX * NT);
+  double (*const sRt)[NT * NT] = reinterpret_cast<double (*)[NT * NT]>(sm + 2 * MMAX * NT);
+  double (*const sY)[27 * NT] = reinterpret_cast<double (*)[27 * NT]>(sm + 2 * MMAX * NT + NT * NT);
+  double (*const sDot)[NT] = reinterpret_cast<double (*)[NT]>(sm + 2 * MMAX * NT + NT * NT + 27 * NT);
+  double (*const sNorm)[3] = reinterpret_cast<double (*)[3]>(sm + 2 * MMAX * NT + NT * NT + 28 * NT);
+  int32_t (*const sS)[MMAX] = reinterpret_cast<int32_t (*)[MMAX]>(sm + 2 * MMAX * NT + NT * NT + 28 * NT + 3);
   const int g = threadIdx.x / LANES, gl = threadIdx.x % LANES;
   const MeshView& m = a.m;
   const int q = a.q, nc = a.nc;
@@ -718,9 +720,9 @@ __global__ __launch_bounds__(64) void k_expand(FitArgs a)
   }
 }
 
-// The expanded sets found (x_len > 0) into the lists the fits walk: by row
-// bucket in the FP64 form, one list in the fast forms.  Wave-aggregated
-// appends; also publishes the item count (one id per queued patch).
+// The expanded sets found (x_len > 0) into the exact fits' lists, by row
+// bucket.  Wave-aggregated appends; also publishes the item count (one id per
+// queued patch).
 __global__ __launch_bounds__(256) void k_bucket_items(FitArgs a)
 {
   const int nq = a.L.count[2 * NBUCKET];
@@ -733,7 +735,7 @@ __global__ __launch_bounds__(256) void k_bucket_items(FitArgs a)
     if (it < nq) {
       const int len = a.L.x_len[it];
       if (len > 0) {
-        target = a.fast ? 0 : bucket_of(len * a.q);
+        target = bucket_of(len * a.q);
         if (target >= NBUCKET) {
           atomicOr(a.L.status, ST_TOO_LARGE);
           target = -1;
@@ -846,18 +848,23 @@ __global__ __launch_bounds__(64) void k_exact_big(FitArgs a, double* ws)
 
 inline unsigned grid_for(int64_t n, int per) { return (unsigned)((n + per - 1) / per); }
 
+// The lists above 32 rows in one launch (their lengths are the device's, and
+// mostly zero).
+template <int NT, int MODE>
+__global__ __launch_bounds__(64, 1) void k_exact_fit(FitArgs a)
+{
+  __shared__ double sm[exact_lds(NT, 192)];
+  static_assert(NSMALL == 3 && NBUCKET == 7, "the buckets below");
+  exact_fit<NT, 64, 64, MODE>(a, 3, sm);
+  exact_fit<NT, 96, 64, MODE>(a, 4, sm);
+  exact_fit<NT, 128, 64, MODE>(a, 5, sm);
+  exact_fit<NT, 192, 64, MODE>(a, 6, sm);
+}
+
 template <int NT, int MODE>
 int fit_lists(const FitArgs& a, hipStream_t s)
 {
-  // Persistent grids: each block loops over its share of the bucket's
-  // device-side item count.
-  const unsigned blocks = (unsigned)std::min<int64_t>(a.shape.exact_blocks, a.npatch);
-  const unsigned quarter = blocks / 4 > 0 ? blocks / 4 : 1;  // the 192-row bucket is rare
-  static_assert(NSMALL == 3 && NBUCKET == 7, "the buckets below");
-  k_exact_fit<NT, 64, 64, MODE><<<blocks, 64, 0, s>>>(a, 3);
-  k_exact_fit<NT, 96, 64, MODE><<<blocks, 64, 0, s>>>(a, 4);
-  k_exact_fit<NT, 128, 64, MODE><<<blocks, 64, 0, s>>>(a, 5);
-  k_exact_fit<NT, 192, 64, MODE><<<quarter, 64, 0, s>>>(a, 6);
+  k_exact_fit<NT, MODE><<<(unsigned)std::min<int64_t>(a.shape.exact_blocks, a.npatch), 64, 0, s>>>(a);
   return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "exact fit launch failed");
 }
 
@@ -901,7 +908,8 @@ int launch_expand(const FitArgs& a, int nterms, hipStream_t s)
     k_expand<10, false><<<blocks, 64, 0, s>>>(a);
     k_expand<10, true><<<exact_blocks, 64, 0, s>>>(a);
   }
-  k_bucket_items<<<256, 256, 0, s>>>(a);
+  // the fast forms walk the queue itself (k_fast)
+  if (!a.fast) k_bucket_items<<<256, 256, 0, s>>>(a);
   return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "expand launch failed");
 }
 

@@ -142,7 +142,8 @@ __device__ __forceinline__ void sample_d(const MeshView& m, const Geo<P2MAP>& g,
 enum { SRC_REGULAR = 0, SRC_EXPANDED = 1, SRC_FALLBACK = 2, SRC_PRE_FALLBACK = 3, SRC_LEFTOVER = 4 };
 
 
-// src SRC_REGULAR walks every patch id (no list); the others walk a list.
+// src SRC_REGULAR walks every patch id and SRC_EXPANDED every queued item; the
+// others walk a list.
 template <class T, int NT, int NC, int NREF, bool P2MAP>
 __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank, float tau_acc)
 {
@@ -150,10 +151,10 @@ __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank
   const int q = a.q;
   constexpr bool p2map = P2MAP;
   const bool regular = src == SRC_REGULAR || src == SRC_LEFTOVER;
-  const int32_t* list = src == SRC_EXPANDED ? a.L.xitems[0] : src == SRC_LEFTOVER ? a.tiles.leftover : a.L.fbq;
+  const int32_t* list = src == SRC_LEFTOVER ? a.tiles.leftover : a.L.fbq;
   const int64_t count = src == SRC_REGULAR    ? a.npatch
                         : src == SRC_LEFTOVER ? a.tiles.nleftover
-                        : src == SRC_EXPANDED ? a.L.count[NBUCKET]
+                        : src == SRC_EXPANDED ? a.L.count[2 * NBUCKET]
                                               : a.L.count[2 * NBUCKET + 1];
   const int64_t first = src == SRC_FALLBACK ? a.L.status[2] : 0;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -162,8 +163,13 @@ __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank
   for (int64_t base = first + xcd_block(blockIdx.x, gridDim.x, XCD_K_FIT) * blockDim.x; base < count;
        base += stride) {
     const int64_t it = base + threadIdx.x;
-    const bool valid = it < count;
-    const int32_t entry = !valid ? 0 : src == SRC_REGULAR ? (int32_t)it : list[it];
+    // the expanded sets are the expansion queue's items that found one
+    const bool valid = it < count && (src != SRC_EXPANDED || a.L.x_len[it] > 0);
+    const int32_t entry = !valid ? 0 : src == SRC_REGULAR || src == SRC_EXPANDED ? (int32_t)it : list[it];
+    if (src == SRC_EXPANDED) {
+      const uint64_t found = __ballot(valid);
+      if ((threadIdx.x & 63) == 0 && found) atomicAdd(a.L.count + NBUCKET, __popcll(found));
+    }
     const bool expanded =
         src == SRC_EXPANDED || ((src == SRC_FALLBACK || src == SRC_PRE_FALLBACK) && entry < 0);
     const int32_t id = entry & 0x7fffffff;

@@ -220,20 +220,23 @@ constexpr int small_rpl(int nt, int mmax)
 }
 constexpr int small_waves(int nt, int mmax) { return mmax == 16 ? 3 : 2; }
 
+// A wave's LDS (doubles): per patch its samples, then the reflectors V
+// [NT][MMAX], then Q's columns [MMAX][NT]; R's triangle; two norms; its tets.
+// The stride keeps the patches' equal offsets 16 bytes apart modulo the banks.
+constexpr int small_stride(int nt, int mmax) { return (nt * mmax + nt * (nt + 1) / 2 + 2 + mmax / 2 + 31) / 32 * 32 + 2; }
+constexpr int small_lds(int nt, int mmax) { return 64 / nt * small_stride(nt, mmax); }
+
+// The fits of one bucket's list, the launch's blocks (one wave each) taking
+// 64 / NT patches in turn.
 template <int NT, int MMAX, int MODE>
-__global__ __launch_bounds__(64, small_waves(NT, MMAX)) void k_qr_small(FitArgs a, int bucket)
+__device__ __forceinline__ void small_fit(const FitArgs& a, int bucket, double* sm)
 {
   constexpr int ORDER = NT == 4 ? 1 : 2;
   constexpr int G = NT, P = 64 / G;  // lanes per patch, patches per wave
   constexpr int RPL = small_rpl(NT, MMAX);
   constexpr int NPASS = (MMAX + G * RPL - 1) / (G * RPL);
   constexpr int VS = NT * MMAX, NRT = NT * (NT + 1) / 2;
-  // a patch's LDS: samples, then the reflectors V [NT][MMAX], then Q's
-  // columns [MMAX][NT]; R's triangle; two norms.  The stride keeps the
-  // patches' equal offsets 16 bytes apart modulo the banks.
-  constexpr int S = (VS + NRT + 2 + 31) / 32 * 32 + 2;
-  __shared__ double sm[P * S];
-  __shared__ int32_t sSet[P * MMAX];
+  constexpr int S = small_stride(NT, MMAX);
   const int lane = threadIdx.x;
   const int g = lane / G < P ? lane / G : P - 1;
   int gl = lane - g * G;
@@ -242,7 +245,7 @@ __global__ __launch_bounds__(64, small_waves(NT, MMAX)) void k_qr_small(FitArgs 
   double* const sV = sm + g * S;
   double* const sRt = sV + VS;
   double* const sN = sRt + NRT;
-  int32_t* const sS = sSet + g * MMAX;
+  int32_t* const sS = reinterpret_cast<int32_t*>(sN + 2);
   int fa, fb;
   term_pair(col, &fa, &fb);
   const MeshView& m = a.m;
@@ -378,6 +381,25 @@ __global__ __launch_bounds__(64, small_waves(NT, MMAX)) void k_qr_small(FitArgs 
     }
     __syncthreads();
   }
+}
+
+template <int NT, int MMAX, int MODE>
+__global__ __launch_bounds__(64, small_waves(NT, MMAX)) void k_qr_small(FitArgs a, int bucket)
+{
+  __shared__ double sm[small_lds(NT, MMAX)];
+  small_fit<NT, MMAX, MODE>(a, bucket, sm);
+}
+
+// The lists whose lengths only the device knows, in one launch (most calls
+// have few sets here or none, and an empty launch costs what a full one waits
+// for).
+template <int NT, int MODE>
+__global__ __launch_bounds__(64, 2) void k_qr_small_lists(FitArgs a)
+{
+  __shared__ double sm[small_lds(NT, 32)];
+  small_fit<NT, 16, MODE>(a, 0, sm);
+  small_fit<NT, 24, MODE>(a, 1, sm);
+  small_fit<NT, 32, MODE>(a, 2, sm);
 }
 
 // ---------------------------------------------------------------------------
@@ -833,19 +855,6 @@ __global__ __launch_bounds__(256) void k_qr_solve(FitArgs a, int bucket, int fir
 // (the reflectors and Q of 36,864 96-row sets take 596 MB).
 constexpr int64_t QR_CHUNK = 36864;
 
-template <int NT, int MODE>
-void small_fits(const FitArgs& a, const int64_t* count, hipStream_t s)
-{
-  constexpr int P = 64 / NT;
-  auto blocks = [&](int b) {
-    const int64_t n = count ? count[b] : a.npatch;
-    return (unsigned)std::max<int64_t>(1, std::min<int64_t>(a.shape.exact_blocks, (n + P - 1) / P));
-  };
-  if (!count || count[0]) k_qr_small<NT, 16, MODE><<<blocks(0), 64, 0, s>>>(a, 0);
-  if (!count || count[1]) k_qr_small<NT, 24, MODE><<<blocks(1), 64, 0, s>>>(a, 1);
-  if (!count || count[2]) k_qr_small<NT, 32, MODE><<<blocks(2), 64, 0, s>>>(a, 2);
-}
-
 template <int NT, int MMAX>
 void large_fits(const FitArgs& a, int bucket, int64_t count, double* ws, size_t ws_bytes, hipStream_t s)
 {
@@ -869,7 +878,11 @@ int regular_fits(const FitArgs& a, const int64_t* count, double* ws, size_t ws_b
   for (int b = NSMALL; b < NBUCKET; ++b)
     if (count[b] && ws_bytes < qr_set_bytes(NT, bucket_rows(b)))
       return sprg_fail(SPRG_ENOMEM, "exact fit: no workspace for a set of %d rows", bucket_rows(b));
-  small_fits<NT, FIT_REGULAR>(a, count, s);
+  constexpr int P = 64 / NT;
+  auto blocks = [&](int b) { return (unsigned)std::min<int64_t>(a.shape.exact_blocks, (count[b] + P - 1) / P); };
+  if (count[0]) k_qr_small<NT, 16, FIT_REGULAR><<<blocks(0), 64, 0, s>>>(a, 0);
+  if (count[1]) k_qr_small<NT, 24, FIT_REGULAR><<<blocks(1), 64, 0, s>>>(a, 1);
+  if (count[2]) k_qr_small<NT, 32, FIT_REGULAR><<<blocks(2), 64, 0, s>>>(a, 2);
   large_fits<NT, 64>(a, 3, count[3], ws, ws_bytes, s);
   large_fits<NT, 96>(a, 4, count[4], ws, ws_bytes, s);
   large_fits<NT, 128>(a, 5, count[5], ws, ws_bytes, s);
@@ -907,10 +920,18 @@ int launch_rank_test(const FitArgs& a, int nterms, hipStream_t s)
 int launch_qr_lists(const FitArgs& a, int nterms, int mode, hipStream_t s)
 {
   if (a.npatch == 0) return 0;
+  const int P = nterms == 4 ? 16 : 6;
+  const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(a.shape.exact_blocks, (a.npatch + P - 1) / P));
   if (mode == FIT_EXPANDED) {
-    if (nterms == 4) small_fits<4, FIT_EXPANDED>(a, nullptr, s); else small_fits<10, FIT_EXPANDED>(a, nullptr, s);
+    if (nterms == 4)
+      k_qr_small_lists<4, FIT_EXPANDED><<<blocks, 64, 0, s>>>(a);
+    else
+      k_qr_small_lists<10, FIT_EXPANDED><<<blocks, 64, 0, s>>>(a);
   } else {
-    if (nterms == 4) small_fits<4, FIT_MIXED>(a, nullptr, s); else small_fits<10, FIT_MIXED>(a, nullptr, s);
+    if (nterms == 4)
+      k_qr_small_lists<4, FIT_MIXED><<<blocks, 64, 0, s>>>(a);
+    else
+      k_qr_small_lists<10, FIT_MIXED><<<blocks, 64, 0, s>>>(a);
   }
   if (hipGetLastError() != hipSuccess) return sprg_fail(SPRG_EHIP, "exact fit launch failed");
   return launch_exact_lists(a, nterms, mode, s);

@@ -741,24 +741,31 @@ int setup_lists(sprg_mesh* m, FitArgs& a, DBuf& ws)
   return 0;
 }
 
-int read_status(sprg_mesh* m, const FitArgs& a, int32_t* st)
+// counts [0, 2 NBUCKET + 2) and the status words follow each other
+constexpr int NCOUNTS = 2 * NBUCKET + 7;
+
+// The counters and status words of a finished recovery into last_stats.
+int32_t keep_status(sprg_mesh* m, int64_t npatch, const int32_t* c)
 {
-  hipStream_t s = m->ctx->stream;
-  // counts [0, 2 NBUCKET + 2), the status word and the exact-expansion
-  // count follow each other
-  int32_t c[2 * NBUCKET + 7];
-  HIP_OK(hipMemcpyAsync(c, a.L.count, sizeof c, hipMemcpyDeviceToHost, s), "status");
-  HIP_OK(hipStreamSynchronize(s), "recover sync");
-  *st = c[2 * NBUCKET + 2];
   int64_t expanded = 0;
   for (int b = 0; b < NBUCKET; ++b) expanded += c[NBUCKET + b];
-  m->last_stats[0] = a.npatch;
+  m->last_stats[0] = npatch;
   m->last_stats[1] = c[2 * NBUCKET];
   m->last_stats[2] = expanded;
   m->last_stats[3] = c[2 * NBUCKET + 1];
-  m->last_stats[4] = *st;
+  m->last_stats[4] = c[2 * NBUCKET + 2];
   m->last_stats[5] = c[2 * NBUCKET + 3] + c[2 * NBUCKET + 6];
   m->last_stats[6] = c[2 * NBUCKET + 5];
+  return c[2 * NBUCKET + 2];
+}
+
+int read_status(sprg_mesh* m, const FitArgs& a, int32_t* st)
+{
+  hipStream_t s = m->ctx->stream;
+  int32_t c[NCOUNTS];
+  HIP_OK(hipMemcpyAsync(c, a.L.count, sizeof c, hipMemcpyDeviceToHost, s), "status");
+  HIP_OK(hipStreamSynchronize(s), "recover sync");
+  *st = keep_status(m, a.npatch, c);
   return 0;
 }
 
@@ -776,11 +783,9 @@ int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, void* qr_ws, size_
   const bool fast = form != SPRG_FP64;
   const int nterms = m->order == 1 ? 4 : 10;
   int rc;
-  // counters, status, the exact-expansion count and the fallback start
-  // (the status words follow the counters: bits, exact count, fallback start,
-  // big count, rank-tested count)
-  if ((rc = launch_copy_i32(a.L.count, nullptr, 2 * NBUCKET + 7, s))) return rc;
-  if ((rc = launch_copy_i32(reinterpret_cast<int32_t*>(a.L.x_cursor), nullptr, 4, s))) return rc;
+  // the expanded sets' cursors, the counters and the status words (bits, exact
+  // count, fallback start, big count, rank-tested count) follow each other
+  if ((rc = launch_copy_i32(reinterpret_cast<int32_t*>(a.L.x_cursor), nullptr, 4 + NCOUNTS, s))) return rc;
   if (marks) {
     m->phase_last = 0;
     m->mark(0);
@@ -812,7 +817,9 @@ int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, void* qr_ws, size_
   if (marks) m->mark(2);
   if (fast) {
     if ((rc = launch_fast_fit(a, nterms, form, 1, s))) return rc;
-    if ((rc = launch_fast_fit(a, nterms, form, 2, s))) return rc;
+    // (an FP64 pass leaves to it only sets above the exact kernels' rows)
+    if ((form == SPRG_FP32R || (int64_t)m->max_set * a.q > BIG_MMAX) && (rc = launch_fast_fit(a, nterms, form, 2, s)))
+      return rc;
     // poorly conditioned sets: the reference's arithmetic
     if ((rc = launch_qr_lists(a, nterms, 2, s))) return rc;
   } else {
@@ -864,11 +871,17 @@ int status_code(sprg_mesh* m, int32_t st, bool* retry)
   return 0;
 }
 
-int run_recover(sprg_mesh* m, int q, int nc, const double* ip, double* out, int form)
+int check_form(int form, int q)
 {
   if (!valid_form(form)) return sprg_fail(SPRG_EINVAL, "unknown numeric form %d", form);
   if (form != SPRG_FP64 && q > 4)
     return sprg_fail(SPRG_EUNSUPPORTED, "the fast forms take at most 4 points per element");
+  return 0;
+}
+
+int run_recover(sprg_mesh* m, int q, int nc, const double* ip, double* out, int form)
+{
+  if (int rc = check_form(form, q)) return rc;
   hipStream_t s = m->ctx->stream;
   for (int attempt = 0; attempt < 4; ++attempt) {
     FitArgs a = fit_args(m, q, nc, ip, out, form);
@@ -891,9 +904,7 @@ int run_recover(sprg_mesh* m, int q, int nc, const double* ip, double* out, int 
 // scratch holds the expanded sets.
 int run_recover_noalloc(sprg_mesh* m, int q, int nc, const double* ip, double* out, int form)
 {
-  if (!valid_form(form)) return sprg_fail(SPRG_EINVAL, "unknown numeric form %d", form);
-  if (form != SPRG_FP64 && q > 4)
-    return sprg_fail(SPRG_EUNSUPPORTED, "the fast forms take at most 4 points per element");
+  if (int rc = check_form(form, q)) return rc;
   char* base = static_cast<char*>(m->ctx->scratch);
   if (!base) return sprg_fail(SPRG_EHIP, "recover_noalloc: no scratch on this context's device");
   const int64_t np = m->npatch();
@@ -976,6 +987,13 @@ extern "C" int sprg_recover_noalloc(sprg_mesh* m, int ip_order, int nc, const do
 
 namespace {
 
+// What a size-field call brings back to the host, in one copy (after the
+// scalars in their buffer).
+struct Report {
+  double sc[3];
+  int32_t counts[NCOUNTS];
+};
+
 // Buffers of one size-field call (recovered field, element sizes, block
 // partials, scalars): allocated before any capture.
 int estimate_buffers(sprg_mesh* m, int nc)
@@ -985,14 +1003,23 @@ int estimate_buffers(sprg_mesh* m, int nc)
   if ((rc = m->rec.ensure(sizeof(double) * m->nnodes * nc))) return rc;
   if ((rc = m->elem.ensure(sizeof(double) * 2 * m->nt))) return rc;
   if ((rc = m->partial.ensure(sizeof(double) * 2 * nblocks))) return rc;
-  if ((rc = m->scalars.ensure(sizeof(double) * 4))) return rc;
+  if ((rc = m->scalars.ensure(sizeof(double) * 4 + sizeof(Report)))) return rc;
   return 0;
 }
 
-EstArgs est_args(sprg_mesh* m, int ip_order, int nc, const double* ip, int target, double ar,
-                 double tn, double alpha, double beta, double* size)
+// L: the work lists of the recovery before; status_out: null, or where its
+// status word goes.
+EstArgs est_args(sprg_mesh* m, const Lists& L, int ip_order, int nc, const double* ip, int target, double ar,
+                 double tn, double alpha, double beta, double* size, int32_t* status_out)
 {
   EstArgs e;
+  Report* const r = reinterpret_cast<Report*>(m->scalars.as<double>() + 4);
+  e.counts = L.count;
+  e.status = L.status;
+  e.ncounts = NCOUNTS;
+  e.report_counts = r->counts;
+  e.report_status = status_out;
+  e.report_sc = r->sc;
   e.m = m->view();
   e.ip_order = ip_order;
   e.nc = nc;
@@ -1021,15 +1048,28 @@ int run_estimate(sprg_mesh* m, int ip_order, int nc, const double* ip, int targe
   if (nc != 1 && nc != 3 && nc != 9 && nc != 27)
     return sprg_fail(SPRG_EUNSUPPORTED, "estimator: %d components", nc);
   HIP_OK(hipSetDevice(m->ctx->device), "hipSetDevice");
+  if ((rc = check_form(form, q))) return rc;
   if ((rc = estimate_buffers(m, nc))) return rc;
-  if ((rc = run_recover(m, q, nc, ip, m->rec.as<double>(), form))) return rc;
-  EstArgs e = est_args(m, ip_order, nc, ip, target, ar, tn, alpha, beta, size);
-  if ((rc = launch_estimate(e, m->ctx->stream, [m](int i) { m->mark(i); }))) return rc;
-  double sc[4] = {0, 0, 0, 0};
-  HIP_OK(hipMemcpyAsync(sc, e.scalars, sizeof(double) * 3, hipMemcpyDeviceToHost, m->ctx->stream),
-         "scalars");
-  HIP_OK(hipStreamSynchronize(m->ctx->stream), "estimate sync");
-  collect_phases(m);
+  // recovery and estimate without a wait between them: the estimate of a
+  // recovery that failed is not used (and writes no sizes)
+  hipStream_t s = m->ctx->stream;
+  double sc[3] = {0, 0, 0};
+  bool retry = true;
+  for (int attempt = 0; attempt < 4 && retry; ++attempt) {
+    FitArgs a = fit_args(m, q, nc, ip, m->rec.as<double>(), form);
+    DBuf& ws = m->ctx->qr_ws;
+    if ((rc = setup_lists(m, a, ws))) return rc;
+    if ((rc = enqueue_recover(m, a, form, ws.p, ws.bytes, s, true))) return rc;
+    EstArgs e = est_args(m, a.L, ip_order, nc, ip, target, ar, tn, alpha, beta, size, nullptr);
+    if ((rc = launch_estimate(e, s, [m](int i) { m->mark(i); }))) return rc;
+    Report r;
+    HIP_OK(hipMemcpyAsync(&r, m->scalars.as<double>() + 4, sizeof r, hipMemcpyDeviceToHost, s), "report");
+    HIP_OK(hipStreamSynchronize(s), "estimate sync");
+    collect_phases(m);
+    if ((rc = status_code(m, keep_status(m, a.npatch, r.counts), &retry))) return rc;
+    for (int i = 0; i < 3; ++i) sc[i] = r.sc[i];
+  }
+  if (retry) return sprg_fail(SPRG_ENOMEM, "SPR: expanded patch storage kept overflowing");
   auto t1 = std::chrono::steady_clock::now();
   if (diag) {
     if (!target) {
@@ -1396,11 +1436,10 @@ int record_batch(sprg_batch* b, int ip_order, int nc, const double* const* ip,
       rc = enqueue_recover(m, fa[i], form, ws.p, ws.bytes, s, false);
       if (!rc) {
         const bool tgt = target != nullptr;
-        EstArgs e = est_args(m, ip_order, nc, ip[i], tgt ? 1 : 0, ar, tgt ? (double)target[i] : 0,
-                             alpha, beta, size[i]);
+        EstArgs e = est_args(m, fa[i].L, ip_order, nc, ip[i], tgt ? 1 : 0, ar, tgt ? (double)target[i] : 0,
+                             alpha, beta, size[i], b->bstat.as<int32_t>() + i);
         rc = launch_estimate(e, s, [](int) {});
       }
-      if (!rc) rc = launch_copy_i32(b->bstat.as<int32_t>() + i, fa[i].L.status, 1, s);
     }
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(s, &g);
