@@ -402,18 +402,12 @@ __device__ __forceinline__ double readlane_d(double v, int lane)
   return __hiloint2double(hi, lo);
 }
 
-__device__ __forceinline__ void term_factors(int k, int* a, int* b)
-{
-  // 1, x, y, z, xy, yz, zx, xx, yy, zz
-  *a = k < 4 ? k : k < 7 ? k - 3 : k - 6;
-  *b = k < 4 ? 0 : k == 4 ? 2 : k == 5 ? 3 : k == 6 ? 1 : k - 6;
-}
-
 // Rank screen of a candidate set, one wave: the FP64 Gram matrix of the
 // monomials centred at the patch node and its Cholesky pivots.  The rows'
-// centred sample points go to LDS (sD, 3 doubles per row); lane l < NT(NT+1)/2
-// owns Gram entry l of the packed lower triangle, sums it over the rows and
-// keeps it through a right-looking factorisation whose columns travel by
+// monomials go to LDS (sF, 64 rows at a time, a lane per row); lane
+// l < NT(NT+1)/2 owns Gram entry l of the packed lower triangle, sums it over
+// the rows -- two reads and a fused multiply-add a row -- and keeps it
+// through a right-looking factorisation whose columns travel by
 // lane shuffles (the fused multiply-adds of each entry run in the same order
 // as a left-looking Cholesky's).  Centring is a unit-triangular change of the
 // graded monomial basis, so in exact arithmetic pivot k equals the
@@ -425,55 +419,56 @@ __device__ __forceinline__ void term_factors(int k, int* a, int* b)
 // pivot came out at +-5e-11 of its diagonal, so a bound near 1e-11 does not
 // separate rank-deficient sets from full ones.)  A false return decides
 // nothing: the exact test runs.
+// FP64 issue bounds it.  With the sample points staged and every lane forming
+// its own two monomials (eleven FP64 operations a row and lane) k_expand<10,
+// false> took 3.29 ms on an undistorted box of 384,000 tets; formed once, by
+// the row's own lane, and read back, one is left of them: 2.64 ms.
 // Every lane of the block (one wave) must call it.
+constexpr int CERT_ROWS = 64;  // rows whose monomials are in LDS at a time
+constexpr int cert_stride(int nt) { return nt + 1; }  // odd: a column's entries in different banks
+
 template <int NT>
 __device__ bool certify_full_rank(const MeshView& m, int q, const int32_t* S, int nrows,
-                                  int64_t p, int lane, double* sD)
+                                  int64_t p, int lane, double* sF)
 {
-  constexpr int NG = NT * (NT + 1) / 2;
+  constexpr int NG = NT * (NT + 1) / 2, FS = cert_stride(NT);
   const double xn[3] = {m.xyz[3 * p], m.xyz[3 * p + 1], m.xyz[3 * p + 2]};
-  for (int i = lane; i < nrows; i += 64) {
-    double x[3];
-    sample_point<NT == 4 ? 1 : 2>(m, S[i / q], i % q, x);
-    for (int j = 0; j < 3; ++j) sD[3 * i + j] = x[j] - xn[j];
-  }
-  __syncthreads();
   const bool own = lane < NG;
   int r = 0;
   while (own && (r + 1) * (r + 2) / 2 <= lane) ++r;
   const int c = own ? lane - r * (r + 1) / 2 : 0;
-  int ra, rb, ca, cb;
-  term_factors(r, &ra, &rb);
-  term_factors(c, &ca, &cb);
-  // this lane's two monomials as v[a] * v[b] over v = (1, x, y, z) (the
-  // products poly_terms forms; a unit factor is exact), each factor a
-  // one-hot combination of v (the zero weights add +-0, so a factor is
-  // exactly its component), the rows four at a time
-  const double wa[4] = {ra == 0 ? 1.0 : 0.0, ra == 1 ? 1.0 : 0.0, ra == 2 ? 1.0 : 0.0, ra == 3 ? 1.0 : 0.0};
-  const double wb[4] = {rb == 0 ? 1.0 : 0.0, rb == 1 ? 1.0 : 0.0, rb == 2 ? 1.0 : 0.0, rb == 3 ? 1.0 : 0.0};
-  const double wc[4] = {ca == 0 ? 1.0 : 0.0, ca == 1 ? 1.0 : 0.0, ca == 2 ? 1.0 : 0.0, ca == 3 ? 1.0 : 0.0};
-  const double wd[4] = {cb == 0 ? 1.0 : 0.0, cb == 1 ? 1.0 : 0.0, cb == 2 ? 1.0 : 0.0, cb == 3 ? 1.0 : 0.0};
-  auto pick = [](const double* w, const double* d) { return fma(w[3], d[2], fma(w[2], d[1], fma(w[1], d[0], w[0]))); };
   double g = 0;
-  if (own) {
-    int i = 0;
-    for (; i + 4 <= nrows; i += 4) {
-      double ta[4], tb[4];
+  for (int c0 = 0; c0 < nrows; c0 += CERT_ROWS) {
+    const int n = nrows - c0 < CERT_ROWS ? nrows - c0 : CERT_ROWS;
+    if (c0 > 0) __syncthreads();
+    if (lane < n) {
+      const int i = c0 + lane;
+      double x[3], f[10];
+      sample_point<NT == 4 ? 1 : 2>(m, S[i / q], i % q, x);
+      for (int j = 0; j < 3; ++j) x[j] -= xn[j];
+      poly_terms(NT == 4 ? 1 : 2, x, f);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const double d[3] = {sD[3 * (i + u)], sD[3 * (i + u) + 1], sD[3 * (i + u) + 2]};
-        ta[u] = pick(wa, d) * pick(wb, d);
-        tb[u] = pick(wc, d) * pick(wd, d);
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) g = fma(ta[u], tb[u], g);
+      for (int k = 0; k < NT; ++k) sF[lane * FS + k] = f[k];
     }
-    for (; i < nrows; ++i) {
-      const double d[3] = {sD[3 * i], sD[3 * i + 1], sD[3 * i + 2]};
-      g = fma(pick(wa, d) * pick(wb, d), pick(wc, d) * pick(wd, d), g);
+    __syncthreads();
+    if (own) {
+      const double* fr = sF + r;
+      const double* fc = sF + c;
+      int i = 0;
+      for (; i + 8 <= n; i += 8) {
+        double a[8], b[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          a[u] = fr[(i + u) * FS];
+          b[u] = fc[(i + u) * FS];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) g = fma(a[u], b[u], g);
+      }
+      for (; i < n; ++i) g = fma(fr[i * FS], fc[i * FS], g);
     }
   }
-  __syncthreads();  // sD is free again
+  __syncthreads();  // sF is free again
   const double diag_own = g;
   bool rank_ok = true;
   for (int k = 0; k < NT; ++k) {
@@ -506,11 +501,11 @@ __global__ __launch_bounds__(64) void k_expand(FitArgs a)
   __shared__ double sV[EXACT ? NT * XMAXR : 1];
   __shared__ double sDot[NT];
   __shared__ double sNorm[3];
-  // the candidate hash during enumeration, the screen's sample points after
-  // it (barriers separate the two uses)
-  __shared__ double sD[3 * XMAXR];
-  static_assert(HSIZE * sizeof(int32_t) <= sizeof(double) * 3 * XMAXR, "hash must fit the sample buffer");
-  int32_t* const sHash = reinterpret_cast<int32_t*>(sD);
+  // the candidate hash during enumeration, the screen's monomials after it
+  // (barriers separate the two uses)
+  constexpr int NF = CERT_ROWS * cert_stride(NT) > HSIZE / 2 ? CERT_ROWS * cert_stride(NT) : HSIZE / 2;
+  __shared__ double sF[NF];
+  int32_t* const sHash = reinterpret_cast<int32_t*>(sF);
   __shared__ int32_t sCur[256];
   __shared__ int32_t sOld[XSET];
   __shared__ int32_t sTmp[XSET];
@@ -662,7 +657,7 @@ __global__ __launch_bounds__(64) void k_expand(FitArgs a)
         bool ok = false;
         if (mrows >= NT && mrows <= XMAXR) {
           // a certified full rank needs no exact test; anything else does
-          ok = certify_full_rank<NT>(m, q, sCur, mrows, p, lane, sD);
+          ok = certify_full_rank<NT>(m, q, sCur, mrows, p, lane, sF);
           if (!ok && !EXACT) {
             if (lane == 0) {
               a.L.xq_exact[atomicAdd(nexact, 1)] = it;
