@@ -848,7 +848,8 @@ inline unsigned grid_for(int64_t n, int per) { return (unsigned)((n + per - 1) /
 template <int NT, int MODE>
 __global__ __launch_bounds__(64, 1) void k_exact_fit(FitArgs a)
 {
-  __shared__ double sm[exact_lds(NT, 192)];
+  constexpr int SM = exact_lds(NT, 192);
+  __shared__ double sm[SM];
   static_assert(NSMALL == 3 && NBUCKET == 7, "the buckets below");
   exact_fit<NT, 64, 64, MODE>(a, 3, sm);
   exact_fit<NT, 96, 64, MODE>(a, 4, sm);

@@ -193,6 +193,7 @@ __device__ __forceinline__ bool small_r(double (&r)[MMAX], double* sV, double* s
     double v[MMAX];
 #pragma unroll
     for (int i = k; i < MMAX; ++i) v[i] = sV[k * KS + i];
+    if (!KEEP) __syncthreads();  // read by every lane before the next takes its place
     double dot = 0;
 #pragma unroll
     for (int i = k; i < MMAX; ++i) dot += r[i] * v[i];
@@ -386,7 +387,8 @@ __device__ __forceinline__ void small_fit(const FitArgs& a, int bucket, double* 
 template <int NT, int MMAX, int MODE>
 __global__ __launch_bounds__(64, small_waves(NT, MMAX)) void k_qr_small(FitArgs a, int bucket)
 {
-  __shared__ double sm[small_lds(NT, MMAX)];
+  constexpr int SM = small_lds(NT, MMAX);
+  __shared__ double sm[SM];
   small_fit<NT, MMAX, MODE>(a, bucket, sm);
 }
 
@@ -396,7 +398,8 @@ __global__ __launch_bounds__(64, small_waves(NT, MMAX)) void k_qr_small(FitArgs 
 template <int NT, int MODE>
 __global__ __launch_bounds__(64, 2) void k_qr_small_lists(FitArgs a)
 {
-  __shared__ double sm[small_lds(NT, 32)];
+  constexpr int SM = small_lds(NT, 32);
+  __shared__ double sm[SM];
   small_fit<NT, 16, MODE>(a, 0, sm);
   small_fit<NT, 24, MODE>(a, 1, sm);
   small_fit<NT, 32, MODE>(a, 2, sm);
