@@ -156,6 +156,30 @@ __device__ __forceinline__ int64_t xcd_block(int64_t b, int64_t nblocks, int K)
   return (i / K) * span + x * K + (i % K);
 }
 
+// Stores of a result that is not read again by this kernel, one and two
+// doubles (p on 8 bytes): streamed past the caches' working set, where a
+// plain store of a large result evicts the inputs other blocks still share.
+__device__ __forceinline__ void store_stream(double* p, double a)
+{
+#if __has_builtin(__builtin_nontemporal_store)
+  __builtin_nontemporal_store(a, p);
+#else
+  *p = a;  // a host build of the kernels
+#endif
+}
+
+__device__ __forceinline__ void store_stream2(double* p, double a, double b)
+{
+#if __has_builtin(__builtin_nontemporal_store)
+  typedef double pair __attribute__((ext_vector_type(2), aligned(8)));
+  const pair v = {a, b};
+  __builtin_nontemporal_store(v, reinterpret_cast<pair*>(p));
+#else
+  p[0] = a;
+  p[1] = b;
+#endif
+}
+
 // Appends v to list[*counter] with one atomic per wave and target list.
 // Every lane of the wave calls it (convergent), so the ballot sees the whole
 // wave.
