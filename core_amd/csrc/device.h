@@ -25,6 +25,10 @@ struct MeshView {
   const int32_t* e2t;      // [6nt]
 };
 
+// Bits a mesh build sets: an index out of range, tet->edge and tet->vertex
+// that disagree, an edge node off its edge's midpoint.
+enum { MESH_RANGE = 1, MESH_DISAGREE = 2, MESH_CURVED = 4 };
+
 // Patch work lists.  Bucket b holds patches whose row count m = q*|set|
 // fits rows_of_bucket(b); larger sets, up to BIG_MMAX rows, go to the big
 // list.
@@ -118,6 +122,10 @@ struct TileView {
   const int32_t* leftover = nullptr;  // patches outside every tile
   int64_t nleftover = 0;
 };
+// log2 of the lanes that fit a patch of ns tets in the tiled pass: about six
+// tets per lane, at most eight lanes, and never more lanes than tets
+// (k_tile's weighted sum gives every lane of a solved set a first tet)
+__host__ __device__ inline int group_log2(int ns) { return ns <= 6 ? 0 : ns <= 12 ? 1 : ns <= 24 ? 2 : 3; }
 constexpr int TILE_DESC = 6;         // ints describing a tile to its build
 constexpr int TILE_SORT_CAP = 2048;  // candidate tets a tile build sorts
 constexpr int TILE_B = 64;           // lanes per tile: one wave, so a tile's
@@ -200,8 +208,10 @@ __device__ __forceinline__ void wave_append(int target, int my_target, int32_t* 
 }
 
 // Launchers (return 0 or an SPRG_E* code).
-int launch_csr(const MeshView& m, int dim, int32_t* off, int32_t* idx,
-               int32_t* tmp, hipStream_t s);
+int launch_csr(const MeshView& m, int dim, int32_t* off, int32_t* idx, int32_t* work, int32_t* status,
+               hipStream_t s);
+// status |= MESH_CURVED unless every edge node is its edge's midpoint.
+int launch_straight(const MeshView& m, int32_t* status, hipStream_t s);
 int launch_scan_i32(int32_t* a, int64_t n, int32_t* work, hipStream_t s);
 int launch_copy_i32(int32_t* dst, const int32_t* src, int64_t n, hipStream_t s);
 int launch_classify(const FitArgs& a, int nterms, hipStream_t s);
@@ -230,13 +240,12 @@ int launch_tile_fit(const FitArgs& a, int nterms, int form, hipStream_t s);
 // Tile construction: desc [TILE_DESC ntile] (each tile's candidate vertex
 // rows [cv0, cv1), the vertices whose patches it fits [pv0, pv1) and the
 // owned edges it fits own_e[pe0, pe1)), own_e (the edges grouped by their
-// owning vertex, in vertex order; null for an order-1 mesh); fills tet_off
-// (device, [ntile+1]), tets and the loc arrays.  pass 0 writes each tile's
-// union size to tet_off[tile + 1], pass 1 (after the scan) the unions and
-// the positions of the tile's patches' tets.
-int launch_tile_build(const MeshView& m, int64_t ntile, const int32_t* desc, const int32_t* own_e, int pass,
-                      int32_t* tet_off, int32_t* tets, uint16_t* v2t_loc, uint16_t* e2t_loc, int32_t* status,
-                      hipStream_t s);
+// owning vertex, in vertex order; null for an order-1 mesh), tet_off and
+// slot_off (the scans of the tiles' union sizes and lanes); fills tets, slot
+// and the loc arrays.
+int launch_tile_build(const MeshView& m, int64_t ntile, const int32_t* desc, const int32_t* own_e,
+                      const int32_t* tet_off, const int32_t* slot_off, int32_t* tets, int4* slot,
+                      uint16_t* v2t_loc, uint16_t* e2t_loc, int32_t* status, hipStream_t s);
 int launch_grad(const MeshView& m, int field_order, int nc_in,
                 const double* nodal, int ip_order, double* ip, hipStream_t s);
 

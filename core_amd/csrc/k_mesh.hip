@@ -6,6 +6,7 @@
 // (spr/sprRecoverField.cc:110, handles of mds/apfMDS.cc:98-107), so the CSR
 // is deterministic and bit-comparable with the reference adjacency.
 #include "device.h"
+#include "spr_math.h"
 
 namespace sprg {
 namespace {
@@ -21,7 +22,7 @@ __global__ void k_count(const int32_t* __restrict__ conn, int64_t n, int32_t* cn
   if (i >= n) return;
   int32_t r = conn[i];
   if (r < 0 || r >= nrows) {
-    atomicOr(status, 1);
+    atomicOr(status, MESH_RANGE);
     return;
   }
   atomicAdd(cnt + r + 1, 1);
@@ -112,6 +113,30 @@ __global__ void k_sort_rows(const int32_t* __restrict__ off, int64_t nrows, int3
   }
 }
 
+// Straight-sided test: every edge node is the midpoint (0 + a 0.5) + b 0.5;
+// else status MESH_CURVED.  A thread per tet (an edge is tested by each of
+// its tets).  8 us for 83k tets behind the uploads, where the host's walk
+// took 0.49 ms.
+__global__ __launch_bounds__(256) void k_straight(MeshView m, int32_t* status)
+{
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  bool curved = false;
+  if (t < m.nt)
+    for (int k = 0; k < 6; ++k) {
+      const double* a = m.xyz + 3 * (int64_t)m.tv[4 * t + tet_edge_vert(k, 0)];
+      const double* b = m.xyz + 3 * (int64_t)m.tv[4 * t + tet_edge_vert(k, 1)];
+      const double* c = m.xyz + 3 * (m.nv + (int64_t)m.te[6 * t + k]);
+      for (int j = 0; j < 3; ++j) {
+        double mid = 0;
+        mid += a[j] * 0.5;
+        mid += b[j] * 0.5;
+        if (mid != c[j]) curved = true;
+      }
+    }
+  const uint64_t any = __ballot(curved);
+  if (any && (int)(threadIdx.x % 64) == __ffsll((unsigned long long)any) - 1) atomicOr(status, MESH_CURVED);
+}
+
 inline unsigned grid(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
 __global__ void k_copy_i32(int32_t* __restrict__ dst, const int32_t* __restrict__ src, int64_t n)
@@ -142,18 +167,15 @@ int launch_scan_i32(int32_t* a, int64_t n, int32_t* work, hipStream_t s)
   return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "scan launch failed");
 }
 
-// tmp must hold max(nrows, ceil(nrows/SCAN_B)) + 2 int32.
-int launch_csr(const MeshView& m, int dim, int32_t* off, int32_t* idx,
-               int32_t* tmp, hipStream_t s)
+// work must hold max(nrows, ceil(nrows/SCAN_B)) int32.
+int launch_csr(const MeshView& m, int dim, int32_t* off, int32_t* idx, int32_t* work, int32_t* status,
+               hipStream_t s)
 {
   const int32_t* conn = dim == 0 ? m.tv : m.te;
   int per = dim == 0 ? 4 : 6;
   int64_t nrows = dim == 0 ? m.nv : m.ne;
   int64_t n = per * m.nt;
-  int32_t* status = tmp;       // 1 int
-  int32_t* work = tmp + 2;     // cursor / block sums
-  if (hipMemsetAsync(off, 0, sizeof(int32_t) * (nrows + 1), s) != hipSuccess ||
-      hipMemsetAsync(status, 0, sizeof(int32_t), s) != hipSuccess)
+  if (hipMemsetAsync(off, 0, sizeof(int32_t) * (nrows + 1), s) != hipSuccess)
     return sprg_fail(SPRG_EHIP, "csr: memset failed");
   if (n > 0) k_count<<<grid(n, 256), 256, 0, s>>>(conn, n, off, nrows, status);
   // inclusive scan of off[1..nrows] gives the exclusive offsets
@@ -167,12 +189,13 @@ int launch_csr(const MeshView& m, int dim, int32_t* off, int32_t* idx,
     return sprg_fail(SPRG_EHIP, "csr: copy failed");
   if (n > 0) k_fill<<<grid(n, 256), 256, 0, s>>>(conn, n, per, nrows, work, idx);
   if (nrows > 0) k_sort_rows<<<grid(nrows, 256), 256, 0, s>>>(off, nrows, idx);
-  int32_t st = 0;
-  if (hipMemcpyAsync(&st, status, sizeof st, hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipStreamSynchronize(s) != hipSuccess)
-    return sprg_fail(SPRG_EHIP, "csr: %s", hipGetErrorString(hipGetLastError()));
-  if (st) return sprg_fail(SPRG_EINVAL, "mesh: connectivity index out of range");
-  return 0;
+  return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "csr launch failed");
+}
+
+int launch_straight(const MeshView& m, int32_t* status, hipStream_t s)
+{
+  if (m.nt > 0) k_straight<<<grid(m.nt, 256), 256, 0, s>>>(m, status);
+  return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "straight test launch failed");
 }
 
 }  // namespace sprg

@@ -247,10 +247,12 @@ extern "C" int sprg_download(sprg_ctx* ctx, void* dst, const void* src, size_t b
 
 namespace {
 
-// log2 of the lanes that fit a patch of ns tets in the tiled pass: about
-// six tets per lane, at most eight lanes, and never more lanes than tets
-// (k_tile's weighted sum gives every lane of a solved set a first tet)
-int group_log2(int64_t ns) { return ns <= 6 ? 0 : ns <= 12 ? 1 : ns <= 24 ? 2 : 3; }
+// The host side of a tile build: what the tiles hold.  Kept until the uploads
+// that read it are done.
+struct TilePlan {
+  std::vector<int32_t> desc, tet_off, slot_off, own_e, leftover;
+  DBuf d_desc, d_own_e;
+};
 
 // Builds the tiles of the regular fast pass (k_tile.hip) from the host
 // connectivity and the device CSR: the host takes the patches in vertex
@@ -258,11 +260,12 @@ int group_log2(int64_t ns) { return ns <= 6 ? 0 : ns <= 12 ? 1 : ns <= 24 ? 2 : 
 // owning an edge) into tiles of at most TILE_B lanes whose tet unions (of
 // the v2t rows of the vertices whose patches or edges they take) hold at
 // most TILE_MAX_UNION tets -- a tile may end inside a vertex's edges, so
-// tiles fill their lanes -- and the device sorts each tile's union and
-// records every patch's positions in it.  A vertex with more than
-// TILE_MAX_UNION tets stays outside, with its owned edges: the
-// thread-per-patch pass fits those.
-int build_tiles(sprg_mesh* m, const int32_t* tet_verts, const int32_t* tet_edges)
+// tiles fill their lanes -- and the device sorts each tile's union, lays out
+// its slots and records every patch's positions in the union.  A vertex with
+// more than TILE_MAX_UNION tets stays outside, with its owned edges: the
+// thread-per-patch pass fits those.  The host's part runs while the device
+// uploads and sorts the adjacency; nothing here waits.
+int build_tiles(sprg_mesh* m, const int32_t* tet_verts, const int32_t* tet_edges, TilePlan& plan, int32_t* d_status)
 {
   const int64_t nv = m->nv, nt = m->nt;
   const bool edges = m->order == 2;
@@ -273,8 +276,7 @@ int build_tiles(sprg_mesh* m, const int32_t* tet_verts, const int32_t* tet_edges
     for (int64_t t = 0; t < nt; ++t)
       for (int k = 0; k < 6; ++k) {
         const int32_t e = tet_edges[6 * t + k];
-        ++ecount[e];
-        if (owner[e] < 0) {
+        if (ecount[e]++ == 0) {
           const int32_t a = tet_verts[4 * t + tet_edge_vert(k, 0)], b = tet_verts[4 * t + tet_edge_vert(k, 1)];
           owner[e] = a < b ? a : b;
         }
@@ -292,69 +294,87 @@ int build_tiles(sprg_mesh* m, const int32_t* tet_verts, const int32_t* tet_edges
     m->set_count.resize(ns);
     for (size_t k = 0; k < ns; ++k) m->set_count[k] = n[k] + n[ns + k] + n[2 * ns + k] + n[3 * ns + k];
   }
+  m->ntile = 0;
+  m->nleftover = 0;
+  m->max_union = 0;
   if (nv + ne >= (1 << 27)) return 0;  // the slot encoding holds 27-bit patch ids
   if (10 * nt >= INT32_MAX) return 0;  // loc offsets are int32
-  std::vector<int32_t> own_off(nv + 1, 0), own_e(ne);
-  for (int64_t e = 0; e < ne; ++e) ++own_off[owner[e] + 1];
+  std::vector<int32_t> own_off(nv + 1, 0);
+  std::vector<int32_t>& own_e = plan.own_e;
+  own_e.resize(ne);
+  for (int64_t e = 0; e < ne; ++e) {
+    if (owner[e] < 0) owner[e] = 0;  // an edge without tets
+    ++own_off[owner[e] + 1];
+  }
   for (int64_t v = 0; v < nv; ++v) own_off[v + 1] += own_off[v];
   {
     std::vector<int32_t> cur(own_off.begin(), own_off.end() - 1);
     for (int64_t e = 0; e < ne; ++e) own_e[cur[owner[e]]++] = (int32_t)e;
   }
-  hipStream_t s = m->ctx->stream;
-  DBuf d_desc, d_own_e, d_status;
-  int rc = 0;
-  if ((rc = d_own_e.ensure(sizeof(int32_t) * (ne + 1))) || (rc = d_status.ensure(sizeof(int32_t)))) return rc;
-  if (ne) HIP_OK(hipMemcpyAsync(d_own_e.p, own_e.data(), sizeof(int32_t) * ne, hipMemcpyHostToDevice, s), "tiles");
-  HIP_OK(hipMemsetAsync(d_status.p, 0, sizeof(int32_t), s), "tiles");
   // A tile takes patches in vertex order (a vertex's patch, then the edges
   // it owns) while they fit TILE_B lanes, the union of the v2t rows of the
   // vertices they need holds at most TILE_MAX_UNION tets and those rows at
   // most TILE_SORT_CAP entries; it may end inside a vertex's edges, the next
-  // tile taking the rest.  The unions are followed on the host (the rows
-  // are ascending tet ids, as the device CSR's).  Per tile (TILE_DESC
-  // ints): candidate rows [cv0, cv1), vertex patches [pv0, pv1), owned
-  // edges own_e[pe0, pe1).
-  std::vector<int32_t> hoff(nv + 1, 0), hrow((size_t)4 * nt);
+  // tile taking the rest.  The host follows the unions' sizes with a mark per
+  // tet, the last tile that holds it (merging the sorted unions took 1.2 ms
+  // for 83k tets).  Per tile (TILE_DESC ints): candidate rows [cv0, cv1), vertex
+  // patches [pv0, pv1), owned edges own_e[pe0, pe1).
+  std::vector<int32_t> hoff(nv + 1, 0), hrow((size_t)4 * nt), mark(nt, -1);
   for (int64_t v = 0; v < nv; ++v) hoff[v + 1] = hoff[v] + vcount[v];
   {
     std::vector<int32_t> cur(hoff.begin(), hoff.end() - 1);
     for (int64_t t = 0; t < nt; ++t)
       for (int k = 0; k < 4; ++k) hrow[cur[tet_verts[4 * t + k]]++] = (int32_t)t;
   }
-  std::vector<int32_t> desc, counts, leftover, uni, merged;
+  std::vector<int32_t>&desc = plan.desc, &tet_off = plan.tet_off, &slot_off = plan.slot_off, &leftover = plan.leftover;
+  tet_off.assign(1, 0);
+  slot_off.assign(1, 0);
   int32_t d[TILE_DESC] = {0, 0, 0, 0, 0, 0};
   bool open = false;
-  int sl = 0, cand = 0;
+  int sl = 0, cand = 0, uni = 0;  // the open tile's lanes, candidates and union size
+  int32_t tile = 0;               // marks are never reused
   auto close = [&]() {
-    if (open) desc.insert(desc.end(), d, d + TILE_DESC);
+    if (!open) return;
+    desc.insert(desc.end(), d, d + TILE_DESC);
+    tet_off.push_back(tet_off.back() + uni);
+    slot_off.push_back(slot_off.back() + sl);
+    m->max_union = std::max(m->max_union, uni);
     open = false;
   };
   auto start = [&](int32_t v) {
     d[0] = d[1] = d[2] = d[3] = v;
     d[4] = d[5] = own_off[v];
-    sl = cand = 0;
-    uni.clear();
+    sl = cand = uni = 0;
+    ++tile;
     open = true;
   };
-  auto row = [&](int32_t v) { return hrow.begin() + hoff[v]; };
+  // the tets of v's row that the open tile does not hold yet
+  auto mark_row = [&](int32_t v) {
+    int n = 0;
+    for (int32_t k = hoff[v]; k < hoff[v + 1]; ++k) {
+      int32_t& mk = mark[hrow[k]];
+      n += mk != tile;
+      mk = tile;
+    }
+    return n;
+  };
   // an item of vertex v taking `lanes` lanes: the tile in progress takes it
   // if it fits, else a new tile starts with it
   auto take = [&](int32_t v, int lanes) {
     if (!open) start(v);
     bool fits = sl + lanes <= TILE_B;
+    int add = 0;
     if (fits && d[1] <= v) {  // v's row would join the candidates
-      merged.clear();
-      std::set_union(uni.begin(), uni.end(), row(v), row(v + 1), std::back_inserter(merged));
-      fits = (int)merged.size() <= TILE_MAX_UNION && cand + vcount[v] <= TILE_SORT_CAP;
+      add = mark_row(v);
+      fits = uni + add <= TILE_MAX_UNION && cand + vcount[v] <= TILE_SORT_CAP;
     }
     if (!fits) {
       close();
       start(v);
-      merged.assign(row(v), row(v + 1));
+      add = mark_row(v);
     }
     if (d[1] <= v) {
-      uni.swap(merged);
+      uni += add;
       d[1] = v + 1;
       cand += vcount[v];
     }
@@ -377,93 +397,41 @@ int build_tiles(sprg_mesh* m, const int32_t* tet_verts, const int32_t* tet_edges
     }
   }
   close();
-  std::vector<int32_t>().swap(hrow);
-  const MeshView mv = m->view();
-  {
-    // the union sizes, from the device build (the same unions)
-    const int64_t ntile = (int64_t)desc.size() / TILE_DESC;
-    counts.assign(ntile + 1, 0);
-    if (ntile) {
-      if ((rc = d_desc.ensure(sizeof(int32_t) * TILE_DESC * ntile)) ||
-          (rc = m->t_tet_off.ensure(sizeof(int32_t) * (ntile + 1))))
-        return rc;
-      HIP_OK(hipMemcpyAsync(d_desc.p, desc.data(), sizeof(int32_t) * TILE_DESC * ntile, hipMemcpyHostToDevice, s),
-             "tiles");
-      if ((rc = launch_tile_build(mv, ntile, d_desc.as<int32_t>(), nullptr, 0, m->t_tet_off.as<int32_t>(), nullptr,
-                                  nullptr, nullptr, d_status.as<int32_t>(), s)))
-        return rc;
-      HIP_OK(hipMemcpyAsync(counts.data() + 1, m->t_tet_off.as<int32_t>() + 1, sizeof(int32_t) * ntile,
-                            hipMemcpyDeviceToHost, s), "tiles");
-      HIP_OK(hipStreamSynchronize(s), "tiles");
-    }
-    int mx = 0;
-    for (int64_t i = 1; i <= ntile; ++i) mx = std::max(mx, counts[i]);
-    if (mx > TILE_MAX_UNION) {  // not expected: every patch fits thread per patch
-      desc.clear();
-      counts.assign(1, 0);
-      leftover.clear();
-    }
-    m->max_union = mx <= TILE_MAX_UNION ? mx : 0;
-  }
   const int64_t ntile = (int64_t)desc.size() / TILE_DESC;
-  m->ntile = ntile;
-  m->nleftover = 0;
   if (!ntile) return 0;
-  for (int64_t i = 0; i < ntile; ++i) counts[i + 1] += counts[i];
-  // slots: every tile's patches in descending group size, groups aligned;
-  // each with the start and size of its set in the loc array (the CSR
-  // offsets are the prefix sums of the valences)
-  std::vector<int64_t> vfirst(nv + 1, 0), efirst(ne + 1, 0);
-  for (int64_t v = 0; v < nv; ++v) vfirst[v + 1] = vfirst[v] + vcount[v];
-  for (int64_t e = 0; e < ne; ++e) efirst[e + 1] = efirst[e] + ecount[e];
-  std::vector<int32_t> slot_off(ntile + 1, 0);
-  std::vector<int4> slot;
-  slot.reserve((size_t)(4 * nv + ne));
-  std::vector<std::pair<int, int32_t>> pat;
-  for (int64_t k = 0; k < ntile; ++k) {
-    pat.clear();
-    const int32_t* dk = desc.data() + TILE_DESC * k;
-    for (int32_t v = dk[2]; v < dk[3]; ++v) pat.push_back({group_log2(vcount[v]), v});
-    for (int32_t i = dk[4]; i < dk[5]; ++i) pat.push_back({group_log2(ecount[own_e[i]]), (int32_t)(nv + own_e[i])});
-    std::stable_sort(pat.begin(), pat.end(),
-                     [](const std::pair<int, int32_t>& x, const std::pair<int, int32_t>& y) { return x.first > y.first; });
-    for (const auto& pr : pat) {
-      const int32_t p = pr.second;
-      const int64_t first = p < nv ? vfirst[p] : 4 * nt + efirst[p - nv];
-      const int32_t ns = p < nv ? vcount[p] : ecount[p - nv];
-      for (int r = 0; r < (1 << pr.first); ++r) {
-        int4 sl;
-        sl.x = (int32_t)((uint32_t)p | ((uint32_t)pr.first << 27) | ((uint32_t)r << 29));
-        sl.y = (int32_t)first;
-        sl.z = ns;
-        sl.w = 0;
-        slot.push_back(sl);
-      }
-    }
-    slot_off[k + 1] = (int32_t)slot.size();
-  }
-  if ((rc = m->t_slot_off.ensure(sizeof(int32_t) * (ntile + 1))) || (rc = m->t_slot.ensure(sizeof(int4) * slot.size())) ||
-      (rc = m->t_tets.ensure(sizeof(int32_t) * ((size_t)counts[ntile] + 1))) ||
-      (rc = m->t_loc.ensure(sizeof(uint16_t) * (edges ? 10 * nt : 4 * nt))) ||
-      (rc = m->t_leftover.ensure(sizeof(int32_t) * (leftover.size() + 1))))
+  hipStream_t s = m->ctx->stream;
+  int rc = 0;
+  auto up = [&](DBuf& b, const std::vector<int32_t>& v) {
+    if (rc || v.empty()) return;
+    if ((rc = b.ensure(sizeof(int32_t) * v.size()))) return;
+    if (hipMemcpyAsync(b.p, v.data(), sizeof(int32_t) * v.size(), hipMemcpyHostToDevice, s) != hipSuccess)
+      rc = sprg_fail(SPRG_EHIP, "mesh_create: tile upload failed");
+  };
+  up(plan.d_desc, desc);
+  up(plan.d_own_e, own_e);
+  up(m->t_tet_off, tet_off);
+  up(m->t_slot_off, slot_off);
+  up(m->t_leftover, leftover);
+  if (rc || (rc = m->t_slot.ensure(sizeof(int4) * slot_off[ntile])) ||
+      (rc = m->t_tets.ensure(sizeof(int32_t) * ((size_t)tet_off[ntile] + 1))) ||
+      (rc = m->t_loc.ensure(sizeof(uint16_t) * (edges ? 10 * nt : 4 * nt))))
     return rc;
-  HIP_OK(hipMemcpyAsync(m->t_tet_off.p, counts.data(), sizeof(int32_t) * (ntile + 1), hipMemcpyHostToDevice, s), "tiles");
-  HIP_OK(hipMemcpyAsync(m->t_slot_off.p, slot_off.data(), sizeof(int32_t) * (ntile + 1), hipMemcpyHostToDevice, s), "tiles");
-  HIP_OK(hipMemcpyAsync(m->t_slot.p, slot.data(), sizeof(int4) * slot.size(), hipMemcpyHostToDevice, s), "tiles");
-  if (!leftover.empty())
-    HIP_OK(hipMemcpyAsync(m->t_leftover.p, leftover.data(), sizeof(int32_t) * leftover.size(), hipMemcpyHostToDevice, s),
-           "tiles");
-  if ((rc = launch_tile_build(mv, ntile, d_desc.as<int32_t>(), edges ? d_own_e.as<int32_t>() : nullptr, 1,
-                              m->t_tet_off.as<int32_t>(), m->t_tets.as<int32_t>(),
-                              m->t_loc.as<uint16_t>(), m->t_loc.as<uint16_t>() + 4 * nt, d_status.as<int32_t>(),
-                              s)))
+  if ((rc = launch_tile_build(m->view(), ntile, plan.d_desc.as<int32_t>(), edges ? plan.d_own_e.as<int32_t>() : nullptr,
+                              m->t_tet_off.as<int32_t>(), m->t_slot_off.as<int32_t>(), m->t_tets.as<int32_t>(),
+                              m->t_slot.as<int4>(), m->t_loc.as<uint16_t>(), m->t_loc.as<uint16_t>() + 4 * nt,
+                              d_status, s)))
     return rc;
-  int32_t st = 0;
-  HIP_OK(hipMemcpyAsync(&st, d_status.p, sizeof st, hipMemcpyDeviceToHost, s), "tiles");
-  HIP_OK(hipStreamSynchronize(s), "tiles");
-  if (st) return sprg_fail(SPRG_EINVAL, "mesh_create: tet->edge and tet->vertex connectivity disagree");
+  m->ntile = ntile;
   m->nleftover = (int64_t)leftover.size();
   return 0;
+}
+
+// Is every index in [0, n)?
+bool in_range(const int32_t* idx, int64_t count, int64_t n)
+{
+  uint32_t top = 0;  // a negative index is above every count
+  for (int64_t i = 0; i < count; ++i) top = std::max(top, (uint32_t)idx[i]);
+  return (int64_t)top < n;
 }
 
 }  // namespace
@@ -484,11 +452,12 @@ extern "C" int sprg_mesh_create(sprg_ctx* ctx, int64_t nv, int64_t nt, int64_t n
   if (4 * nt > INT32_MAX || 6 * nt > INT32_MAX || nv + ne > INT32_MAX)
     return sprg_fail(SPRG_EUNSUPPORTED, "mesh_create: part too large for int32 indices");
   // host-side validation: every index in range
-  for (int64_t i = 0; i < 4 * nt; ++i)
-    if (tet_verts[i] < 0 || tet_verts[i] >= nv)
-      return sprg_fail(SPRG_EINVAL, "mesh_create: tet %lld vertex index %d out of range",
-                       (long long)(i / 4), tet_verts[i]);
-  if (tet_edges)
+  if (!in_range(tet_verts, 4 * nt, nv))
+    for (int64_t i = 0; i < 4 * nt; ++i)
+      if (tet_verts[i] < 0 || tet_verts[i] >= nv)
+        return sprg_fail(SPRG_EINVAL, "mesh_create: tet %lld vertex index %d out of range",
+                         (long long)(i / 4), tet_verts[i]);
+  if (tet_edges && !in_range(tet_edges, 6 * nt, ne))
     for (int64_t i = 0; i < 6 * nt; ++i)
       if (tet_edges[i] < 0 || tet_edges[i] >= ne)
         return sprg_fail(SPRG_EINVAL, "mesh_create: tet %lld edge index %d out of range",
@@ -505,21 +474,6 @@ extern "C" int sprg_mesh_create(sprg_ctx* ctx, int64_t nv, int64_t nt, int64_t n
   m->ne = tet_edges ? ne : 0;
   m->order = order;
   m->nnodes = nv + (order == 2 ? ne : 0);
-  // straight-sided test: every edge node is the midpoint (0 + a*0.5) + b*0.5
-  if (order == 2) {
-    for (int64_t t = 0; t < nt && m->straight; ++t)
-      for (int k = 0; k < 6 && m->straight; ++k) {
-        const double* a = node_xyz + 3 * (int64_t)tet_verts[4 * t + tet_edge_vert(k, 0)];
-        const double* b = node_xyz + 3 * (int64_t)tet_verts[4 * t + tet_edge_vert(k, 1)];
-        const double* c = node_xyz + 3 * (nv + (int64_t)tet_edges[6 * t + k]);
-        for (int j = 0; j < 3; ++j) {
-          double mid = 0;
-          mid += a[j] * 0.5;
-          mid += b[j] * 0.5;
-          if (mid != c[j]) m->straight = 0;
-        }
-      }
-  }
   hipStream_t s = ctx->stream;
   int rc = 0;
   auto up = [&](DBuf& d, const void* src, size_t bytes) {
@@ -531,20 +485,33 @@ extern "C" int sprg_mesh_create(sprg_ctx* ctx, int64_t nv, int64_t nt, int64_t n
   up(m->tv, tet_verts, sizeof(int32_t) * 4 * nt);
   if (tet_edges) up(m->te, tet_edges, sizeof(int32_t) * 6 * nt);
   up(m->xyz, node_xyz, sizeof(double) * 3 * m->nnodes);
-  DBuf tmp;
-  int64_t tmpn = std::max(nv, m->ne) + 4;
-  if (!rc) rc = tmp.ensure(sizeof(int32_t) * tmpn);
+  TilePlan plan;
+  DBuf work, status;
+  if (!rc) rc = work.ensure(sizeof(int32_t) * (std::max(nv, m->ne) + 2));
+  if (!rc) rc = status.ensure(sizeof(int32_t));
+  if (!rc && hipMemsetAsync(status.p, 0, sizeof(int32_t), s) != hipSuccess)
+    rc = sprg_fail(SPRG_EHIP, "mesh_create: status");
   if (!rc) rc = m->v2t_off.ensure(sizeof(int32_t) * (nv + 1));
   if (!rc) rc = m->v2t.ensure(sizeof(int32_t) * 4 * nt);
-  if (!rc) rc = launch_csr(m->view(), 0, m->v2t_off.as<int32_t>(), m->v2t.as<int32_t>(), tmp.as<int32_t>(), s);
+  int32_t* const st = status.as<int32_t>();
+  if (!rc) rc = launch_csr(m->view(), 0, m->v2t_off.as<int32_t>(), m->v2t.as<int32_t>(), work.as<int32_t>(), st, s);
   if (!rc && m->ne) {
     rc = m->e2t_off.ensure(sizeof(int32_t) * (m->ne + 1));
     if (!rc) rc = m->e2t.ensure(sizeof(int32_t) * 6 * nt);
-    if (!rc) rc = launch_csr(m->view(), 1, m->e2t_off.as<int32_t>(), m->e2t.as<int32_t>(), tmp.as<int32_t>(), s);
+    if (!rc) rc = launch_csr(m->view(), 1, m->e2t_off.as<int32_t>(), m->e2t.as<int32_t>(), work.as<int32_t>(), st, s);
   }
-  if (!rc && hipStreamSynchronize(s) != hipSuccess) rc = sprg_fail(SPRG_EHIP, "mesh_create: sync failed");
-  tmp.release();
-  if (!rc) rc = build_tiles(m, tet_verts, tet_edges);
+  if (!rc && order == 2) rc = launch_straight(m->view(), st, s);
+  if (!rc) rc = build_tiles(m, tet_verts, tet_edges, plan, st);
+  int32_t bits = 0;
+  if (!rc && hipMemcpyAsync(&bits, status.p, sizeof bits, hipMemcpyDeviceToHost, s) != hipSuccess)
+    rc = sprg_fail(SPRG_EHIP, "mesh_create: status");
+  // the uploads read the caller's arrays and the plan
+  if (hipStreamSynchronize(s) != hipSuccess && !rc) rc = sprg_fail(SPRG_EHIP, "mesh_create: sync failed");
+  for (DBuf* b : {&work, &status, &plan.d_desc, &plan.d_own_e}) b->release();
+  if (!rc && (bits & MESH_RANGE)) rc = sprg_fail(SPRG_EINVAL, "mesh: connectivity index out of range");
+  if (!rc && (bits & MESH_DISAGREE))
+    rc = sprg_fail(SPRG_EINVAL, "mesh_create: tet->edge and tet->vertex connectivity disagree");
+  m->straight = bits & MESH_CURVED ? 0 : 1;
   if (rc) {
     sprg_mesh_destroy(m);
     return rc;
