@@ -262,8 +262,13 @@ __device__ __forceinline__ void next_verts(const MeshView& m, TileNext& n)
   if (l + TILE_B < n.U) n.vb = *reinterpret_cast<const int4*>(m.tv + 4 * (int64_t)n.tb);
 }
 
+// Doubles from one staged tet's sample points to the next's: odd, so that
+// the lanes' tets start in any bank (a stride of 12 doubles starts them in 8
+// of the 64 and cost the fits a quarter of their LDS cycles in conflicts).
+__host__ __device__ inline int x_stride(int q) { return (3 * q) | 1; }
+
 // Stages the tile's union into LDS: tet ids into sTet, the q sample points
-// of tet u into sX[(u q + l) 3 ..].  A lane per tet (at most 2 TILE_B tets
+// of tet u into sX[u x_stride(q) + 3 l ..].  A lane per tet (at most 2 TILE_B tets
 // per tile: the union cap is below that for TILE_B = 64 lanes is checked by
 // the builder).  Straight-sided meshes use the prefetched vertex ids; curved
 // Lagrange-2 meshes map through all ten nodes.
@@ -271,7 +276,7 @@ template <bool P2MAP>
 __device__ __forceinline__ void stage_tets(const MeshView& m, const TileNext& n, int q, int32_t* sTet,
                                            double* sX)
 {
-  const int l = threadIdx.x;
+  const int l = threadIdx.x, xs = x_stride(q);
   if constexpr (P2MAP) {
     for (int k = 0; k < 2; ++k) {
       const int u = l + k * TILE_B;
@@ -281,7 +286,7 @@ __device__ __forceinline__ void stage_tets(const MeshView& m, const TileNext& n,
       for (int r = 0; r < q; ++r) {
         double x[3];
         sample_x<true>(m, t, r, x);
-        for (int j = 0; j < 3; ++j) sX[3 * (u * q + r) + j] = x[j];
+        for (int j = 0; j < 3; ++j) sX[u * xs + 3 * r + j] = x[j];
       }
     }
   } else {
@@ -309,7 +314,7 @@ __device__ __forceinline__ void stage_tets(const MeshView& m, const TileNext& n,
         const double l0 = 1 - xi[0] - xi[1] - xi[2];
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-          sX[3 * (u * q + r) + j] =
+          sX[u * xs + 3 * r + j] =
               fma(xi[2], P[k][3][j], fma(xi[1], P[k][2][j], fma(xi[0], P[k][1][j], l0 * P[k][0][j])));
       }
     }
@@ -437,8 +442,9 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
   const MeshView& m = a.m;
   const TileView& tv = a.tiles;
   const int q = a.q;
-  double* const sX = smem;                                                         // [umax*q][3]
-  int32_t* const sTet = reinterpret_cast<int32_t*>(smem + 3 * tv.max_union * q);  // [umax]
+  const int xs = x_stride(q);
+  double* const sX = smem;                                                         // [umax][x_stride(q)]
+  int32_t* const sTet = reinterpret_cast<int32_t*>(smem + xs * tv.max_union);  // [umax]
   constexpr int NG = NT * (NT + 1) / 2;
   const TileWalk w = tile_walk(tv.ntile);
   TileNext nx;
@@ -479,7 +485,7 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
       for (int k = 0; k < NMOM; ++k) M[k] = 0;
       if (work)
         for_lane_tets(loc, rank, g, ns, [&](int u) {
-          const double* X = sX + 3 * q * u;
+          const double* X = sX + xs * u;
           for_points(q, [&](int l) {
             const double d[3] = {X[3 * l] - xn[0], X[3 * l + 1] - xn[1], X[3 * l + 2] - xn[2]};
             moments_row<T>(d, M);
@@ -494,7 +500,7 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
       for (int k = 0; k < NG; ++k) G[k] = 0;
       if (work)
         for_lane_tets(loc, rank, g, ns, [&](int u) {
-          const double* X = sX + 3 * q * u;
+          const double* X = sX + xs * u;
           for_points(q, [&](int l) {
             const double d[3] = {X[3 * l] - xn[0], X[3 * l + 1] - xn[1], X[3 * l + 2] - xn[2]};
             T f[NT];
@@ -571,7 +577,7 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
         for (int k = 0; k < NT; ++k) u[k] = 0;
         if (refine)
           for_lane_tets(loc, rank, g, ns, [&](int ut) {
-            const double* X = sX + 3 * q * ut;
+            const double* X = sX + xs * ut;
             for_points(q, [&](int l) {
               const double d[3] = {X[3 * l] - xn[0], X[3 * l + 1] - xn[1], X[3 * l + 2] - xn[2]};
               double f[NT];
@@ -619,12 +625,16 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
 #pragma unroll
     for (int c = 0; c < NC; ++c) v[c] = 0;
     auto accumulate = [&](const double* X, const double* b) {
-      const double d[3] = {X[0] - xn[0], X[1] - xn[1], X[2] - xn[2]};
-      double f[NT];
-      basis<double, NT>(d, f);
-      double w = 0;
-#pragma unroll
-      for (int k = 0; k < NT; ++k) w = fma(f[k], z[k], w);
+      // the weight phi . z, nested: 9 operations for 10 terms, not 16
+      const double x = X[0] - xn[0], y = X[1] - xn[1], t = X[2] - xn[2];
+      double w;
+      if constexpr (NT == 4) {
+        w = fma(t, z[3], fma(y, z[2], fma(x, z[1], z[0])));
+      } else {
+        const double cx = fma(z[6], t, fma(z[4], y, fma(z[7], x, z[1])));
+        const double cy = fma(z[5], t, fma(z[8], y, z[2]));
+        w = fma(t, fma(z[9], t, z[3]), fma(y, cy, fma(x, cx, z[0])));
+      }
 #pragma unroll
       for (int c = 0; c < NC; ++c) v[c] = fma(w, b[c] - b0[c], v[c]);
     };
@@ -652,11 +662,11 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
       for (int c = 0; c < NC; ++c) b0[c] = __shfl(b[c], src);
       if (solve) {
 #pragma unroll
-        for (int l = 0; l < 4; ++l) accumulate(sX + 12 * uf + 3 * l, b + l * NC);
+        for (int l = 0; l < 4; ++l) accumulate(sX + xs * uf + 3 * l, b + l * NC);
         for (int s = rank + g; s < ns; s += g) {
           const int u = un;
           un = loc[s + g < ns ? s + g : ns - 1];
-          const double* X = sX + 12 * u;
+          const double* X = sX + xs * u;
           const double* bt = a.ip + (int64_t)sTet[u] * 4 * NC;
 #pragma unroll
           for (int i = 0; i < 4 * NC; ++i) b[i] = bt[i];
@@ -669,7 +679,7 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
 #pragma unroll
       for (int c = 0; c < NC; ++c) b0[c] = bp[c];
       for_lane_tets(loc, rank, g, ns, [&](int u) {
-        const double* X = sX + 3 * q * u;
+        const double* X = sX + xs * u;
         const double* bt = a.ip + (int64_t)sTet[u] * q * NC;
         for (int l = 0; l < q; ++l) {
           double b[NC];
@@ -693,7 +703,7 @@ template <class T, int NT, int NREF, bool P2>
 int launch_tile_nc(const FitArgs& a, float tau_rank, float tau_acc, hipStream_t s)
 {
   const TileView& tv = a.tiles;
-  const size_t lds = sizeof(double) * 3 * (size_t)tv.max_union * a.q + sizeof(int32_t) * tv.max_union;
+  const size_t lds = sizeof(double) * (size_t)tv.max_union * x_stride(a.q) + sizeof(int32_t) * tv.max_union;
   // at least 8 blocks: tile_walk gives each XCD's range to its own blocks
   const unsigned blocks = (unsigned)std::max<int64_t>(8, std::min<int64_t>(a.shape.tile_blocks, tv.ntile));
   switch (a.nc) {
