@@ -53,6 +53,23 @@ __device__ __forceinline__ void term_pair(int k, int* a, int* b)
   *b = k < 4 ? 0 : k == 4 ? 2 : k == 5 ? 3 : k == 6 ? 1 : k - 6;
 }
 
+// The one point of an affine tet with vertices v (sample_tet's operations).
+__device__ __forceinline__ void sample_p1(const MeshView& m, const int4& v, double* X)
+{
+  const int32_t node[4] = {v.x, v.y, v.z, v.w};
+  double xi[3], N[10], x[3] = {0, 0, 0};
+  rule_point(1, 0, xi);
+  tet_values(1, xi, N);
+#pragma unroll
+  for (int n = 0; n < 4; ++n)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) x[j] += m.xyz[3 * (int64_t)node[n] + j] * N[n];
+  X[0] = 1;
+  X[1] = x[0];
+  X[2] = x[1];
+  X[3] = x[2];
+}
+
 // Samples of tet t (getSamplePoints, spr/sprRecoverField.cc:193-211): point
 // l < q of the MESH order's rule (the order-1 rule ignores l), mapped by the
 // coordinate field in the summation order of apf/apfElement.cc:106-114; each
@@ -215,9 +232,9 @@ __device__ __forceinline__ bool small_r(double (&r)[MMAX], double* sV, double* s
 // many rows as the registers take (each reflector entry read from LDS then
 // serves several rows, and the rows' independent sums hide each other's
 // latency).
-constexpr int small_rpl(int nt, int mmax)
+constexpr int small_rpl(int mmax)
 {
-  return nt == 4 ? (mmax == 16 ? 4 : mmax == 24 ? 3 : 2) : mmax == 24 ? 3 : 2;
+  return mmax == 24 ? 3 : 2;
 }
 constexpr int small_waves(int nt, int mmax) { return mmax == 16 ? 3 : 2; }
 
@@ -234,7 +251,7 @@ __device__ __forceinline__ void small_fit(const FitArgs& a, int bucket, double* 
 {
   constexpr int ORDER = NT == 4 ? 1 : 2;
   constexpr int G = NT, P = 64 / G;  // lanes per patch, patches per wave
-  constexpr int RPL = small_rpl(NT, MMAX);
+  constexpr int RPL = small_rpl(MMAX);
   constexpr int NPASS = (MMAX + G * RPL - 1) / (G * RPL);
   constexpr int VS = NT * MMAX, NRT = NT * (NT + 1) / 2;
   constexpr int S = small_stride(NT, MMAX);
@@ -261,12 +278,33 @@ __device__ __forceinline__ void small_fit(const FitArgs& a, int bucket, double* 
     const int32_t* set = nullptr;
     if (act) fit_item<MODE>(a, list[base + g], &p, &set, &ns);
     const int rows = ns * q;  // <= MMAX
-    if (on)
+    if (NT == 4 && q == 1) {
+      // up to MMAX / 4 tets a lane: every id, then every tet's vertices, then
+      // the coordinates, instead of three round trips for each (with the
+      // values below eight at a time, 275k sets of 24 rows and nine
+      // components take 255 us; a load after another took 412)
+      constexpr int K = (MMAX + G - 1) / G;
+      int32_t t[K];
+      int4 v[K];
+#pragma unroll
+      for (int k = 0; k < K; ++k) t[k] = ns > 0 ? set[gl + k * G < ns ? gl + k * G : 0] : 0;
+#pragma unroll
+      for (int k = 0; k < K; ++k) v[k] = *reinterpret_cast<const int4*>(m.tv + 4 * (int64_t)t[k]);
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const int s = gl + k * G;
+        if (on && s < ns) {
+          sS[s] = t[k];
+          sample_p1(m, v[k], sV + 4 * s);
+        }
+      }
+    } else if (on) {
       for (int s = gl; s < ns; s += G) {
         const int32_t t = set[s];
         sS[s] = t;
         sample_tet<ORDER>(m, t, q, sV + 4 * s * q);
       }
+    }
     __syncthreads();
     // R: this lane's column
     double r[MMAX];
@@ -372,6 +410,22 @@ __device__ __forceinline__ void small_fit(const FitArgs& a, int bucket, double* 
             for (int l = 0; l < 4; ++l) bn[l] = src[l * nc];
 #pragma unroll
             for (int l = 0; l < 4; ++l) add_row(4 * s + l, b[l]);
+          }
+        } else if (NT == 4 && q == 1) {
+          // eight tets' values in flight while eight are summed
+          double b[8], bn[8];
+          auto fetch = [&](int s0) {
+#pragma unroll
+            for (int l = 0; l < 8; ++l) bn[l] = a.ip[(int64_t)sS[s0 + l < ns ? s0 + l : 0] * nc + c];
+          };
+          fetch(0);
+          for (int s0 = 0; s0 < ns; s0 += 8) {
+#pragma unroll
+            for (int l = 0; l < 8; ++l) b[l] = bn[l];
+            if (s0 + 8 < ns) fetch(s0 + 8);
+#pragma unroll
+            for (int l = 0; l < 8; ++l)
+              if (s0 + l < ns) add_row(s0 + l, b[l]);
           }
         } else {
           for (int s = 0; s < ns; ++s)
