@@ -12,7 +12,7 @@ size factor, vertex average) with the IP field resident in HBM.
 Prints one JSON line.  value = recovered patches (V + E) per second of the
 whole size-field step in the chosen form (default fp64f: FP64 normal
 equations, the fastest form that meets 1e-6 relative on the size field);
-"forms" reports the other two forms on the same mesh (FP32 + FP64 refinement,
+"forms" reports the other two forms on the same mesh (with FP64 refinement,
 and the exact FP64 form that reproduces the reference bit for bit) with
 their accuracy against the exact form; roofline = the dominant kernel (the
 patch fit over every patch, one launch) with the recovery's algorithmic HBM
@@ -335,7 +335,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f32+f64" if args.form == "fp32r" else "f64",
+        "dtype": "f64",
         "data": "synthetic",
         "config": {"workload": "strain_120: getSPRSizeField(0.05) on n=120 P2 jittered cube, "
                                "10,368,000 tets, 9-comp strain IP field, IP order 2",

@@ -13,10 +13,8 @@
 // the reference's Householder R_kk on raw coordinates in exact arithmetic)
 // is unchanged.
 //
-//   T = float : G and its Cholesky factor in FP32; NREF (3) residual
-//               refinement steps r = e_0 - A^T (A z) in FP64;
-//   T = double: G and the factor in FP64 (NREF = 0), or the FP64 fallback
-//               for ill-conditioned patches (NREF = 2).
+// G and its Cholesky factor are FP64.  NREF = 2 (the refined form and the
+// fallback): residual refinement steps r = e_0 - A^T (A z).
 //
 // Rank: the reference rejects a patch when a Householder column norm falls
 // below 1e-10 (mth/mthQR.cc:31).  The Cholesky pivot L_kk is that norm; a
@@ -24,8 +22,8 @@
 // margin and was computed without heavy cancellation (pivot / diagonal >=
 // tau_rank).  Anything else goes to the exact FP64 path (k_expand tests the
 // initial set with the reference's arithmetic before growing it).  Certified
-// patches whose smallest pivot ratio is below tau_acc go to the FP64
-// fallback.  Three passes over the rows: Gram, refinement, weighted sum;
+// patches whose smallest pivot ratio is below tau_acc go to the exact kernel
+// (the fallback, above its rows).  Three passes over the rows: Gram, refinement, weighted sum;
 // sample positions are recomputed in each (affine in the four vertices for a
 // straight-sided mesh, the Lagrange-2 map otherwise).
 #include "device.h"
@@ -134,17 +132,14 @@ __device__ __forceinline__ void sample_d(const MeshView& m, const Geo<P2MAP>& g,
   d[2] = x[2] - xn[2];
 }
 
-// SRC_PRE_FALLBACK: the FP32 form's FP64 pass over its fallback queue before
-// the expansion (it may still send a set to the rank test); SRC_FALLBACK then
-// walks only the entries queued after it.
+// SRC_FALLBACK: poor sets of more rows than the exact kernels take.
 // SRC_LEFTOVER: the initial sets of the patches outside every tile of the
 // tiled pass (k_tile.hip), with the regular pass's decisions.
-enum { SRC_REGULAR = 0, SRC_EXPANDED = 1, SRC_FALLBACK = 2, SRC_PRE_FALLBACK = 3, SRC_LEFTOVER = 4 };
-
+enum { SRC_REGULAR = 0, SRC_EXPANDED = 1, SRC_FALLBACK = 2, SRC_LEFTOVER = 4 };
 
 // src SRC_REGULAR walks every patch id and SRC_EXPANDED every queued item; the
 // others walk a list.
-template <class T, int NT, int NC, int NREF, bool P2MAP>
+template <int NT, int NC, int NREF, bool P2MAP>
 __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank, float tau_acc)
 {
   const MeshView& m = a.m;
@@ -156,11 +151,10 @@ __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank
                         : src == SRC_LEFTOVER ? a.tiles.nleftover
                         : src == SRC_EXPANDED ? a.L.count[2 * NBUCKET]
                                               : a.L.count[2 * NBUCKET + 1];
-  const int64_t first = src == SRC_FALLBACK ? a.L.status[2] : 0;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   // The trip count is the same for every lane of a block, so the list
   // appends below run on whole waves; lanes past the end carry ACT_NONE.
-  for (int64_t base = first + xcd_block(blockIdx.x, gridDim.x, XCD_K_FIT) * blockDim.x; base < count;
+  for (int64_t base = xcd_block(blockIdx.x, gridDim.x, XCD_K_FIT) * blockDim.x; base < count;
        base += stride) {
     const int64_t it = base + threadIdx.x;
     // the expanded sets are the expansion queue's items that found one
@@ -170,8 +164,7 @@ __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank
       const uint64_t found = __ballot(valid);
       if ((threadIdx.x & 63) == 0 && found) atomicAdd(a.L.count + NBUCKET, __popcll(found));
     }
-    const bool expanded =
-        src == SRC_EXPANDED || ((src == SRC_FALLBACK || src == SRC_PRE_FALLBACK) && entry < 0);
+    const bool expanded = src == SRC_EXPANDED || (src == SRC_FALLBACK && entry < 0);
     const int32_t id = entry & 0x7fffffff;
     int64_t p = 0;
     const int32_t* set = nullptr;
@@ -196,7 +189,7 @@ __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank
     const bool short_set = valid && regular && ns * q < NT;
     const bool work = valid && !short_set;
     constexpr int NG = NT * (NT + 1) / 2;
-    T G[NG];
+    double G[NG];
 #pragma unroll
     for (int k = 0; k < NG; ++k) G[k] = 0;
     bool rank_ok = true;
@@ -211,8 +204,8 @@ __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank
         for (int l = 0; l < q; ++l) {
           double d[3];
           sample_d(m, g, p2map, l, xn, d);
-          T f[NT];
-          basis<T, NT>(d, f);
+          double f[NT];
+          basis<double, NT>(d, f);
 #pragma unroll
           for (int i = 0; i < NT; ++i)
 #pragma unroll
@@ -222,18 +215,18 @@ __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank
       // Cholesky in place, with the rank certificate and the conditioning
 #pragma unroll
       for (int k = 0; k < NT; ++k) {
-        const T diag = G[tri(k, k)];
-        T dk = diag;
+        const double diag = G[tri(k, k)];
+        double dk = diag;
 #pragma unroll
         for (int j = 0; j < k; ++j) dk = fma(-G[tri(k, j)], G[tri(k, j)], dk);
         const float ratio = (diag > 0 && dk > 0) ? (float)(dk / diag) : 0.0f;
         min_ratio = fminf(min_ratio, ratio);
-        const T lkk = dk > 0 ? sqrt(dk) : (T)0;
-        if (!(ratio >= tau_rank) || !((double)lkk >= 1.05e-10)) rank_ok = false;
-        G[tri(k, k)] = lkk > 0 ? lkk : (T)1;
+        const double lkk = dk > 0 ? sqrt(dk) : 0.0;
+        if (!(ratio >= tau_rank) || !(lkk >= 1.05e-10)) rank_ok = false;
+        G[tri(k, k)] = lkk > 0 ? lkk : 1.0;
 #pragma unroll
         for (int i = k + 1; i < NT; ++i) {
-          T s = G[tri(i, k)];
+          double s = G[tri(i, k)];
 #pragma unroll
           for (int j = 0; j < k; ++j) s = fma(-G[tri(i, j)], G[tri(k, j)], s);
           G[tri(i, k)] = s / G[tri(k, k)];
@@ -241,26 +234,22 @@ __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank
       }
     }
     // Short sets and uncertified ranks: the exact path decides (bit 31: test
-    // the initial set before growing it).  Below tau_acc the FP32 regular
-    // pass hands the patch to the FP64 fallback; an FP64 pass hands it to
-    // the exact kernel (normal equations square the condition number; the
+    // the initial set before growing it).  Below tau_acc the exact kernel
+    // refits the patch (normal equations square the condition number; the
     // reference's Householder arithmetic reproduces its own answer), when the
     // set fits the exact kernel's rows.
     const int bucket = bucket_of(ns * q);
-    const int poor = (regular && sizeof(T) == 4) ? ACT_FALLBACK
-                     : bucket < NBUCKET                     ? ACT_REFIT
-                     : ns * q <= BIG_MMAX                   ? ACT_BIG
-                     : src != SRC_FALLBACK && src != SRC_PRE_FALLBACK ? ACT_FALLBACK
+    const int poor = bucket < NBUCKET      ? ACT_REFIT
+                     : ns * q <= BIG_MMAX  ? ACT_BIG
+                     : src != SRC_FALLBACK ? ACT_FALLBACK
                      // more rows than the exact kernels take: the refined
                      // FP64 solve, unless hopeless
                      : min_ratio >= 1e-13f ? ACT_SOLVE : ACT_ILLCOND;
     int act = ACT_NONE;
     if (short_set)
       act = ACT_EXACT;
-    else if (work && (regular || src == SRC_PRE_FALLBACK) && !rank_ok)
-      // the FP32 pass leaves the rank to its FP64 pass, which certifies
-      // most sets the FP32 certificate could not
-      act = (regular && sizeof(T) == 4) ? ACT_FALLBACK : ACT_EXACT;
+    else if (work && regular && !rank_ok)
+      act = ACT_EXACT;
     else if (work && !(min_ratio >= tau_acc))
       act = poor;
     else if (work)
@@ -270,12 +259,10 @@ __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank
     // conditioned
     double z[NT];
     if (act == ACT_SOLVE) {
-      T e0[NT], zt[NT];
+      double e0[NT];
 #pragma unroll
       for (int k = 0; k < NT; ++k) e0[k] = k == 0 ? 1 : 0;
-      chol_solve<T, NT>(G, e0, zt);
-#pragma unroll
-      for (int k = 0; k < NT; ++k) z[k] = (double)zt[k];
+      chol_solve<double, NT>(G, e0, z);
       double last_dz = 0, zmax = 0;
       for (int r = 0; r < NREF; ++r) {
         double u[NT];
@@ -293,16 +280,16 @@ __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank
             for (int k = 0; k < NT; ++k) u[k] = fma(f[k], t, u[k]);
           }
         });
-        T res[NT], dz[NT];
+        double res[NT], dz[NT];
 #pragma unroll
-        for (int k = 0; k < NT; ++k) res[k] = (T)((k == 0 ? 1.0 : 0.0) - u[k]);
-        chol_solve<T, NT>(G, res, dz);
+        for (int k = 0; k < NT; ++k) res[k] = (k == 0 ? 1.0 : 0.0) - u[k];
+        chol_solve<double, NT>(G, res, dz);
         last_dz = 0;
         zmax = 0;
 #pragma unroll
         for (int k = 0; k < NT; ++k) {
-          z[k] += (double)dz[k];
-          last_dz = fmax(last_dz, fabs((double)dz[k]));
+          z[k] += dz[k];
+          last_dz = fmax(last_dz, fabs(dz[k]));
           zmax = fmax(zmax, fabs(z[k]));
         }
       }
@@ -347,7 +334,7 @@ __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank
   }
 }
 
-template <class T, int NT, int NREF, bool P2>
+template <int NT, int NREF, bool P2>
 int launch_nc2(const FitArgs& a, int src, float tau_rank, float tau_acc, hipStream_t s)
 {
   const unsigned threads = (unsigned)a.shape.fast_threads;
@@ -357,51 +344,48 @@ int launch_nc2(const FitArgs& a, int src, float tau_rank, float tau_acc, hipStre
   const unsigned blocks =
       (unsigned)std::max<int64_t>(1, std::min<int64_t>(a.shape.fast_blocks, (work + threads - 1) / threads));
   switch (a.nc) {
-    case 1: k_fast<T, NT, 1, NREF, P2><<<blocks, threads, 0, s>>>(a, src, tau_rank, tau_acc); break;
-    case 3: k_fast<T, NT, 3, NREF, P2><<<blocks, threads, 0, s>>>(a, src, tau_rank, tau_acc); break;
-    case 9: k_fast<T, NT, 9, NREF, P2><<<blocks, threads, 0, s>>>(a, src, tau_rank, tau_acc); break;
-    case 27: k_fast<T, NT, 27, NREF, P2><<<blocks, threads, 0, s>>>(a, src, tau_rank, tau_acc); break;
+    case 1: k_fast<NT, 1, NREF, P2><<<blocks, threads, 0, s>>>(a, src, tau_rank, tau_acc); break;
+    case 3: k_fast<NT, 3, NREF, P2><<<blocks, threads, 0, s>>>(a, src, tau_rank, tau_acc); break;
+    case 9: k_fast<NT, 9, NREF, P2><<<blocks, threads, 0, s>>>(a, src, tau_rank, tau_acc); break;
+    case 27: k_fast<NT, 27, NREF, P2><<<blocks, threads, 0, s>>>(a, src, tau_rank, tau_acc); break;
     default: return sprg_fail(SPRG_EUNSUPPORTED, "fast recovery: %d components", a.nc);
   }
   return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "fast fit launch failed");
 }
 
-template <class T, int NT, int NREF>
+template <int NT, int NREF>
 int launch_nc(const FitArgs& a, int src, float tau_rank, float tau_acc, hipStream_t s)
 {
   if (a.m.order == 2 && !a.m.straight)
-    return launch_nc2<T, NT, NREF, true>(a, src, tau_rank, tau_acc, s);
-  return launch_nc2<T, NT, NREF, false>(a, src, tau_rank, tau_acc, s);
+    return launch_nc2<NT, NREF, true>(a, src, tau_rank, tau_acc, s);
+  return launch_nc2<NT, NREF, false>(a, src, tau_rank, tau_acc, s);
 }
 
-template <class T, int NREF>
+template <int NREF>
 int launch_t(const FitArgs& a, int nterms, int src, float tau_rank, float tau_acc, hipStream_t s)
 {
-  return nterms == 4 ? launch_nc<T, 4, NREF>(a, src, tau_rank, tau_acc, s)
-                     : launch_nc<T, 10, NREF>(a, src, tau_rank, tau_acc, s);
+  return nterms == 4 ? launch_nc<4, NREF>(a, src, tau_rank, tau_acc, s)
+                     : launch_nc<10, NREF>(a, src, tau_rank, tau_acc, s);
 }
 
 }  // namespace
 
-// form SPRG_FP32R: FP32 Gram + 3 FP64 refinement steps; SPRG_FP64F: FP64
-// Gram, no refinement.  src: 0 regular, 1 expanded,
-// 2 the FP64 fallback queue (FP64 Gram + 2 refinement steps).
+// src: 0 regular, 1 expanded, 2 the fallback queue, 4 the patches outside the
+// tiles.  The refined form (SPRG_FP32R) and the fallback take two refinement
+// steps, the second of which only confirms the first on all but poor sets.
 int launch_fast_fit(const FitArgs& a, int nterms, int form, int src, hipStream_t s)
 {
   if (a.q > NQ_MAX) return sprg_fail(SPRG_EUNSUPPORTED, "fast recovery: %d points per element", a.q);
-  // FP64 passes refit sets whose smallest pivot ratio is below 1e-6 with the
-  // exact kernel.  Expanded sets (often barely full rank) always take the
-  // FP64 pass.
-  if (src == 2) return launch_t<double, 2>(a, nterms, src, 0.0f, 1e-6f, s);
-  if (src == 3) return launch_t<double, 2>(a, nterms, src, 1e-6f, 1e-6f, s);
-  if (src == 1) return launch_t<double, 0>(a, nterms, src, 0.0f, 1e-6f, s);
-  // FP32: three FP64 refinement steps; each contracts the error by about
-  // kappa(G) * 2^-24, and the size field needs the recovered field to ~1e-12
-  if (form == SPRG_FP32R) return launch_t<float, 3>(a, nterms, src, 1e-4f, 1e-3f, s);
+  // Sets whose smallest pivot ratio is below 1e-6 are refitted by the exact
+  // kernel.  Expanded sets (often barely full rank) are not refined: the
+  // exact kernel takes their poor ones.
+  if (src == SRC_FALLBACK) return launch_t<2>(a, nterms, src, 0.0f, 1e-6f, s);
+  if (src == SRC_EXPANDED) return launch_t<0>(a, nterms, src, 0.0f, 1e-6f, s);
   // a pivot that keeps less than 1e-6 of its diagonal is not a rank
   // certificate in FP64 (its rounding can exceed 1e-11 of the diagonal after
   // earlier cancellation): such sets take the reference's rank test
-  return launch_t<double, 0>(a, nterms, src, 1e-6f, 1e-6f, s);
+  return form == SPRG_FP32R ? launch_t<2>(a, nterms, src, 1e-6f, 1e-6f, s)
+                            : launch_t<0>(a, nterms, src, 1e-6f, 1e-6f, s);
 }
 
 }  // namespace sprg

@@ -340,12 +340,6 @@ __device__ __forceinline__ double xor_lane(double x)
   return __hiloint2double(hi, lo);
 }
 
-template <int ST>
-__device__ __forceinline__ float xor_lane(float x)
-{
-  return __int_as_float(xor_lane<ST>(__float_as_int(x)));
-}
-
 // One butterfly level: lanes of groups wider than ST add their partner's
 // value, the others add it times zero.  The partner of a lane outside such a
 // group belongs to another group or to no patch, whose sums are finite (or
@@ -371,9 +365,8 @@ __device__ __forceinline__ void group_sum(T* v, int g, int gmax)
   if (gmax > 4) group_step<4, T, N>(v, g);
 }
 
-// 1 / sqrt(d) for d > 0: the hardware estimate and Newton steps
-// r <- r + r (1/2 - (d/2) r^2), two in FP64 (each doubles the correct bits)
-// and one in FP32.
+// 1 / sqrt(d) for d > 0: the hardware estimate and two Newton steps
+// r <- r + r (1/2 - (d/2) r^2), each doubling the correct bits.
 __device__ __forceinline__ double rsqrt_nr(double d)
 {
   double r = __builtin_amdgcn_rsq(d);
@@ -381,12 +374,6 @@ __device__ __forceinline__ double rsqrt_nr(double d)
 #pragma unroll
   for (int i = 0; i < 2; ++i) r = fma(r, fma(-h, r * r, 0.5), r);
   return r;
-}
-
-__device__ __forceinline__ float rsqrt_nr(float d)
-{
-  const float r = __builtin_amdgcn_rsqf(d);
-  return fmaf(r, fmaf(-0.5f * d, r * r, 0.5f), r);
 }
 
 // body(u) for the lane's tets s = rank, rank + g, ... < ns of its patch set
@@ -435,7 +422,7 @@ __device__ __forceinline__ void chol_solve_rcp(const T* L, const T* rhs, T* z)
   }
 }
 
-template <class T, int NT, int NC, int NREF, bool P2MAP>
+template <int NT, int NC, int NREF, bool P2MAP>
 __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, float tau_acc)
 {
   extern __shared__ double smem[];
@@ -477,10 +464,10 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
     const uint64_t b2 = __ballot(g >= 2), b4 = __ballot(g >= 4), b8 = __ballot(g >= 8);
     const int gmax = b8 ? 8 : b4 ? 4 : b2 ? 2 : 1;
     // Gram matrix of the group's tets, packed lower triangle
-    T G[NG];
+    double G[NG];
     if constexpr (NT == 10) {
       // from the moments of the lane's rows, summed over the group
-      T M[NMOM];
+      double M[NMOM];
 #pragma unroll
       for (int k = 0; k < NMOM; ++k) M[k] = 0;
       if (work)
@@ -488,13 +475,13 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
           const double* X = sX + xs * u;
           for_points(q, [&](int l) {
             const double d[3] = {X[3 * l] - xn[0], X[3 * l + 1] - xn[1], X[3 * l + 2] - xn[2]};
-            moments_row<T>(d, M);
+            moments_row<double>(d, M);
           });
         });
       next_ids(tv, nx);  // arrives during the reduction and the factorisation
-      group_sum<T, NMOM>(M, g, gmax);
-      M[0] = (T)(ns * q);
-      gram_from_moments<T>(M, G);
+      group_sum<double, NMOM>(M, g, gmax);
+      M[0] = (double)(ns * q);
+      gram_from_moments<double>(M, G);
     } else {
 #pragma unroll
       for (int k = 0; k < NG; ++k) G[k] = 0;
@@ -503,8 +490,8 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
           const double* X = sX + xs * u;
           for_points(q, [&](int l) {
             const double d[3] = {X[3 * l] - xn[0], X[3 * l + 1] - xn[1], X[3 * l + 2] - xn[2]};
-            T f[NT];
-            basis<T, NT>(d, f);
+            double f[NT];
+            basis<double, NT>(d, f);
 #pragma unroll
             for (int i = 0; i < NT; ++i)
 #pragma unroll
@@ -512,7 +499,7 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
           });
         });
       next_ids(tv, nx);  // arrives during the reduction and the factorisation
-      group_sum<T, NG>(G, g, gmax);
+      group_sum<double, NG>(G, g, gmax);
     }
     // Cholesky in place, with the rank certificate and the conditioning
     bool rank_ok = true;
@@ -520,19 +507,19 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
     if (work) {
 #pragma unroll
       for (int k = 0; k < NT; ++k) {
-        const T diag = G[tri(k, k)];
-        T dk = diag;
+        const double diag = G[tri(k, k)];
+        double dk = diag;
 #pragma unroll
         for (int j = 0; j < k; ++j) dk = fma(-G[tri(k, j)], G[tri(k, j)], dk);
         const float ratio = (diag > 0 && dk > 0) ? (float)(dk / diag) : 0.0f;
         min_ratio = fminf(min_ratio, ratio);
         // L_kk = sqrt(dk) must clear 1.05e-10: dk >= 1.05e-10^2
-        if (!(ratio >= tau_rank) || !((double)dk >= 1.1025e-20)) rank_ok = false;
-        const T rk = dk > 0 ? rsqrt_nr(dk) : (T)1;  // the diagonal keeps 1 / L_kk
+        if (!(ratio >= tau_rank) || !(dk >= 1.1025e-20)) rank_ok = false;
+        const double rk = dk > 0 ? rsqrt_nr(dk) : 1.0;  // the diagonal keeps 1 / L_kk
         G[tri(k, k)] = rk;
 #pragma unroll
         for (int i = k + 1; i < NT; ++i) {
-          T s = G[tri(i, k)];
+          double s = G[tri(i, k)];
 #pragma unroll
           for (int j = 0; j < k; ++j) s = fma(-G[tri(i, j)], G[tri(k, j)], s);
           G[tri(i, k)] = s * rk;
@@ -542,15 +529,14 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
     }
     // the regular pass's routes (k_fast.hip, SRC_REGULAR)
     const int bucket = bucket_of(ns * q);
-    const int poor = sizeof(T) == 4        ? ACT_FALLBACK
-                     : bucket < NBUCKET      ? ACT_REFIT
-                     : ns * q <= BIG_MMAX    ? ACT_BIG
-                                             : ACT_FALLBACK;
+    const int poor = bucket < NBUCKET     ? ACT_REFIT
+                     : ns * q <= BIG_MMAX ? ACT_BIG
+                                          : ACT_FALLBACK;
     int act = ACT_NONE;
     if (short_set)
       act = ACT_EXACT;
     else if (work && !rank_ok)
-      act = sizeof(T) == 4 ? ACT_FALLBACK : ACT_EXACT;
+      act = ACT_EXACT;
     else if (work && !(min_ratio >= tau_acc))
       act = poor;
     else if (work)
@@ -561,12 +547,10 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
 #pragma unroll
     for (int k = 0; k < NT; ++k) z[k] = 0;
     if (act == ACT_SOLVE) {
-      T e0[NT], zt[NT];
+      double e0[NT];
 #pragma unroll
       for (int k = 0; k < NT; ++k) e0[k] = k == 0 ? 1 : 0;
-      chol_solve_rcp<T, NT>(G, e0, zt);
-#pragma unroll
-      for (int k = 0; k < NT; ++k) z[k] = (double)zt[k];
+      chol_solve_rcp<double, NT>(G, e0, z);
     }
     if (NREF > 0) {
       double last_dz = 0, zmax = 0;
@@ -591,16 +575,16 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
           });
         group_sum<double, NT>(u, g, gmax);
         if (refine) {
-          T res[NT], dz[NT];
+          double res[NT], dz[NT];
 #pragma unroll
-          for (int k = 0; k < NT; ++k) res[k] = (T)((k == 0 ? 1.0 : 0.0) - u[k]);
-          chol_solve_rcp<T, NT>(G, res, dz);
+          for (int k = 0; k < NT; ++k) res[k] = (k == 0 ? 1.0 : 0.0) - u[k];
+          chol_solve_rcp<double, NT>(G, res, dz);
           last_dz = 0;
           zmax = 0;
 #pragma unroll
           for (int k = 0; k < NT; ++k) {
-            z[k] += (double)dz[k];
-            last_dz = fmax(last_dz, fabs((double)dz[k]));
+            z[k] += dz[k];
+            last_dz = fmax(last_dz, fabs(dz[k]));
             zmax = fmax(zmax, fabs(z[k]));
           }
         }
@@ -699,7 +683,7 @@ __global__ __launch_bounds__(TILE_B) void k_tile(FitArgs a, float tau_rank, floa
   }
 }
 
-template <class T, int NT, int NREF, bool P2>
+template <int NT, int NREF, bool P2>
 int launch_tile_nc(const FitArgs& a, float tau_rank, float tau_acc, hipStream_t s)
 {
   const TileView& tv = a.tiles;
@@ -707,20 +691,20 @@ int launch_tile_nc(const FitArgs& a, float tau_rank, float tau_acc, hipStream_t 
   // at least 8 blocks: tile_walk gives each XCD's range to its own blocks
   const unsigned blocks = (unsigned)std::max<int64_t>(8, std::min<int64_t>(a.shape.tile_blocks, tv.ntile));
   switch (a.nc) {
-    case 1: k_tile<T, NT, 1, NREF, P2><<<blocks, TILE_B, lds, s>>>(a, tau_rank, tau_acc); break;
-    case 3: k_tile<T, NT, 3, NREF, P2><<<blocks, TILE_B, lds, s>>>(a, tau_rank, tau_acc); break;
-    case 9: k_tile<T, NT, 9, NREF, P2><<<blocks, TILE_B, lds, s>>>(a, tau_rank, tau_acc); break;
-    case 27: k_tile<T, NT, 27, NREF, P2><<<blocks, TILE_B, lds, s>>>(a, tau_rank, tau_acc); break;
+    case 1: k_tile<NT, 1, NREF, P2><<<blocks, TILE_B, lds, s>>>(a, tau_rank, tau_acc); break;
+    case 3: k_tile<NT, 3, NREF, P2><<<blocks, TILE_B, lds, s>>>(a, tau_rank, tau_acc); break;
+    case 9: k_tile<NT, 9, NREF, P2><<<blocks, TILE_B, lds, s>>>(a, tau_rank, tau_acc); break;
+    case 27: k_tile<NT, 27, NREF, P2><<<blocks, TILE_B, lds, s>>>(a, tau_rank, tau_acc); break;
     default: return sprg_fail(SPRG_EUNSUPPORTED, "tiled recovery: %d components", a.nc);
   }
   return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "tiled fit launch failed");
 }
 
-template <class T, int NT, int NREF>
+template <int NT, int NREF>
 int launch_tile_p2(const FitArgs& a, float tau_rank, float tau_acc, hipStream_t s)
 {
-  if (a.m.order == 2 && !a.m.straight) return launch_tile_nc<T, NT, NREF, true>(a, tau_rank, tau_acc, s);
-  return launch_tile_nc<T, NT, NREF, false>(a, tau_rank, tau_acc, s);
+  if (a.m.order == 2 && !a.m.straight) return launch_tile_nc<NT, NREF, true>(a, tau_rank, tau_acc, s);
+  return launch_tile_nc<NT, NREF, false>(a, tau_rank, tau_acc, s);
 }
 
 }  // namespace
@@ -735,17 +719,18 @@ int launch_tile_build(const MeshView& m, int64_t ntile, const int32_t* desc, con
   return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "tile build launch failed");
 }
 
-// The fast forms' regular pass over the tiles (the same tolerances as the
-// thread-per-patch pass: FP32 Gram with three FP64 refinement steps, or an
-// FP64 Gram).
+// The fast forms' regular pass over the tiles (the thread-per-patch pass's
+// tolerances).  The refined form (SPRG_FP32R) takes two refinement steps: a
+// recovery of 913k patches takes 0.67 ms, 0.38 of it here.  With an FP32 Gram
+// and factor the pass took 0.42 ms, three steps, and left 432k patches (pivot
+// ratios below FP32's reach) to an FP64 refit of 0.43 ms; the recovered
+// fields' errors against the exact form are the same (RMS 4e-14 to 9e-13).
 int launch_tile_fit(const FitArgs& a, int nterms, int form, hipStream_t s)
 {
   if (a.tiles.ntile == 0) return 0;
   if (form == SPRG_FP32R)
-    return nterms == 4 ? launch_tile_p2<float, 4, 3>(a, 1e-4f, 1e-3f, s)
-                       : launch_tile_p2<float, 10, 3>(a, 1e-4f, 1e-3f, s);
-  return nterms == 4 ? launch_tile_p2<double, 4, 0>(a, 1e-6f, 1e-6f, s)
-                     : launch_tile_p2<double, 10, 0>(a, 1e-6f, 1e-6f, s);
+    return nterms == 4 ? launch_tile_p2<4, 2>(a, 1e-6f, 1e-6f, s) : launch_tile_p2<10, 2>(a, 1e-6f, 1e-6f, s);
+  return nterms == 4 ? launch_tile_p2<4, 0>(a, 1e-6f, 1e-6f, s) : launch_tile_p2<10, 0>(a, 1e-6f, 1e-6f, s);
 }
 
 }  // namespace sprg

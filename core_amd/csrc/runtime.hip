@@ -641,8 +641,7 @@ void carve_lists(const sprg_mesh* m, char* base, int64_t cap, int32_t* x_set, in
   L.x_cursor = x_cursor;
   L.count = p;
   p += 2 * NBUCKET + 2;
-  // [0] status bits, [1] exact-expansion count, [2] fallback entries taken
-  // before the expansion, [3] big-list count, [4] sets k_rank_test tested
+  // [0] status bits, [1] exact-expansion count, [2] unused, [3] big-list count, [4] sets k_rank_test tested
   L.status = p;
   p += 5;
   int32_t* const items = p;
@@ -743,7 +742,7 @@ bool valid_form(int form) { return form == SPRG_FP64 || form == SPRG_FP32R || fo
 // so the sequence can be captured into a HIP graph.  FP64 form: classify ->
 // exact fit of the initial sets -> expansion -> exact fit of the expanded
 // sets.  Fast forms: fit of every patch -> expansion -> fit of the expanded
-// sets -> FP64 fallback -> exact refits.  marks: record the phase events.
+// sets -> fallback -> exact refits.  marks: record the phase events.
 // qr_ws: the exact fits' workspace (FP64 form).
 int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, void* qr_ws, size_t qr_bytes, hipStream_t s, bool marks)
 {
@@ -751,7 +750,7 @@ int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, void* qr_ws, size_
   const int nterms = m->order == 1 ? 4 : 10;
   int rc;
   // the expanded sets' cursors, the counters and the status words (bits, exact
-  // count, fallback start, big count, rank-tested count) follow each other
+  // count, an unused word, big count, rank-tested count) follow each other
   if ((rc = launch_copy_i32(reinterpret_cast<int32_t*>(a.L.x_cursor), nullptr, 4 + NCOUNTS, s))) return rc;
   if (marks) {
     m->phase_last = 0;
@@ -765,13 +764,6 @@ int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, void* qr_ws, size_
     } else if ((rc = launch_fast_fit(a, nterms, form, 0, s))) {
       return rc;
     }
-    if (form == SPRG_FP32R) {
-      // the FP64 pass over the FP32 pass's fallback queue, before the
-      // expansion so that sets it cannot certify still reach the rank test;
-      // the later fallback pass starts after these entries
-      if ((rc = launch_fast_fit(a, nterms, form, 3, s))) return rc;
-      if ((rc = launch_copy_i32(a.L.status + 2, a.L.count + 2 * NBUCKET + 1, 1, s))) return rc;
-    }
   } else {
     if ((rc = launch_classify(a, nterms, s))) return rc;
     int64_t count[NBUCKET];
@@ -784,9 +776,8 @@ int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, void* qr_ws, size_
   if (marks) m->mark(2);
   if (fast) {
     if ((rc = launch_fast_fit(a, nterms, form, 1, s))) return rc;
-    // (an FP64 pass leaves to it only sets above the exact kernels' rows)
-    if ((form == SPRG_FP32R || (int64_t)m->max_set * a.q > BIG_MMAX) && (rc = launch_fast_fit(a, nterms, form, 2, s)))
-      return rc;
+    // the fallback: sets above the exact kernels' rows
+    if ((int64_t)m->max_set * a.q > BIG_MMAX && (rc = launch_fast_fit(a, nterms, form, 2, s))) return rc;
     // poorly conditioned sets: the reference's arithmetic
     if ((rc = launch_qr_lists(a, nterms, 2, s))) return rc;
   } else {

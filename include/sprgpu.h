@@ -51,10 +51,12 @@ enum {
   SPRG_FP64 = 0,   /* plain FP64 form: the reference's Householder QR with
                       explicit Q, operation for operation (bit-identical
                       recovered field) */
-  SPRG_FP32R = 1,  /* FP32 normal equations in a node-centred basis + FP64
-                      residual refinement (3 steps); FP64 fallback for
-                      ill-conditioned patches */
-  SPRG_FP64F = 2   /* the same fast algorithm with FP64 normal equations */
+  SPRG_FP32R = 1,  /* normal equations in a node-centred basis + FP64
+                      residual refinement.  (Factored in FP64: the vector
+                      ALU's FP32 rate is no higher without packed operations,
+                      and an FP32 factor needs one more refinement step and an
+                      FP64 refit of half the patches.) */
+  SPRG_FP64F = 2   /* the same fast algorithm, not refined */
 };
 
 typedef struct sprg_ctx sprg_ctx;
@@ -100,7 +102,8 @@ int sprg_mesh_counts(sprg_mesh* mesh, int64_t* counts);
 int sprg_mesh_phase_times(sprg_mesh* mesh, double* ms, int n);
 /* Patch routes of the last recovery on the mesh: [0] patches, [1] patches
  * queued for the exact rank test / expansion, [2] expanded sets fitted,
- * [3] patches refitted by the fast forms' FP64 fallback, [4] status bits,
+ * [3] patches refitted by the fast forms' fallback
+ * (poorly conditioned sets of more than 512 rows), [4] status bits,
  * [5] queued patches whose expansion needed the reference's rank test,
  * [6] sets above 192 sample rows fitted by the large-set kernel.
  * Writes min(n, 7) values and returns 7.  No reference counterpart. */
