@@ -69,6 +69,59 @@ __device__ __forceinline__ void chol_solve(const T* L, const T* rhs, T* z)
   }
 }
 
+// Forward and back substitution with the Cholesky factor whose diagonal
+// holds the reciprocals of the pivots.
+template <class T, int NT>
+__device__ __forceinline__ void chol_solve_rcp(const T* L, const T* rhs, T* z)
+{
+  T y[NT];
+#pragma unroll
+  for (int k = 0; k < NT; ++k) {
+    T s = rhs[k];
+#pragma unroll
+    for (int j = 0; j < k; ++j) s = fma(-L[tri(k, j)], y[j], s);
+    y[k] = s * L[tri(k, k)];
+  }
+#pragma unroll
+  for (int kk = 0; kk < NT; ++kk) {
+    const int k = NT - 1 - kk;
+    T s = y[k];
+#pragma unroll
+    for (int j = k + 1; j < NT; ++j) s = fma(-L[tri(j, k)], z[j], s);
+    z[k] = s * L[tri(k, k)];
+  }
+}
+
+// 1 / sqrt(d) for d > 0: the hardware estimate and two Newton steps
+// r <- r + r (1/2 - (d/2) r^2), each doubling the correct bits.
+__device__ __forceinline__ double rsqrt_nr(double d)
+{
+  double r = __builtin_amdgcn_rsq(d);
+  const double h = 0.5 * d;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) r = fma(r, fma(-h, r * r, 0.5), r);
+  return r;
+}
+
+// Lane l's value of x from lane l ^ ST (ST = 1, 2, 4), within rows of 16:
+// DPP quad permutations for 1 and 2, a swizzle for 4.
+template <int ST>
+__device__ __forceinline__ int xor_lane(int x)
+{
+  static_assert(ST == 1 || ST == 2 || ST == 4, "lane exchange distance");
+  // every lane reads a lane of its own quad, so no lane needs an old value
+  if constexpr (ST == 1) return __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, true);  // quad_perm 1,0,3,2
+  if constexpr (ST == 2) return __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, true);  // quad_perm 2,3,0,1
+  return __builtin_amdgcn_ds_swizzle(x, 0x101F);                                          // xor 4 in 32 lanes
+}
+
+template <int ST>
+__device__ __forceinline__ double xor_lane(double x)
+{
+  const int lo = xor_lane<ST>(__double2loint(x)), hi = xor_lane<ST>(__double2hiint(x));
+  return __hiloint2double(hi, lo);
+}
+
 // The Gram matrix of the 10-term basis from moments.  Its 55 entries
 // sum_rows f_i f_j are sums of the 35 monomials x^a y^b z^c of degree <= 4
 // of the centred coordinates, so each such moment is accumulated once: per

@@ -137,10 +137,10 @@ __device__ __forceinline__ void sample_d(const MeshView& m, const Geo<P2MAP>& g,
 // tiled pass (k_tile.hip), with the regular pass's decisions.
 enum { SRC_REGULAR = 0, SRC_EXPANDED = 1, SRC_FALLBACK = 2, SRC_LEFTOVER = 4 };
 
-// src SRC_REGULAR walks every patch id and SRC_EXPANDED every queued item; the
-// others walk a list.
+// A thread per patch.  src SRC_REGULAR walks every patch id and SRC_EXPANDED
+// every queued item; the others walk a list.
 template <int NT, int NC, int NREF, bool P2MAP>
-__global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank, float tau_acc)
+__device__ __forceinline__ void fit_threads(const FitArgs& a, int src, float tau_rank, float tau_acc)
 {
   const MeshView& m = a.m;
   const int q = a.q;
@@ -334,6 +334,171 @@ __global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank
   }
 }
 
+template <int NT, int NC, int NREF, bool P2MAP>
+__global__ __launch_bounds__(256) void k_fast(FitArgs a, int src, float tau_rank, float tau_acc)
+{
+  fit_threads<NT, NC, NREF, P2MAP>(a, src, tau_rank, tau_acc);
+}
+
+// Sums v over each eight lanes, every lane ending with the sum.
+template <int N>
+__device__ __forceinline__ void sum8(double* v)
+{
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] += xor_lane<1>(v[k]);
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] += xor_lane<2>(v[k]);
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] += xor_lane<4>(v[k]);
+}
+
+// The expanded sets (the expansion queue's items that found one).  Few sets
+// are fitted by eight lanes each, lane r taking the tets r, r + 8, ...: a
+// thread per set takes as long as its tets' chain of loads and sums, however
+// few the sets (35 us for some hundred; 12 here).  Up to SETS_GROUPED queued
+// sets, a wave of them for every SIMD; with more the threads fill the chip by
+// themselves and do not repeat the factorisation (349 us at 452,700 queued
+// sets of mostly six tets; 714 by groups).
+constexpr int64_t SETS_GROUPED = 65536;
+
+template <int NT, int NC, bool P2MAP>
+__global__ __launch_bounds__(256) void k_fast_sets(FitArgs a, float tau_acc)
+{
+  constexpr int GL = 8;
+  const MeshView& m = a.m;
+  const int q = a.q, rank = threadIdx.x % GL;
+  const int64_t count = a.L.count[2 * NBUCKET];
+  if (count > SETS_GROUPED) {
+    fit_threads<NT, NC, 0, P2MAP>(a, SRC_EXPANDED, 0.0f, tau_acc);
+    return;
+  }
+  const int per = blockDim.x / GL;
+  // (the trip count is the same for every lane of a block: the appends below
+  // and the lane exchanges run on whole waves)
+  for (int64_t base = xcd_block(blockIdx.x, gridDim.x, XCD_K_FIT) * per; base < count;
+       base += (int64_t)gridDim.x * per) {
+    const int64_t it = base + threadIdx.x / GL;
+    const int ns = it < count ? a.L.x_len[it] : 0;
+    const bool valid = ns > 0;
+    const uint64_t found = __ballot(valid && rank == 0);
+    if (!found) continue;
+    if ((threadIdx.x & 63) == 0) atomicAdd(a.L.count + NBUCKET, __popcll(found));
+    const int64_t p = valid ? a.L.x_patch[it] : 0;
+    const int32_t* const set = valid ? a.L.x_set + a.L.x_off[it] : nullptr;
+    const double xn[3] = {m.xyz[3 * p], m.xyz[3 * p + 1], m.xyz[3 * p + 2]};
+    constexpr int NG = NT * (NT + 1) / 2;
+    double G[NG];
+    auto rows = [&](auto body) {
+      for (int s = rank; s < ns; s += GL) {
+        const int32_t t = set[s];
+        Geo<P2MAP> g;
+        load_geo(m, t, P2MAP, g);
+        for (int l = 0; l < q; ++l) {
+          double d[3];
+          sample_d(m, g, P2MAP, l, xn, d);
+          body(t, l, d);
+        }
+      }
+    };
+    if constexpr (NT == 10) {
+      double M[NMOM];
+#pragma unroll
+      for (int k = 0; k < NMOM; ++k) M[k] = 0;
+      rows([&](int32_t, int, const double* d) { moments_row<double>(d, M); });
+      sum8<NMOM>(M);
+      M[0] = (double)(ns * q);
+      gram_from_moments<double>(M, G);
+    } else {
+#pragma unroll
+      for (int k = 0; k < NG; ++k) G[k] = 0;
+      rows([&](int32_t, int, const double* d) {
+        double f[NT];
+        basis<double, NT>(d, f);
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+          for (int j = 0; j <= i; ++j) G[tri(i, j)] = fma(f[i], f[j], G[tri(i, j)]);
+      });
+      sum8<NG>(G);
+    }
+    // Cholesky in place (every lane of the group alike), the diagonal keeping
+    // 1 / L_kk
+    float min_ratio = 1.0f;
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+      const double diag = G[tri(k, k)];
+      double dk = diag;
+#pragma unroll
+      for (int j = 0; j < k; ++j) dk = fma(-G[tri(k, j)], G[tri(k, j)], dk);
+      min_ratio = fminf(min_ratio, diag > 0 && dk > 0 ? (float)(dk / diag) : 0.0f);
+      const double rk = dk > 0 ? rsqrt_nr(dk) : 1.0;
+      G[tri(k, k)] = rk;
+#pragma unroll
+      for (int i = k + 1; i < NT; ++i) {
+        double s = G[tri(i, k)];
+#pragma unroll
+        for (int j = 0; j < k; ++j) s = fma(-G[tri(i, j)], G[tri(k, j)], s);
+        G[tri(i, k)] = s * rk;
+        asm volatile("" : "+v"(G[tri(i, k)]));  // keeps the column's temporaries few
+      }
+    }
+    // an expanded set has passed the reference's rank test; a poor one is
+    // refitted by the exact kernel, which takes every row count it can have
+    const bool solve = valid && min_ratio >= tau_acc;
+    const int bucket = bucket_of(ns * q);
+    const bool poor = valid && rank == 0 && !solve;
+    if (__ballot(poor)) {  // wave-uniform
+      const int32_t e = (int32_t)(it | 0x80000000u);
+      for (int b = 0; b < NBUCKET; ++b) wave_append(b, poor ? bucket : -1, a.L.count + b, a.L.items[b], e);
+      big_append(poor && bucket >= NBUCKET, a.L, e);
+    }
+    double v[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) v[c] = 0;
+    double b0[NC];
+    if (solve) {
+      double e0[NT], z[NT];
+#pragma unroll
+      for (int k = 0; k < NT; ++k) e0[k] = k == 0 ? 1 : 0;
+      chol_solve_rcp<double, NT>(G, e0, z);
+      const double* const bp = a.ip + (int64_t)set[0] * q * NC;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) b0[c] = bp[c];
+      rows([&](int32_t t, int l, const double* d) {
+        const double* const bl = a.ip + ((int64_t)t * q + l) * NC;
+        double f[NT], w = 0;
+        basis<double, NT>(d, f);
+#pragma unroll
+        for (int k = 0; k < NT; ++k) w = fma(f[k], z[k], w);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) v[c] = fma(w, bl[c] - b0[c], v[c]);
+      });
+    }
+    sum8<NC>(v);
+    if (solve && rank == 0) {
+      double* const out = a.out + p * NC;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) out[c] = b0[c] + v[c];
+    }
+  }
+}
+
+template <int NT, bool P2>
+int launch_sets(const FitArgs& a, hipStream_t s)
+{
+  const unsigned threads = (unsigned)a.shape.fast_threads;
+  const unsigned blocks =
+      (unsigned)std::max<int64_t>(1, std::min<int64_t>(a.shape.fast_blocks, (a.npatch + threads - 1) / threads));
+  switch (a.nc) {
+    case 1: k_fast_sets<NT, 1, P2><<<blocks, threads, 0, s>>>(a, 1e-6f); break;
+    case 3: k_fast_sets<NT, 3, P2><<<blocks, threads, 0, s>>>(a, 1e-6f); break;
+    case 9: k_fast_sets<NT, 9, P2><<<blocks, threads, 0, s>>>(a, 1e-6f); break;
+    case 27: k_fast_sets<NT, 27, P2><<<blocks, threads, 0, s>>>(a, 1e-6f); break;
+    default: return sprg_fail(SPRG_EUNSUPPORTED, "fast recovery: %d components", a.nc);
+  }
+  return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "expanded-set fit launch failed");
+}
+
 template <int NT, int NREF, bool P2>
 int launch_nc2(const FitArgs& a, int src, float tau_rank, float tau_acc, hipStream_t s)
 {
@@ -380,7 +545,10 @@ int launch_fast_fit(const FitArgs& a, int nterms, int form, int src, hipStream_t
   // kernel.  Expanded sets (often barely full rank) are not refined: the
   // exact kernel takes their poor ones.
   if (src == SRC_FALLBACK) return launch_t<2>(a, nterms, src, 0.0f, 1e-6f, s);
-  if (src == SRC_EXPANDED) return launch_t<0>(a, nterms, src, 0.0f, 1e-6f, s);
+  if (src == SRC_EXPANDED) {
+    if (nterms == 4) return launch_sets<4, false>(a, s);
+    return a.m.straight ? launch_sets<10, false>(a, s) : launch_sets<10, true>(a, s);
+  }
   // a pivot that keeps less than 1e-6 of its diagonal is not a rank
   // certificate in FP64 (its rounding can exceed 1e-11 of the diagonal after
   // earlier cancellation): such sets take the reference's rank test

@@ -321,25 +321,6 @@ __device__ __forceinline__ void stage_tets(const MeshView& m, const TileNext& n,
   }
 }
 
-// Lane l's value of x from lane l ^ ST (ST = 1, 2, 4), within rows of 16:
-// DPP quad permutations for 1 and 2, a swizzle for 4.
-template <int ST>
-__device__ __forceinline__ int xor_lane(int x)
-{
-  static_assert(ST == 1 || ST == 2 || ST == 4, "lane exchange distance");
-  // every lane reads a lane of its own quad, so no lane needs an old value
-  if constexpr (ST == 1) return __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, true);  // quad_perm 1,0,3,2
-  if constexpr (ST == 2) return __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, true);  // quad_perm 2,3,0,1
-  return __builtin_amdgcn_ds_swizzle(x, 0x101F);                                          // xor 4 in 32 lanes
-}
-
-template <int ST>
-__device__ __forceinline__ double xor_lane(double x)
-{
-  const int lo = xor_lane<ST>(__double2loint(x)), hi = xor_lane<ST>(__double2hiint(x));
-  return __hiloint2double(hi, lo);
-}
-
 // One butterfly level: lanes of groups wider than ST add their partner's
 // value, the others add it times zero.  The partner of a lane outside such a
 // group belongs to another group or to no patch, whose sums are finite (or
@@ -365,17 +346,6 @@ __device__ __forceinline__ void group_sum(T* v, int g, int gmax)
   if (gmax > 4) group_step<4, T, N>(v, g);
 }
 
-// 1 / sqrt(d) for d > 0: the hardware estimate and two Newton steps
-// r <- r + r (1/2 - (d/2) r^2), each doubling the correct bits.
-__device__ __forceinline__ double rsqrt_nr(double d)
-{
-  double r = __builtin_amdgcn_rsq(d);
-  const double h = 0.5 * d;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) r = fma(r, fma(-h, r * r, 0.5), r);
-  return r;
-}
-
 // body(u) for the lane's tets s = rank, rank + g, ... < ns of its patch set
 // (u: the tet's position in the tile's union), the next position loaded
 // while the current tet is processed.
@@ -397,29 +367,6 @@ template <class F>
 __device__ __forceinline__ void for_points(int q, F body)
 {
   for (int l = 0; l < q; ++l) body(l);
-}
-
-// Forward and back substitution with the Cholesky factor whose diagonal
-// holds the reciprocals of the pivots.
-template <class T, int NT>
-__device__ __forceinline__ void chol_solve_rcp(const T* L, const T* rhs, T* z)
-{
-  T y[NT];
-#pragma unroll
-  for (int k = 0; k < NT; ++k) {
-    T s = rhs[k];
-#pragma unroll
-    for (int j = 0; j < k; ++j) s = fma(-L[tri(k, j)], y[j], s);
-    y[k] = s * L[tri(k, k)];
-  }
-#pragma unroll
-  for (int kk = 0; kk < NT; ++kk) {
-    const int k = NT - 1 - kk;
-    T s = y[k];
-#pragma unroll
-    for (int j = k + 1; j < NT; ++j) s = fma(-L[tri(j, k)], z[j], s);
-    z[k] = s * L[tri(k, k)];
-  }
 }
 
 template <int NT, int NC, int NREF, bool P2MAP>
