@@ -389,10 +389,9 @@ constexpr int HSIZE = 1024;  // LDS hash of candidate tets (at most 319 entries)
 
 __device__ __forceinline__ int shared_verts(const int32_t* a, const int32_t* b)
 {
-  int s = 0;
-  for (int i = 0; i < 4; ++i)
-    for (int j = 0; j < 4; ++j) s += (a[i] == b[j]);
-  return s;
+  const int4 x = *reinterpret_cast<const int4*>(a), y = *reinterpret_cast<const int4*>(b);
+  auto in = [&](int v) { return (int)((v == y.x) | (v == y.y) | (v == y.z) | (v == y.w)); };
+  return in(x.x) + in(x.y) + in(x.z) + in(x.w);
 }
 
 __device__ __forceinline__ double readlane_d(double v, int lane)
@@ -407,9 +406,8 @@ __device__ __forceinline__ double readlane_d(double v, int lane)
 // monomials go to LDS (sF, 64 rows at a time, a lane per row); lane
 // l < NT(NT+1)/2 owns Gram entry l of the packed lower triangle, sums it over
 // the rows -- two reads and a fused multiply-add a row -- and keeps it
-// through a right-looking factorisation whose columns travel by
-// lane shuffles (the fused multiply-adds of each entry run in the same order
-// as a left-looking Cholesky's).  Centring is a unit-triangular change of the
+// through a right-looking factorisation whose unscaled columns travel by
+// lane shuffles.  Centring is a unit-triangular change of the
 // graded monomial basis, so in exact arithmetic pivot k equals the
 // reference's Householder column norm R_kk (mth/mthQR.cc:31).  Returns true
 // only when every pivot clears the reference's 1e-10 by 5% and keeps at least
@@ -422,7 +420,9 @@ __device__ __forceinline__ double readlane_d(double v, int lane)
 // FP64 issue bounds it.  With the sample points staged and every lane forming
 // its own two monomials (eleven FP64 operations a row and lane) k_expand<10,
 // false> took 3.29 ms on an undistorted box of 384,000 tets; formed once, by
-// the row's own lane, and read back, one is left of them: 2.64 ms.
+// the row's own lane, and read back, one is left of them: 2.64 ms.  (With
+// the walk's shorter lists 2.33; with the affine map on straight-sided meshes
+// and the pivots' divisions and square roots gone, 2.14.)
 // Every lane of the block (one wave) must call it.
 constexpr int CERT_ROWS = 64;  // rows whose monomials are in LDS at a time
 constexpr int cert_stride(int nt) { return nt + 1; }  // odd: a column's entries in different banks
@@ -444,8 +444,25 @@ __device__ bool certify_full_rank(const MeshView& m, int q, const int32_t* S, in
     if (lane < n) {
       const int i = c0 + lane;
       double x[3], f[10];
-      sample_point<NT == 4 ? 1 : 2>(m, S[i / q], i % q, x);
-      for (int j = 0; j < 3; ++j) x[j] -= xn[j];
+      if (NT == 10 && m.straight) {
+        // the affine map of the four vertices: the same point to rounding
+        const int32_t t = S[i / q];
+        const int l = i % q;
+        const double xa = 0.138196601125011, xb = 0.585410196624969;
+        double w[4];
+        for (int v = 1; v < 4; ++v) w[v] = l == v ? xb : xa;
+        w[0] = 1 - w[1] - w[2] - w[3];
+        const int4 tv = *reinterpret_cast<const int4*>(m.tv + 4 * (int64_t)t);
+        const int32_t node[4] = {tv.x, tv.y, tv.z, tv.w};
+        for (int j = 0; j < 3; ++j) {
+          double y = 0;
+          for (int v = 0; v < 4; ++v) y = fma(w[v], m.xyz[3 * (int64_t)node[v] + j], y);
+          x[j] = y - xn[j];
+        }
+      } else {
+        sample_point<NT == 4 ? 1 : 2>(m, S[i / q], i % q, x);
+        for (int j = 0; j < 3; ++j) x[j] -= xn[j];
+      }
       poly_terms(NT == 4 ? 1 : 2, x, f);
 #pragma unroll
       for (int k = 0; k < NT; ++k) sF[lane * FS + k] = f[k];
@@ -470,22 +487,20 @@ __device__ bool certify_full_rank(const MeshView& m, int q, const int32_t* S, in
   }
   __syncthreads();  // sF is free again
   const double diag_own = g;
-  bool rank_ok = true;
   for (int k = 0; k < NT; ++k) {
     const int kk = k * (k + 1) / 2 + k;
     // the pivot's lane is the same for the whole wave: a lane read, not a
     // shuffle through LDS
     const double dk = readlane_d(g, kk);
     const double diag = readlane_d(diag_own, kk);
-    const double lkk = dk > 0 ? sqrt(dk) : 0.0;
-    if (!(diag > 0 && dk >= 1e-6 * diag) || !(lkk >= 1.05e-10)) rank_ok = false;
-    const double piv = lkk > 0 ? lkk : 1.0;
-    if (own && r > k && c == k) g = g / piv;  // L[r][k]
+    // pivot k of the Cholesky factor is sqrt(dk)
+    if (!(diag > 0 && dk >= 1e-6 * diag) || !(dk >= 1.1025e-20)) return false;
+    const double rk = rsqrt_nr(dk);
     const double lr = __shfl(g, own && r > k ? r * (r + 1) / 2 + k : 0);
     const double lc = __shfl(g, own && c > k ? c * (c + 1) / 2 + k : 0);
-    if (own && c > k) g = fma(-lr, lc, g);
+    if (own && c > k) g = fma(-lr * (rk * rk), lc, g);
   }
-  return rank_ok;
+  return true;
 }
 
 // EXACT = false: the screen alone, with no QR workspace in LDS (several
@@ -592,18 +607,21 @@ __global__ __launch_bounds__(64) void k_expand(FitArgs a)
         for (int i = lane; i < HSIZE; i += 64) sHash[i] = -1;
         if (lane == 0) sN = 0;
         __syncthreads();
-        // items: (tet of the old set, one of its vertices); with P >= the
-        // item count (a power of two, at most 64) each item gets R = 64 / P
-        // lanes, which take its neighbour list's chunks of 8 in turn (the
-        // same candidate pairs as one lane per item, walked in parallel)
-        const int nitem = nold * 4;
+        // items: (tet of the old set, one of its first 4 - sd vertices: a
+        // tet that shares sd + 1 of the four has one of any 4 - sd; walking
+        // all four rows for face neighbours met each of them three times: 2.63
+        // ms for the 452,700 sets of a lattice box, 2.33 now); with P >=
+        // the item count (a power of two, at most 64) each item gets R =
+        // 64 / P lanes, which take its neighbour list's chunks of 8 in turn
+        // (the same candidate pairs as one lane per item, walked in parallel)
+        const int nscan = 4 - sd, nitem = nold * nscan;
         int P = 64;
         while (P > 1 && P / 2 >= nitem) P /= 2;
         const int R = 64 / P, sub = lane / P;
         for (int w = lane % P; w < nitem; w += P) {
-          const int32_t t = sOld[w >> 2];
-          const int32_t* tv = m.tv + 4 * (int64_t)t;
-          const int32_t v = tv[w & 3];
+          const int o = nscan == 3 ? w / 3 : nscan == 2 ? w >> 1 : w >> 2;
+          const int32_t* tv = m.tv + 4 * (int64_t)sOld[o];
+          const int32_t v = tv[w - o * nscan];
           const int32_t k0 = m.v2t_off[v], k1 = m.v2t_off[v + 1];
           // neighbour ids and their vertices eight at a time, so the
           // dependent loads overlap
