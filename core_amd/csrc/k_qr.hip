@@ -245,9 +245,9 @@ constexpr int small_stride(int nt, int mmax) { return (nt * mmax + nt * (nt + 1)
 constexpr int small_lds(int nt, int mmax) { return 64 / nt * small_stride(nt, mmax); }
 
 // The fits of one bucket's list, the launch's blocks (one wave each) taking
-// 64 / NT patches in turn.
+// 64 / NT patches in turn; this one is block `block` of them.
 template <int NT, int MMAX, int MODE>
-__device__ __forceinline__ void small_fit(const FitArgs& a, int bucket, double* sm)
+__device__ __forceinline__ void small_fit(const FitArgs& a, int bucket, double* sm, int block)
 {
   constexpr int ORDER = NT == 4 ? 1 : 2;
   constexpr int G = NT, P = 64 / G;  // lanes per patch, patches per wave
@@ -270,7 +270,7 @@ __device__ __forceinline__ void small_fit(const FitArgs& a, int bucket, double* 
   const int q = a.q, nc = a.nc;
   int nitems;
   const int32_t* const list = fit_list<MODE>(a, bucket, &nitems);
-  for (int base = blockIdx.x * P; base < nitems; base += gridDim.x * P) {
+  for (int base = block * P; base < nitems; base += gridDim.x * P) {
     asm volatile("" : "+v"(gl));  // its many comparisons stay inside the loop (hoisted, they spill)
     const bool act = base + g < nitems;
     int64_t p = 0;
@@ -443,20 +443,29 @@ __global__ __launch_bounds__(64, small_waves(NT, MMAX)) void k_qr_small(FitArgs 
 {
   constexpr int SM = small_lds(NT, MMAX);
   __shared__ double sm[SM];
-  small_fit<NT, MMAX, MODE>(a, bucket, sm);
+  small_fit<NT, MMAX, MODE>(a, bucket, sm, blockIdx.x);
 }
 
-// The lists whose lengths only the device knows, in one launch (most calls
-// have few sets here or none, and an empty launch costs what a full one waits
-// for).
+// The three lists in one launch: the ones whose lengths only the device
+// knows (most calls have few sets there or none, and an empty launch costs
+// what a full one waits for), and the initial sets of small meshes.  A list
+// starts at the block after the last that the one before it needs, so that
+// short lists run side by side.
 template <int NT, int MODE>
 __global__ __launch_bounds__(64, 2) void k_qr_small_lists(FitArgs a)
 {
   constexpr int SM = small_lds(NT, 32);
   __shared__ double sm[SM];
-  small_fit<NT, 16, MODE>(a, 0, sm);
-  small_fit<NT, 24, MODE>(a, 1, sm);
-  small_fit<NT, 32, MODE>(a, 2, sm);
+  constexpr int P = 64 / NT;
+  const int nb = gridDim.x;
+  int block = blockIdx.x, n;
+  small_fit<NT, 16, MODE>(a, 0, sm, block);
+  fit_list<MODE>(a, 0, &n);
+  block = (block + nb - (n + P - 1) / P % nb) % nb;
+  small_fit<NT, 24, MODE>(a, 1, sm, block);
+  fit_list<MODE>(a, 1, &n);
+  block = (block + nb - (n + P - 1) / P % nb) % nb;
+  small_fit<NT, 32, MODE>(a, 2, sm, block);
 }
 
 // ---------------------------------------------------------------------------
@@ -928,6 +937,8 @@ void large_fits(const FitArgs& a, int bucket, int64_t count, double* ws, size_t 
   }
 }
 
+constexpr int64_t SMALL_TOGETHER = 2048;  // two waves a SIMD
+
 template <int NT>
 int regular_fits(const FitArgs& a, const int64_t* count, double* ws, size_t ws_bytes, hipStream_t s)
 {
@@ -937,9 +948,17 @@ int regular_fits(const FitArgs& a, const int64_t* count, double* ws, size_t ws_b
       return sprg_fail(SPRG_ENOMEM, "exact fit: no workspace for a set of %d rows", bucket_rows(b));
   constexpr int P = 64 / NT;
   auto blocks = [&](int b) { return (unsigned)std::min<int64_t>(a.shape.exact_blocks, (count[b] + P - 1) / P); };
-  if (count[0]) k_qr_small<NT, 16, FIT_REGULAR><<<blocks(0), 64, 0, s>>>(a, 0);
-  if (count[1]) k_qr_small<NT, 24, FIT_REGULAR><<<blocks(1), 64, 0, s>>>(a, 1);
-  if (count[2]) k_qr_small<NT, 32, FIT_REGULAR><<<blocks(2), 64, 0, s>>>(a, 2);
+  // all three in one launch while every block of it is on the chip at once
+  // (729 patches: 32 us in two launches, 19 in one); beyond, each by its own
+  // kernel's registers (four more waves a CU for the 16-row sets)
+  const int64_t small = blocks(0) + blocks(1) + blocks(2);
+  if (small > 0 && small <= SMALL_TOGETHER) {
+    k_qr_small_lists<NT, FIT_REGULAR><<<(unsigned)small, 64, 0, s>>>(a);
+  } else {
+    if (count[0]) k_qr_small<NT, 16, FIT_REGULAR><<<blocks(0), 64, 0, s>>>(a, 0);
+    if (count[1]) k_qr_small<NT, 24, FIT_REGULAR><<<blocks(1), 64, 0, s>>>(a, 1);
+    if (count[2]) k_qr_small<NT, 32, FIT_REGULAR><<<blocks(2), 64, 0, s>>>(a, 2);
+  }
   large_fits<NT, 64>(a, 3, count[3], ws, ws_bytes, s);
   large_fits<NT, 96>(a, 4, count[4], ws, ws_bytes, s);
   large_fits<NT, 128>(a, 5, count[5], ws, ws_bytes, s);
