@@ -916,10 +916,13 @@ __global__ __launch_bounds__(256) void k_qr_solve(FitArgs a, int bucket, int fir
   a.out[p * a.nc + c] = backsub_eval<NT>(y, [&](int i, int j) { return Rt[i * NT + j]; }, node);
 }
 
-// Sets per k_qr_reflect / k_qr_rows / k_qr_solve sequence: enough to keep
-// every SIMD's waves busy through several rounds of each launch, and no more
-// (the reflectors and Q of 36,864 96-row sets take 596 MB).
-constexpr int64_t QR_CHUNK = 36864;
+// Sets per k_qr_reflect / k_qr_rows / k_qr_solve sequence: two waves of
+// k_qr_reflect (six sets each) for every SIMD and twelve rounds of k_qr_rows,
+// so no launch ends in a part round, and little enough (199 MB of reflectors
+// and Q at 96 rows) that each launch finds the last one's results in the
+// 256 MB memory-side cache.  A step at 10.4M tets: 84.2 ms; 36,864 sets at a
+// time 90.3, 18,432 86.0, 6,144 99.6.
+constexpr int64_t QR_CHUNK = 12288;
 
 template <int NT, int MMAX>
 void large_fits(const FitArgs& a, int bucket, int64_t count, double* ws, size_t ws_bytes, hipStream_t s)
