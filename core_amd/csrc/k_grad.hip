@@ -24,9 +24,9 @@
 // loads its nodes itself, and the results leave the same way.
 // Measured (calls on an order-2 mesh and field, four points): vector fields
 // on 5.3M tets 0.73 -> 0.67 ms, the vector ALU 75% busy with the 560 FP64
-// operations a point needs and the address unit 78%; matrix fields on 664k
-// tets 0.245 -> 0.126 ms, 4.7 TB/s of stores in the kernel (a thread per point
-// with run-time orders and 27 strided stores before).
+// operations a point needs and the address unit 78%; matrix fields on 384k
+// tets 0.245 -> 0.127 ms, 2.7 TB/s of stores in the kernel at three waves per
+// SIMD (a thread per point with run-time orders and 27 strided stores before).
 #include "device.h"
 #include "spr_math.h"
 

@@ -29,14 +29,13 @@
 // vector registers) and leaves Q's columns, k_qr_solve finishes.
 //
 // Measured, 14.0M patches of a 10.4M-tet mesh, 9 components: 225 ms with one
-// lane group per patch running the sums, 87.5 ms so; sets of 16 rows (6.1M)
-// 24.8 -> 9.2 ms, of 24 rows (6.1M) 69.8 -> 18.2 ms, of 65 to 96 rows (1.7M)
-// 123.6 -> 60.4 ms (reflectors 12.1, Q 40.1, solve 8.2).  Bounds: the FP64
+// lane group per patch running the sums, 81.4 ms so; sets of 16 rows (6.1M)
+// 24.8 -> 8.8 ms, of 24 rows (6.1M) 69.8 -> 17.9 ms, of 65 to 96 rows (1.7M)
+// 123.6 -> 54.6 ms (reflectors 13.4, Q 33.3, solve 7.9).  Bounds: the FP64
 // issue of the separate multiplies and adds (no fused ones exist here): VALU
-// busy 66% in the small fits, 61% in Q, whose two waves per SIMD (96 doubles a
-// lane) wait for the scalar loads.  Q with the reflectors in LDS, a wave's
-// lanes filled with the rows of two sets: 1.39 ms per 36,864 sets instead of
-// 0.87.
+// busy 66% in the small fits; Q's two waves per SIMD (96 doubles a lane) wait
+// for the scalar loads.  Q with the reflectors in LDS, a wave's lanes filled
+// with the rows of two sets, took 1.6 times as long.
 #include <algorithm>
 
 #include "exact_common.h"
