@@ -55,9 +55,11 @@ struct sprg_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   void* scratch = nullptr;  // this device's address of `scratch` (below)
-  // reflectors of the exact fits (k_qr.hip): the context's calls run one
-  // after the other on its stream, so its meshes share it
+  // reflectors of the exact fits (k_qr.hip), shared by the context's meshes:
+  // a call holds qr_mu from the first look at it until its work is complete,
+  // so calls of several threads take turns
   DBuf qr_ws;
+  std::mutex qr_mu;
 };
 
 struct sprg_mesh {
@@ -681,9 +683,8 @@ int ensure_qr_ws(const sprg_mesh* m, int q, DBuf& ws)
   return rc;
 }
 
-// Lays the work lists out in the mesh's own workspaces, and sizes the exact
-// fits' ws (all grown as needed).
-int setup_lists(sprg_mesh* m, FitArgs& a, DBuf& ws)
+// Lays the work lists out in the mesh's own workspaces (grown as needed).
+int setup_lists(sprg_mesh* m, FitArgs& a)
 {
   const int64_t np = m->npatch();
   if (m->list_cap < np) {
@@ -698,8 +699,6 @@ int setup_lists(sprg_mesh* m, FitArgs& a, DBuf& ws)
     m->xset_cap = cap;
   }
   carve_lists(m, m->lists.as<char>(), m->list_cap, m->xset.as<int32_t>(), m->xset_cap, a);
-  if (!a.fast)
-    if (int rc = ensure_qr_ws(m, a.q, ws)) return rc;
   if (big_grid(m, a.q) > 0) {
     int rc = m->big_ws.ensure(big_ws_bytes(big_grid(m, a.q)));
     if (rc) return rc;
@@ -837,16 +836,32 @@ int check_form(int form, int q)
   return 0;
 }
 
+// A call's hold on the context's exact-fit workspace (the fast forms do not
+// use it).
+std::unique_lock<std::mutex> hold_qr_ws(sprg_ctx* c, int form)
+{
+  return form == SPRG_FP64 ? std::unique_lock<std::mutex>(c->qr_mu) : std::unique_lock<std::mutex>();
+}
+
+// enqueue_recover with the context's workspace, sized here; the caller holds it.
+int eager_recover(sprg_mesh* m, const FitArgs& a, int form, hipStream_t s)
+{
+  if (form != SPRG_FP64) return enqueue_recover(m, a, form, nullptr, 0, s, true);
+  DBuf& ws = m->ctx->qr_ws;
+  const int rc = ensure_qr_ws(m, a.q, ws);
+  return rc ? rc : enqueue_recover(m, a, form, ws.p, ws.bytes, s, true);
+}
+
 int run_recover(sprg_mesh* m, int q, int nc, const double* ip, double* out, int form)
 {
   if (int rc = check_form(form, q)) return rc;
+  const auto hold = hold_qr_ws(m->ctx, form);
   hipStream_t s = m->ctx->stream;
   for (int attempt = 0; attempt < 4; ++attempt) {
     FitArgs a = fit_args(m, q, nc, ip, out, form);
-    DBuf& ws = m->ctx->qr_ws;
-    int rc = setup_lists(m, a, ws);
+    int rc = setup_lists(m, a);
+    if (!rc) rc = eager_recover(m, a, form, s);
     if (rc) return rc;
-    if ((rc = enqueue_recover(m, a, form, ws.p, ws.bytes, s, true))) return rc;
     int32_t st = 0;
     if ((rc = read_status(m, a, &st))) return rc;
     collect_phases(m);
@@ -1008,6 +1023,7 @@ int run_estimate(sprg_mesh* m, int ip_order, int nc, const double* ip, int targe
   HIP_OK(hipSetDevice(m->ctx->device), "hipSetDevice");
   if ((rc = check_form(form, q))) return rc;
   if ((rc = estimate_buffers(m, nc))) return rc;
+  const auto hold = hold_qr_ws(m->ctx, form);
   // recovery and estimate without a wait between them: the estimate of a
   // recovery that failed is not used (and writes no sizes)
   hipStream_t s = m->ctx->stream;
@@ -1015,9 +1031,9 @@ int run_estimate(sprg_mesh* m, int ip_order, int nc, const double* ip, int targe
   bool retry = true;
   for (int attempt = 0; attempt < 4 && retry; ++attempt) {
     FitArgs a = fit_args(m, q, nc, ip, m->rec.as<double>(), form);
-    DBuf& ws = m->ctx->qr_ws;
-    if ((rc = setup_lists(m, a, ws))) return rc;
-    if ((rc = enqueue_recover(m, a, form, ws.p, ws.bytes, s, true))) return rc;
+    rc = setup_lists(m, a);
+    if (!rc) rc = eager_recover(m, a, form, s);
+    if (rc) return rc;
     EstArgs e = est_args(m, a.L, ip_order, nc, ip, target, ar, tn, alpha, beta, size, nullptr);
     if ((rc = launch_estimate(e, s, [m](int i) { m->mark(i); }))) return rc;
     Report r;
@@ -1230,7 +1246,7 @@ extern "C" int sprg_patch_sets(sprg_mesh* m, int ip_order, int64_t* set_off, int
   a.q = q;
   a.nc = 0;
   a.npatch = m->npatch();
-  if ((rc = setup_lists(m, a, m->ctx->qr_ws))) return rc;
+  if ((rc = setup_lists(m, a))) return rc;
   hipStream_t s = m->ctx->stream;
   int64_t nitems = 0;
   HIP_OK(hipMemcpyAsync(&nitems, a.L.x_cursor + 1, sizeof(int64_t), hipMemcpyDeviceToHost, s), "items");
@@ -1378,7 +1394,8 @@ int record_batch(sprg_batch* b, int ip_order, int nc, const double* const* ip,
     int rc = estimate_buffers(m, nc);
     if (!rc) {
       fa[i] = fit_args(m, q, nc, ip[i], m->rec.as<double>(), form);
-      rc = setup_lists(m, fa[i], lane_ws(b, b->lane_of[i]));
+      rc = setup_lists(m, fa[i]);
+      if (!rc && form == SPRG_FP64) rc = ensure_qr_ws(m, q, lane_ws(b, b->lane_of[i]));
     }
     if (rc) return rc;
   }
@@ -1391,7 +1408,8 @@ int record_batch(sprg_batch* b, int ip_order, int nc, const double* const* ip,
     for (int i = 0; i < n && !rc; ++i) {
       if (b->lane_of[i] != l) continue;
       sprg_mesh* m = b->meshes[i];
-      rc = enqueue_recover(m, fa[i], form, ws.p, ws.bytes, s, false);
+      rc = form == SPRG_FP64 ? enqueue_recover(m, fa[i], form, ws.p, ws.bytes, s, false)
+                             : enqueue_recover(m, fa[i], form, nullptr, 0, s, false);
       if (!rc) {
         const bool tgt = target != nullptr;
         EstArgs e = est_args(m, fa[i].L, ip_order, nc, ip[i], tgt ? 1 : 0, ar, tgt ? (double)target[i] : 0,
@@ -1425,7 +1443,8 @@ int workspace_key(sprg_batch* b, int q, int nc, int form, std::vector<uint64_t>&
     sprg_mesh* const m = b->meshes[i];
     int rc = estimate_buffers(m, nc);
     FitArgs a = fit_args(m, q, nc, nullptr, nullptr, form);
-    if (!rc) rc = setup_lists(m, a, lane_ws(b, b->lane_of[i]));
+    if (!rc) rc = setup_lists(m, a);
+    if (!rc && form == SPRG_FP64) rc = ensure_qr_ws(m, q, lane_ws(b, b->lane_of[i]));
     if (rc) return rc;
     const DBuf* bufs[] = {&m->rec, &m->lists, &m->xset, &m->elem, &m->partial, &m->scalars, &m->big_ws};
     for (const DBuf* d : bufs) {
@@ -1440,7 +1459,7 @@ int workspace_key(sprg_batch* b, int q, int nc, int form, std::vector<uint64_t>&
     key.push_back((uint64_t)m->shape.expand_blocks);
     key.push_back((uint64_t)m->shape.tile_blocks);
   }
-  for (int l = 0; l < BATCH_LANES; ++l) {
+  for (int l = 0; l < BATCH_LANES && form == SPRG_FP64; ++l) {
     key.push_back((uint64_t)(uintptr_t)lane_ws(b, l).p);
     key.push_back((uint64_t)lane_ws(b, l).bytes);
   }
@@ -1473,6 +1492,7 @@ extern "C" int sprg_batch_size(sprg_batch* b, int ip_order, int nc, const double
     return sprg_fail(SPRG_EINVAL, "getTargetSPRSizeField: alpha must be < beta");
   HIP_OK(hipSetDevice(b->ctx->device), "hipSetDevice");
   hipStream_t s = b->ctx->stream;
+  const auto hold = hold_qr_ws(b->ctx, form);  // lane 0 uses the context's
   for (int attempt = 0; attempt < 4; ++attempt) {
     std::vector<uint64_t> key = {(uint64_t)ip_order, (uint64_t)nc, (uint64_t)form, bits(adapt_ratio),
                                  bits(alpha), bits(beta), target ? 1u : 0u};

@@ -45,7 +45,8 @@ def _read_json(path):
 
 
 def context(device=0):
-    """The library context (one HIP stream) of a device."""
+    """The library context (one HIP stream) of a device, shared by its
+    meshes.  Exact-form calls of several threads on it take turns."""
     if device not in _CTX:
         L = _lib.lib()
         h = _lib.ctypes.c_void_p()

@@ -129,12 +129,26 @@ static std::vector<Rec> g_rec;
 
 void run_launch(const char* where, dim3 grid, dim3 block, size_t shmem, const std::function<void()>& fn);
 
+// Launches of several host threads run one at a time, in the order they ask
+// (a launch owns the globals above; threads that launch in turn interleave
+// launch by launch, as their calls may on one stream).
+static std::atomic<unsigned> g_ticket{0}, g_turn{0};
+struct Turn {
+  const unsigned mine = g_ticket.fetch_add(1);
+  Turn()
+  {
+    while (g_turn.load(std::memory_order_acquire) != mine) std::this_thread::yield();
+  }
+  ~Turn() { g_turn.fetch_add(1, std::memory_order_release); }
+};
+
 void launch(const char* where, dim3 grid, dim3 block, size_t shmem, const std::function<void()>& fn)
 {
   if (g_capturing) {
     g_rec.push_back({where, grid, block, shmem, fn});
     return;
   }
+  Turn turn;
   run_launch(where, grid, block, shmem, fn);
 }
 
@@ -229,8 +243,15 @@ const char* hipGetErrorString(hipError_t) { return "emu error"; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (void*)1; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+// a device that grants no allocation above this many bytes
+static std::atomic<size_t> g_malloc_limit{SIZE_MAX};
+extern "C" void emu_malloc_limit(size_t n) { g_malloc_limit = n; }
 hipError_t hipMalloc(void** p, size_t n)
 {
+  if (n > g_malloc_limit) {
+    *p = nullptr;
+    return hipErrorOutOfMemory;
+  }
   *p = malloc(n ? n : 1);
   if (!*p) return hipErrorOutOfMemory;
   memset(*p, 0xA5, n);  // garbage pattern: uninitialised reads show up as NaN-ish values
