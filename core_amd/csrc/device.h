@@ -218,10 +218,13 @@ int launch_classify(const FitArgs& a, int nterms, hipStream_t s);
 // The exact fits of the lists (k_qr.hip).  launch_qr_regular: the classified
 // regular patches, count[b] of them in bucket b; ws: workspace for the
 // reflectors of sets above 32 rows (any size that holds one set; qr_ws_bytes
-// gives the useful maximum).  launch_qr_lists: mode 1: expanded sets, 2: the
+// gives that and the useful maximum).  launch_qr_lists: mode 1: expanded sets, 2: the
 // fast forms' refits (items[] lists holding patch ids or, with bit 31,
 // expanded-set ids), whose counts only the device knows.
-size_t qr_ws_bytes(int nterms, const int64_t* count);
+struct QrWsBytes {
+  size_t least = 0, most = 0;
+};
+QrWsBytes qr_ws_bytes(int nterms, const int64_t* count);
 int launch_qr_regular(const FitArgs& a, int nterms, const int64_t* count, void* ws, size_t ws_bytes, hipStream_t s);
 int launch_qr_lists(const FitArgs& a, int nterms, int mode, hipStream_t s);
 // The buckets of more than 32 rows of the same lists (k_exact.hip).

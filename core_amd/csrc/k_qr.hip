@@ -970,12 +970,16 @@ int regular_fits(const FitArgs& a, const int64_t* count, double* ws, size_t ws_b
 
 }  // namespace
 
-size_t qr_ws_bytes(int nterms, const int64_t* count)
+QrWsBytes qr_ws_bytes(int nterms, const int64_t* count)
 {
-  size_t most = 0;
+  QrWsBytes n;
   for (int b = NSMALL; b < NBUCKET; ++b)
-    most = std::max(most, qr_set_bytes(nterms, bucket_rows(b)) * (size_t)std::min<int64_t>(count[b], QR_CHUNK));
-  return most;
+    if (count[b]) {
+      const size_t set = qr_set_bytes(nterms, bucket_rows(b));
+      n.least = std::max(n.least, set);
+      n.most = std::max(n.most, set * (size_t)std::min<int64_t>(count[b], QR_CHUNK));
+    }
+  return n;
 }
 
 int launch_qr_regular(const FitArgs& a, int nterms, const int64_t* count, void* ws, size_t ws_bytes, hipStream_t s)

@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <cstdint>
 #include <cstring>
 #include <iterator>
 #include <mutex>
@@ -49,6 +50,46 @@ struct DBuf {
   T* as() const { return static_cast<T*>(p); }
 };
 
+// The exact fits' workspace: the useful maximum, or as much of it as the
+// device grants, but never less than one set.  What is in use is given up only
+// for something larger in hand, so a call never loses a buffer that serves it,
+// and a size the device refused is not asked for again, so a recorded batch's
+// buffer does not move from call to call.
+struct QrWs {
+  DBuf buf;
+  size_t refused = SIZE_MAX;  // the least size refused
+  void release()
+  {
+    buf.release();
+    refused = SIZE_MAX;
+  }
+  int ensure(const QrWsBytes& n)
+  {
+    for (int turn = 0; n.most > buf.bytes; ++turn) {
+      for (size_t want = n.most;; want = std::max(want / 2, n.least)) {
+        if (want <= buf.bytes) return 0;
+        if (want < refused) {
+          void* p = nullptr;
+          if (hipMalloc(&p, want) == hipSuccess) {
+            buf.release();
+            buf.p = p;
+            buf.bytes = want;
+            return 0;
+          }
+          (void)hipGetLastError();
+          refused = want;
+        }
+        if (want == n.least) break;
+      }
+      // not even one set, beside what there is: without it, and afresh
+      release();
+      if (turn == 1)
+        return sprg_fail(SPRG_ENOMEM, "device allocation of %zu bytes failed", n.least);
+    }
+    return 0;
+  }
+};
+
 }  // namespace
 
 struct sprg_ctx {
@@ -58,7 +99,7 @@ struct sprg_ctx {
   // reflectors of the exact fits (k_qr.hip), shared by the context's meshes:
   // a call holds qr_mu from the first look at it until its work is complete,
   // so calls of several threads take turns
-  DBuf qr_ws;
+  QrWs qr_ws;
   std::mutex qr_mu;
 };
 
@@ -534,6 +575,10 @@ extern "C" int sprg_mesh_destroy(sprg_mesh* m)
   for (DBuf* b : all) b->release();
   for (int i = 0; i <= NPHASE; ++i)
     if (m->ev[i]) (void)hipEventDestroy(m->ev[i]);
+  {
+    std::lock_guard<std::mutex> lk(m->ctx->qr_mu);
+    m->ctx->qr_ws.refused = SIZE_MAX;  // there is more memory now
+  }
   delete m;
   return 0;
 }
@@ -671,16 +716,12 @@ void carve_lists(const sprg_mesh* m, char* base, int64_t cap, int32_t* x_set, in
   L.cap = cap;
 }
 
-// The exact fits' workspace, for the mesh's sets at q points per tet: the
-// useful maximum, or as much of it as the device grants.
-int ensure_qr_ws(const sprg_mesh* m, int q, DBuf& ws)
+// What the exact fits of the mesh's sets need at q points per tet.
+QrWsBytes qr_need(const sprg_mesh* m, int q)
 {
   int64_t count[NBUCKET];
   bucket_counts(m, q, count);
-  int rc = 0;
-  for (size_t want = qr_ws_bytes(m->order == 1 ? 4 : 10, count), k = 0; k < 6 && ws.bytes < want >> k; ++k)
-    if (!(rc = ws.ensure(want >> k))) break;
-  return rc;
+  return qr_ws_bytes(m->order == 1 ? 4 : 10, count);
 }
 
 // Lays the work lists out in the mesh's own workspaces (grown as needed).
@@ -847,9 +888,9 @@ std::unique_lock<std::mutex> hold_qr_ws(sprg_ctx* c, int form)
 int eager_recover(sprg_mesh* m, const FitArgs& a, int form, hipStream_t s)
 {
   if (form != SPRG_FP64) return enqueue_recover(m, a, form, nullptr, 0, s, true);
-  DBuf& ws = m->ctx->qr_ws;
-  const int rc = ensure_qr_ws(m, a.q, ws);
-  return rc ? rc : enqueue_recover(m, a, form, ws.p, ws.bytes, s, true);
+  QrWs& ws = m->ctx->qr_ws;
+  const int rc = ws.ensure(qr_need(m, a.q));
+  return rc ? rc : enqueue_recover(m, a, form, ws.buf.p, ws.buf.bytes, s, true);
 }
 
 int run_recover(sprg_mesh* m, int q, int nc, const double* ip, double* out, int form)
@@ -1289,7 +1330,7 @@ struct sprg_batch {
   // lane 0 is the context's stream and uses its exact-fit workspace; the
   // others have their own
   hipStream_t lane[BATCH_LANES] = {};
-  DBuf qr_ws[BATCH_LANES];
+  QrWs qr_ws[BATCH_LANES];
   std::vector<int> lane_of;  // each mesh's lane
   hipGraph_t graph[BATCH_LANES] = {};
   hipGraphExec_t exec[BATCH_LANES] = {};
@@ -1376,7 +1417,7 @@ uint64_t bits(double x)
 }
 
 // The exact-fit workspace of a lane (its meshes run one after the other).
-DBuf& lane_ws(sprg_batch* b, int l) { return l == 0 ? b->ctx->qr_ws : b->qr_ws[l]; }
+QrWs& lane_ws(sprg_batch* b, int l) { return l == 0 ? b->ctx->qr_ws : b->qr_ws[l]; }
 
 // Records the pipelines of every mesh of the batch, a graph per lane.
 // target: NULL (getSPRSizeField for every mesh) or one element count per
@@ -1387,22 +1428,17 @@ int record_batch(sprg_batch* b, int ip_order, int nc, const double* const* ip,
 {
   const int n = (int)b->meshes.size();
   int q = rule_npoints(ip_order);
-  // every allocation happens before the capture
+  // the capture allocates nothing: workspace_key has
   std::vector<FitArgs> fa(n);
   for (int i = 0; i < n; ++i) {
     sprg_mesh* m = b->meshes[i];
-    int rc = estimate_buffers(m, nc);
-    if (!rc) {
-      fa[i] = fit_args(m, q, nc, ip[i], m->rec.as<double>(), form);
-      rc = setup_lists(m, fa[i]);
-      if (!rc && form == SPRG_FP64) rc = ensure_qr_ws(m, q, lane_ws(b, b->lane_of[i]));
-    }
-    if (rc) return rc;
+    fa[i] = fit_args(m, q, nc, ip[i], m->rec.as<double>(), form);
+    if (int rc = setup_lists(m, fa[i])) return rc;
   }
   for (int l = 0; l < BATCH_LANES; ++l) {
     if (std::find(b->lane_of.begin(), b->lane_of.end(), l) == b->lane_of.end()) continue;
     hipStream_t s = b->lane[l];
-    const DBuf& ws = lane_ws(b, l);
+    const DBuf& ws = lane_ws(b, l).buf;
     HIP_OK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture");
     int rc = 0;
     for (int i = 0; i < n && !rc; ++i) {
@@ -1439,13 +1475,19 @@ int record_batch(sprg_batch* b, int ip_order, int nc, const double* const* ip,
 // eager call that grew one since the recording shows up as a new address.
 int workspace_key(sprg_batch* b, int q, int nc, int form, std::vector<uint64_t>& key)
 {
+  QrWsBytes need[BATCH_LANES];  // each lane's, over its meshes
   for (size_t i = 0; i < b->meshes.size(); ++i) {
     sprg_mesh* const m = b->meshes[i];
     int rc = estimate_buffers(m, nc);
     FitArgs a = fit_args(m, q, nc, nullptr, nullptr, form);
     if (!rc) rc = setup_lists(m, a);
-    if (!rc && form == SPRG_FP64) rc = ensure_qr_ws(m, q, lane_ws(b, b->lane_of[i]));
     if (rc) return rc;
+    if (form == SPRG_FP64) {
+      QrWsBytes& lane = need[b->lane_of[i]];
+      const QrWsBytes one = qr_need(m, q);
+      lane.least = std::max(lane.least, one.least);
+      lane.most = std::max(lane.most, one.most);
+    }
     const DBuf* bufs[] = {&m->rec, &m->lists, &m->xset, &m->elem, &m->partial, &m->scalars, &m->big_ws};
     for (const DBuf* d : bufs) {
       key.push_back((uint64_t)(uintptr_t)d->p);
@@ -1460,8 +1502,10 @@ int workspace_key(sprg_batch* b, int q, int nc, int form, std::vector<uint64_t>&
     key.push_back((uint64_t)m->shape.tile_blocks);
   }
   for (int l = 0; l < BATCH_LANES && form == SPRG_FP64; ++l) {
-    key.push_back((uint64_t)(uintptr_t)lane_ws(b, l).p);
-    key.push_back((uint64_t)lane_ws(b, l).bytes);
+    QrWs& ws = lane_ws(b, l);
+    if (int rc = ws.ensure(need[l])) return rc;
+    key.push_back((uint64_t)(uintptr_t)ws.buf.p);
+    key.push_back((uint64_t)ws.buf.bytes);
   }
   return 0;
 }

@@ -59,10 +59,10 @@ class Stars:
         _lib.check(L.sprg_recover(self.m, 1, 3, P(self.ip), P(out), 0))
         return out
 
-    def size(self):
+    def size(self, form=0):
         s = np.full(self.h.nv, np.nan)
         diag = np.zeros(4)
-        _lib.check(L.sprg_spr_size(self.m, 1, 3, P(self.ip), 0.1, P(s), 0, P(diag)))
+        _lib.check(L.sprg_spr_size(self.m, 1, 3, P(self.ip), 0.1, P(s), form, P(diag)))
         return s
 
     def close(self):
@@ -92,7 +92,76 @@ def threads(ctx):
     b.close()
 
 
-CHECKS = {"threads": threads}
+def limit(nbytes):
+    L.emu_malloc_limit(ctypes.c_size_t(nbytes))
+
+
+FREE = 2**64 - 1
+
+
+def refused(ctx):
+    # four sets of 40 rows: 4,224 bytes of workspace each (the reflectors, R's
+    # top and Q of a 4-term fit of up to 64 rows)
+    one = 8 * (4 * 64 + 16 + 64 * 4)
+    s = Stars(ctx, 4, 40, 3)
+    s.size(form=2)  # everything but the exact fits' workspace is there now
+    limit(2 * one)
+    check("half of the workspace granted", np.array_equal(s.recover(), s.ref))
+    limit(0)
+    for k in range(2):
+        check("nothing granted beside it, call %d" % k, np.array_equal(s.recover(), s.ref))
+    limit(FREE)
+    check("all granted again", np.array_equal(s.recover(), s.ref))
+    # a set that the buffer at hand does not hold, on a device without room
+    big = Stars(ctx, 1, 180, 4)
+    big.size(form=2)
+    limit(0)
+    out = np.zeros((big.h.nv, 3))
+    check("no room for one set: refused",
+          L.sprg_recover(big.m, 1, 3, P(big.ip), P(out), 0) == _lib.SPRG_ENOMEM)
+    limit(FREE)
+    check("granted once there is room", np.array_equal(big.recover(), big.ref))
+    check("and the smaller sets still fit", np.array_equal(s.recover(), s.ref))
+    big.close()
+    # batches: recorded once, then replayed, with part of the workspace, and
+    # recorded again where an eager call has moved the context's
+    parts = [Stars(ctx, 4, 40 + 2 * i, 5 + i) for i in range(5)]
+    want = [p.size() for p in parts]
+    fresh = vp()
+    _lib.check(L.sprg_ctx_create(0, ctypes.byref(fresh)))
+    for p in parts:
+        p.close()
+    parts = [Stars(fresh, 4, 40 + 2 * i, 5 + i) for i in range(5)]
+    for p in parts:
+        p.size(form=2)
+    arr = (vp * 5)(*[p.m.value for p in parts])
+    b = vp()
+    _lib.check(L.sprg_batch_create(fresh, 5, arr, ctypes.byref(b)))
+    outs = [np.zeros(p.h.nv) for p in parts]
+    ips = (vp * 5)(*[p.ip.ctypes.data for p in parts])
+    ops = (vp * 5)(*[o.ctypes.data for o in outs])
+    t = np.zeros(1)
+    limit(2 * one)
+    graphs = []
+    for k in range(4):
+        for o in outs:
+            o[:] = -1.0
+        if k == 3:
+            limit(FREE)
+            Stars(fresh, 1, 40, 9).close()  # memory came back: the next call may ask for more
+            check("mesh 0 alone", np.array_equal(parts[0].recover(), parts[0].ref))
+        _lib.check(L.sprg_batch_size(b, 1, 3, ips, None, 0.1, 0.25, 2.0, ops, 0, P(t)))
+        graphs.append(L.emu_graph_count())
+        check("batch run %d equals the per-mesh calls" % k, all(np.array_equal(o, w) for o, w in zip(outs, want)))
+    check("later runs replay: graphs recorded %s" % graphs, graphs[0] == graphs[1] == graphs[2])
+    check("recorded again where the context's workspace moved", graphs[3] > graphs[2])
+    L.sprg_batch_destroy(b)
+    for p in parts + [s]:
+        p.close()
+    _lib.check(L.sprg_ctx_destroy(fresh))
+
+
+CHECKS = {"threads": threads, "refused": refused}
 
 if __name__ == "__main__":
     ctx = vp()

@@ -225,7 +225,14 @@ hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind)
 }
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { emu::begin_capture(); return hipSuccess; }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { *g = new emu_graph{emu::end_capture()}; return hipSuccess; }
-hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, void*, void*, size_t) { *e = new emu_graph{g->nodes}; return hipSuccess; }
+static int g_graphs = 0;  // graphs instantiated so far
+extern "C" int emu_graph_count() { return g_graphs; }
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, void*, void*, size_t)
+{
+  ++g_graphs;
+  *e = new emu_graph{g->nodes};
+  return hipSuccess;
+}
 hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) { emu::replay(e->nodes); return hipSuccess; }
 hipError_t hipGraphDestroy(hipGraph_t g) { delete g; return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t e) { delete e; return hipSuccess; }
