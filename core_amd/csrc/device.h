@@ -56,6 +56,10 @@ enum {
   ST_ILLCOND = 16        // a patch too ill-conditioned for the FP64 fallback
 };
 
+// x_len of an item without a set whose initial set k_rank_test has found to
+// lack rank.
+constexpr int32_t X_TESTED = -1;
+
 struct Lists {
   // FP64 form: the regular patches of each bucket, one after the other in
   // one array (the mesh's set sizes give the bucket sizes beforehand); fast
@@ -66,7 +70,7 @@ struct Lists {
   int32_t* xitems[NBUCKET];
   int32_t* xq;               // patches queued for the exact rank test /
                              // expansion; bit 31: test the initial set
-                             // first, bit 30: it was tested (k_rank_test)
+                             // first
   int32_t* xq_exact;         // queued patches whose expansion needs the exact
                              // rank test (same encoding as xq); its count
                              // follows the status word
@@ -82,7 +86,7 @@ struct Lists {
   int32_t* x_len;
   int32_t* x_set;
   int64_t* x_cursor;         // [0] set entries reserved, [1] item ids (one
-                             // per queued patch; x_len 0: no set stored)
+                             // per queued patch; x_len <= 0: no set stored)
   int64_t x_cap;             // capacity of x_set
   int64_t cap;               // capacity of each list (>= number of patches)
   int32_t* status;

@@ -541,18 +541,21 @@ __global__ __launch_bounds__(64) void k_expand(FitArgs a)
   if (lane == 0) { sBase = 0; sLeft = 0; }
   for (int k = blockIdx.x; k < nq; k += gridDim.x) {
     // the item id of a queued patch is its position in xq; it is marked
-    // empty first (x_len 0: by k_rank_test in the fast forms) and whichever
+    // empty first (by k_rank_test in the fast forms) and whichever
     // pass finds the set fills it
     const int32_t it = EXACT ? queue[k] : k;
     const int32_t entry = a.L.xq[it];
+    bool tested = false;  // k_rank_test has counted this item
     if (!EXACT) {
       if (a.fast) {
-        if (a.L.x_len[it] > 0) continue;  // k_rank_test kept the initial set
+        const int len = a.L.x_len[it];
+        if (len > 0) continue;  // k_rank_test kept the initial set
+        tested = len == X_TESTED;
       } else if (lane == 0) {
         a.L.x_len[it] = 0;
       }
     }
-    const int64_t p = entry & 0x3fffffff;  // bit 30: the initial set's rank is tested
+    const int64_t p = entry & 0x7fffffff;
     const bool test_first = entry < 0;
     const int32_t* set0;
     int ns0;
@@ -679,7 +682,7 @@ __global__ __launch_bounds__(64) void k_expand(FitArgs a)
           if (!ok && !EXACT) {
             if (lane == 0) {
               a.L.xq_exact[atomicAdd(nexact, 1)] = it;
-              if (entry & 0x40000000) atomicAdd(a.L.status + 4, -1);  // counted once
+              if (tested) atomicAdd(a.L.status + 4, -1);  // counted once
             }
             deferred = true;
             break;

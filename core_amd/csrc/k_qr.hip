@@ -471,8 +471,8 @@ __global__ __launch_bounds__(64, 2) void k_qr_small_lists(FitArgs a)
 // The reference's rank test of the initial sets that the fast forms could not
 // certify (xq entries with bit 31), before the expansion: six sets a wave.
 // A set of full rank becomes the patch's set; any other goes on to the
-// expansion without the test (bit 30: tested).  Sets above 32 rows and short
-// ones stay as they are.  Every entry's x_len is set (0: no set yet).
+// expansion without the test (x_len X_TESTED, bit 31 cleared).  Sets above 32
+// rows and short ones stay as they are (x_len 0).
 // (The expansion's own test takes a wave per set, its sums on one lane: 15.9
 // ms for the 452,700 edge sets of a lattice box at n = 40, and 4.5 ms more to
 // queue them one by one; 1.08 ms here.)
@@ -561,13 +561,13 @@ __global__ __launch_bounds__(64, 2) void k_rank_test(FitArgs a)
     if (head) {
       const bool room = off + len <= a.L.x_cap;
       if (len > 0 && !room) atomicOr(a.L.status, ST_XSET_OVERFLOW);
-      a.L.x_len[it] = room ? len : 0;
+      a.L.x_len[it] = len == 0 && act ? X_TESTED : room ? len : 0;
       if (len > 0 && room) {
         a.L.x_patch[it] = (int32_t)p;
         a.L.x_off[it] = off;
         for (int i = 0; i < len; ++i) a.L.x_set[off + i] = set[i];
       }
-      if (act && !ok) a.L.xq[it] = (int32_t)(p | 0x40000000);
+      if (act && !ok) a.L.xq[it] = (int32_t)p;
     }
     const uint64_t tested = __ballot(head && act);
     if (lane == 0 && tested) atomicAdd(a.L.status + 4, __popcll(tested));
