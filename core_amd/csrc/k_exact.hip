@@ -7,8 +7,9 @@
 // reflectors V (NT x m) in LDS, its sequential sums on one lane, its updates
 // on all; lane j keeps row j of Q in registers and only its first NT entries
 // survive to the solve.  (The arithmetic is k_qr.hip's, whose mapping is the
-// faster one; these lists are short and their lengths known to the device
-// alone.)
+// faster one, but plans its launches by set counts that the host knows.  On
+// most meshes these lists are short; on an undistorted order-2 box nearly every
+// patch is here.)
 #include "exact_common.h"
 #include "fit_common.h"
 
@@ -291,7 +292,8 @@ __device__ __forceinline__ void exact_fit(const FitArgs& a, int bucket, double* 
     // Q rows: q_j = e_j, then reflect_rows for k = 0..NT-1 (mth/mthQR.cc:65-80)
 #pragma unroll 1
     for (int rb = 0; rb < MMAX; rb += LANES) {
-      const int j = rb + gl;
+      int j = rb + gl;
+      asm volatile("" : "+v"(j));  // its comparisons stay inside the loop (hoisted, they spill)
       double qr[MMAX];
 #pragma unroll
       for (int l = 0; l < MMAX; ++l) qr[l] = (l == j) ? 1.0 : 0.0;
@@ -864,24 +866,42 @@ __global__ __launch_bounds__(64) void k_exact_big(FitArgs a, double* ws)
 
 inline unsigned grid_for(int64_t n, int per) { return (unsigned)((n + per - 1) / per); }
 
-// The lists above 32 rows in one launch (their lengths are the device's, and
-// mostly zero).
-template <int NT, int MODE>
-__global__ __launch_bounds__(64, 1) void k_exact_fit(FitArgs a)
+// The lists above 32 rows, whose lengths only the device knows.  Up to 96 rows
+// two waves per SIMD fit (253 VGPRs, 18.8 KB of LDS), above one (34.6 KB): the
+// lists of an undistorted box at n = 40 (462,528 sets, nine in ten of 36 to 72
+// rows) take 22.2 ms in two launches, 38.2 in one that holds them all to one
+// wave.  A mesh of up to LISTS_TOGETHER patches has a SIMD for every set, so
+// there the second launch (5 us) would buy nothing.
+enum { ROWS_TO_96 = 1, ROWS_ABOVE_96 = 2, ROWS_ALL = 3 };
+constexpr int64_t LISTS_TOGETHER = 1024;
+
+template <int NT, int MODE, int ROWS>
+__global__ __launch_bounds__(64, ROWS == ROWS_TO_96 ? 2 : 1) void k_exact_fit(FitArgs a)
 {
-  constexpr int SM = exact_lds(NT, 192);
+  constexpr int SM = exact_lds(NT, ROWS == ROWS_TO_96 ? 96 : 192);
   __shared__ double sm[SM];
   static_assert(NSMALL == 3 && NBUCKET == 7, "the buckets below");
-  exact_fit<NT, 64, 64, MODE>(a, 3, sm);
-  exact_fit<NT, 96, 64, MODE>(a, 4, sm);
-  exact_fit<NT, 128, 64, MODE>(a, 5, sm);
-  exact_fit<NT, 192, 64, MODE>(a, 6, sm);
+  if constexpr (ROWS & ROWS_TO_96) {
+    exact_fit<NT, 64, 64, MODE>(a, 3, sm);
+    exact_fit<NT, 96, 64, MODE>(a, 4, sm);
+  }
+  if constexpr (ROWS & ROWS_ABOVE_96) {
+    exact_fit<NT, 128, 64, MODE>(a, 5, sm);
+    exact_fit<NT, 192, 64, MODE>(a, 6, sm);
+  }
 }
 
 template <int NT, int MODE>
 int fit_lists(const FitArgs& a, hipStream_t s)
 {
-  k_exact_fit<NT, MODE><<<(unsigned)std::min<int64_t>(a.shape.exact_blocks, a.npatch), 64, 0, s>>>(a);
+  const int64_t most = std::min<int64_t>(a.shape.exact_blocks, a.npatch);
+  if (a.npatch <= LISTS_TOGETHER) {
+    k_exact_fit<NT, MODE, ROWS_ALL><<<(unsigned)most, 64, 0, s>>>(a);
+  } else {
+    // (few sets have more than 96 rows: a wave for every SIMD)
+    k_exact_fit<NT, MODE, ROWS_TO_96><<<(unsigned)most, 64, 0, s>>>(a);
+    k_exact_fit<NT, MODE, ROWS_ABOVE_96><<<(unsigned)std::min<int64_t>(most, 1024), 64, 0, s>>>(a);
+  }
   return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "exact fit launch failed");
 }
 
