@@ -52,8 +52,7 @@ enum {
   ST_PATCH_FAIL = 1,     // "all hope is lost"
   ST_TOO_LARGE = 2,      // a set exceeded BIG_MMAX rows, or an expansion 192
   ST_XSET_OVERFLOW = 4,  // expanded-set storage too small
-  ST_INTERNAL = 8,
-  ST_ILLCOND = 16        // a patch too ill-conditioned for the FP64 fallback
+  ST_INTERNAL = 8
 };
 
 // x_len of an item without a set whose initial set k_rank_test has found to
@@ -74,8 +73,7 @@ struct Lists {
   int32_t* xq_exact;         // queued patches whose expansion needs the exact
                              // rank test (same encoding as xq); its count
                              // follows the status word
-  int32_t* fbq;              // fast forms: FP64 fallback queue; bit 31: an
-                             // expanded item rather than a patch id
+  int32_t* fbq;              // refined form: the fallback's patches
   int32_t* big;              // sets of more than 192 (at most BIG_MMAX) rows
                              // for the exact kernel k_exact_big; bit 31: an
                              // expanded item, bit 30: rank not yet decided.
@@ -135,14 +133,15 @@ constexpr int TILE_SORT_CAP = 2048;  // candidate tets a tile build sorts
 constexpr int TILE_B = 64;           // lanes per tile: one wave, so a tile's
                                      // barriers never wait on other waves
 // tets a tile union may hold: two per lane (the staging and its prefetch
-// take a lane's two tets), 12.8 KB of LDS at 4 points per tet
+// take a lane's two tets), 13.8 KB of LDS at 4 points per tet
 constexpr int TILE_MAX_UNION = 2 * TILE_B;
 
 struct FitArgs {
   LaunchShape shape;
   MeshView m;
   TileView tiles;
-  int fast;        // fast forms: one regular list, one expanded list
+  int fast;        // fast forms: no classified lists (the regular pass walks
+                   // every patch, the expanded fit the expansion queue)
   int q;           // points per element
   int nc;          // components
   int64_t npatch;  // nv (+ ne)

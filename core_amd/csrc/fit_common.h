@@ -14,11 +14,11 @@
 namespace sprg {
 
 // What a fit pass decides for a patch.  ACT_EXACT: the exact path decides
-// the rank (and expands); ACT_FALLBACK: an FP64 pass refits it; ACT_REFIT:
-// the exact kernel refits the certified set with the reference's
-// arithmetic; ACT_BIG: the same for a set above 192 rows (k_exact_big);
-// ACT_ILLCOND: no form here can fit it.
-enum { ACT_SOLVE = 0, ACT_EXACT = 1, ACT_FALLBACK = 2, ACT_ILLCOND = 3, ACT_NONE = 4, ACT_REFIT = 5, ACT_BIG = 6 };
+// the rank (and expands); ACT_REFIT: the exact kernel refits the certified set
+// with the reference's arithmetic; ACT_BIG: the same for a set above 192 rows
+// (k_exact_big); ACT_FALLBACK: above those kernels' 512 rows, the refined
+// solution as it is (k_fast.hip).
+enum { ACT_SOLVE = 0, ACT_EXACT = 1, ACT_FALLBACK = 2, ACT_NONE = 4, ACT_REFIT = 5, ACT_BIG = 6 };
 
 // Appends v to the big list (count: status[3]); every lane of the wave
 // calls it.

@@ -22,8 +22,8 @@
 // margin and was computed without heavy cancellation (pivot / diagonal >=
 // tau_rank).  Anything else goes to the exact FP64 path (k_expand tests the
 // initial set with the reference's arithmetic before growing it).  Certified
-// patches whose smallest pivot ratio is below tau_acc go to the exact kernel
-// (the fallback, above its rows).  Three passes over the rows: Gram, refinement, weighted sum;
+// patches whose smallest pivot ratio is below tau_acc go to the exact kernel.
+// Three passes over the rows: Gram, refinement, weighted sum;
 // sample positions are recomputed in each (affine in the four vertices for a
 // straight-sided mesh, the Lagrange-2 map otherwise).
 #include "device.h"
@@ -132,7 +132,8 @@ __device__ __forceinline__ void sample_d(const MeshView& m, const Geo<P2MAP>& g,
   d[2] = x[2] - xn[2];
 }
 
-// SRC_FALLBACK: poor sets of more rows than the exact kernels take.
+// SRC_FALLBACK: certified sets of more rows than the exact kernels take whose
+// refinement the regular pass found unsettled; the refined solution stands.
 // SRC_LEFTOVER: the initial sets of the patches outside every tile of the
 // tiled pass (k_tile.hip), with the regular pass's decisions.
 enum { SRC_REGULAR = 0, SRC_EXPANDED = 1, SRC_FALLBACK = 2, SRC_LEFTOVER = 4 };
@@ -234,7 +235,8 @@ __device__ __forceinline__ void fit_threads(const FitArgs& a, int src, float tau
       }
     }
     // Short sets and uncertified ranks: the exact path decides (bit 31: test
-    // the initial set before growing it).  Below tau_acc the exact kernel
+    // the initial set before growing it).  Below tau_acc (an expanded set; a
+    // regular one is not certified there) or unsettled, the exact kernel
     // refits the patch (normal equations square the condition number; the
     // reference's Householder arithmetic reproduces its own answer), when the
     // set fits the exact kernel's rows.
@@ -242,9 +244,8 @@ __device__ __forceinline__ void fit_threads(const FitArgs& a, int src, float tau
     const int poor = bucket < NBUCKET      ? ACT_REFIT
                      : ns * q <= BIG_MMAX  ? ACT_BIG
                      : src != SRC_FALLBACK ? ACT_FALLBACK
-                     // more rows than the exact kernels take: the refined
-                     // FP64 solve, unless hopeless
-                     : min_ratio >= 1e-13f ? ACT_SOLVE : ACT_ILLCOND;
+                     // more rows than the exact kernels take
+                                           : ACT_SOLVE;
     int act = ACT_NONE;
     if (short_set)
       act = ACT_EXACT;
@@ -303,7 +304,6 @@ __device__ __forceinline__ void fit_threads(const FitArgs& a, int src, float tau
       wave_append(b, act == ACT_REFIT ? bucket : -1, a.L.count + b, a.L.items[b],
                   expanded ? (int32_t)(id | 0x80000000u) : (int32_t)p);
     big_append(act == ACT_BIG, a.L, expanded ? (int32_t)(id | 0x80000000u) : (int32_t)p);
-    if (act == ACT_ILLCOND) atomicOr(a.L.status, ST_ILLCOND);
     if (act != ACT_SOLVE) continue;
     // weighted sum, centred on the first sample
     double v[NC], b0[NC];

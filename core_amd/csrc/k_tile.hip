@@ -22,7 +22,7 @@
 //     shuffles, after which every lane of the group holds the same sums (an
 //     FP addition is commutative, so a+b and b+a round alike);
 //   - the decisions (rank certificate, conditioning, routes to the
-//     expansion, the FP64 fallback or the exact refit) are those of the
+//     expansion or the exact refit) are those of the
 //     thread-per-patch regular pass, made by the group's rank-0 lane;
 //   - the IP values are read from HBM in the weighted sum, a tet's q x nc
 //     block contiguous.

@@ -784,8 +784,8 @@ bool valid_form(int form) { return form == SPRG_FP64 || form == SPRG_FP32R || fo
 // synchronisation, counters cleared by a kernel rather than a memset node),
 // so the sequence can be captured into a HIP graph.  FP64 form: classify ->
 // exact fit of the initial sets -> expansion -> exact fit of the expanded
-// sets.  Fast forms: fit of every patch -> expansion -> fit of the expanded
-// sets -> fallback -> exact refits.  marks: record the phase events.
+// sets.  Fast forms: fit of every patch -> rank test -> expansion -> fit of the
+// expanded sets -> fallback (refined form) -> exact refits.  marks: record the phase events.
 // qr_ws: the exact fits' workspace (FP64 form).
 int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, void* qr_ws, size_t qr_bytes, hipStream_t s, bool marks)
 {
@@ -819,8 +819,9 @@ int enqueue_recover(sprg_mesh* m, const FitArgs& a, int form, void* qr_ws, size_
   if (marks) m->mark(2);
   if (fast) {
     if ((rc = launch_fast_fit(a, nterms, form, 1, s))) return rc;
-    // the fallback: sets above the exact kernels' rows
-    if ((int64_t)m->max_set * a.q > BIG_MMAX && (rc = launch_fast_fit(a, nterms, form, 2, s))) return rc;
+    // the fallback: unsettled refinements of sets above the exact kernels' rows
+    if (form == SPRG_FP32R && (int64_t)m->max_set * a.q > BIG_MMAX)
+      if ((rc = launch_fast_fit(a, nterms, form, 2, s))) return rc;
     // poorly conditioned sets: the reference's arithmetic
     if ((rc = launch_qr_lists(a, nterms, 2, s))) return rc;
   } else {
@@ -866,9 +867,6 @@ int status_code(sprg_mesh* m, int32_t st, bool* retry)
                      "SPR: a patch set needs more than %d sample rows, or a set that must grow has more than %d",
                      BIG_MMAX, bucket_rows(NBUCKET - 1));
   if (st & ST_INTERNAL) return sprg_fail(SPRG_EINTERNAL, "SPR: inconsistent rank decision");
-  if (st & ST_ILLCOND)
-    return sprg_fail(SPRG_EUNSUPPORTED,
-                     "SPR: a patch is too ill-conditioned for the fast forms; use SPRG_FP64");
   return 0;
 }
 

@@ -180,8 +180,9 @@ class Mesh:
 
     def last_stats(self):
         """Patch routes of the last recovery: patches, queued for the exact
-        rank test / expansion, expanded sets, FP64 fallback refits, status,
-        queued patches whose expansion needed the reference's rank test."""
+        rank test / expansion, expanded sets, fp32r patches above 512 sample
+        rows kept with an unsettled refinement, status, queued patches whose
+        expansion needed the reference's rank test, sets above 192 rows."""
         st = np.zeros(7, np.int64)
         _lib.lib().sprg_mesh_last_stats(self.handle, st.ctypes.data, 7)
         return dict(zip(["patches", "queued_exact", "expanded", "fallback", "status", "exact_tested",

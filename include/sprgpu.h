@@ -102,8 +102,9 @@ int sprg_mesh_counts(sprg_mesh* mesh, int64_t* counts);
 int sprg_mesh_phase_times(sprg_mesh* mesh, double* ms, int n);
 /* Patch routes of the last recovery on the mesh: [0] patches, [1] patches
  * queued for the exact rank test / expansion, [2] expanded sets fitted,
- * [3] patches refitted by the fast forms' fallback
- * (poorly conditioned sets of more than 512 rows), [4] status bits,
+ * [3] patches of SPRG_FP32R with more than 512 sample rows (more than the
+ * exact kernels refit) kept with a refinement that had not settled, [4] status
+ * bits,
  * [5] queued patches whose expansion needed the reference's rank test,
  * [6] sets above 192 sample rows fitted by the large-set kernel.
  * Writes min(n, 7) values and returns 7.  No reference counterpart. */

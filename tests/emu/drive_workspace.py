@@ -2,7 +2,7 @@
 (tests/emu/build.py): two host threads on one context, and a device that
 grants only part of what is asked for.  The meshes are P1 stars, whose centre
 vertex has more than 32 rows, so that its fit takes the three-launch path
-through the workspace.  Started by tests/test_emu_workspace.py in a child
+through the workspace; "large" takes a star beyond the exact kernels' rows.  Started by tests/test_emu_workspace.py in a child
 process with AddressSanitizer preloaded, with one check's name."""
 import ctypes
 import os
@@ -161,7 +161,35 @@ def refused(ctx):
     _lib.check(L.sprg_ctx_destroy(fresh))
 
 
-CHECKS = {"threads": threads, "refused": refused}
+def large(ctx):
+    # a vertex of 136 tets at four points per tet, 544 rows: more than the exact
+    # kernels take, so the exact form refuses it and the fast forms solve it
+    # where its rank is certain and refuse it where it is not
+    tv, xyz = smb_util.star(70)
+    for skew, certain in ((1.0, True), (1e-4, False)):
+        x = xyz.copy()
+        x[:, 2] = x[:, 0] + skew * x[:, 2]  # pivot ratio about the skew squared
+        h = mesh.HostMesh(tv, x, 1)
+        om = O.Mesh(h.tv, h.xyz, 1)
+        m = vp()
+        _lib.check(L.sprg_mesh_create(ctx, h.nv, h.nt, 0, P(h.tv), None, P(h.xyz), 1, ctypes.byref(m)))
+        _lib.check(L.sprg_mesh_set_shape(m, SHAPE, 5))
+        ip = np.ascontiguousarray(workloads.strain_field(h.ip_points(2)))
+        ref = O.recover(om, ip)
+        for form in (0, 1, 2):
+            out = np.full((h.nv, 9), np.nan)
+            rc = L.sprg_recover(m, 2, 9, P(ip), P(out), form)
+            st = np.zeros(7, np.int64)
+            L.sprg_mesh_last_stats(m, P(st), 7)
+            if form == 0 or not certain:
+                check("544 rows, skew %g, form %d: refused" % (skew, form), rc == _lib.SPRG_EUNSUPPORTED)
+            else:
+                ok = rc == 0 and np.abs(out - ref).max() <= 1e-9 * np.abs(ref).max()
+                check("544 rows, skew %g, form %d: solved, settled" % (skew, form), ok and st[3] == 0)
+        L.sprg_mesh_destroy(m)
+
+
+CHECKS = {"threads": threads, "refused": refused, "large": large}
 
 if __name__ == "__main__":
     ctx = vp()

@@ -13,7 +13,7 @@ from test_emu_cpu import _asan  # noqa: E402
 
 
 @pytest.mark.skipif(_asan() is None, reason="g++ with AddressSanitizer not available")
-@pytest.mark.parametrize("what", ["threads", "refused"])
+@pytest.mark.parametrize("what", ["threads", "refused", "large"])
 def test_emulated_workspace(what):
     import build as emu_build
 
