@@ -854,9 +854,9 @@ int status_code(sprg_mesh* m, int32_t st, bool* retry)
 {
   *retry = false;
   if (st & ST_XSET_OVERFLOW) {
-    int64_t cap = 2 * m->xset_cap;
-    int rc = m->xset.ensure(sizeof(int32_t) * cap);
-    if (rc) return rc;
+    const int64_t cap = 2 * m->xset_cap;
+    m->xset_cap = 0;  // a refused allocation leaves no storage: the next call makes it anew
+    if (int rc = m->xset.ensure(sizeof(int32_t) * cap)) return rc;
     m->xset_cap = cap;
     *retry = true;
     return 0;
