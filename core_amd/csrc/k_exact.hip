@@ -869,23 +869,27 @@ inline unsigned grid_for(int64_t n, int per) { return (unsigned)((n + per - 1) /
 // The lists above 32 rows, whose lengths only the device knows.  Up to 96 rows
 // two waves per SIMD fit (253 VGPRs, 18.8 KB of LDS), above one (34.6 KB): the
 // lists of an undistorted box at n = 40 (462,528 sets, nine in ten of 36 to 72
-// rows) take 22.2 ms in two launches, 38.2 in one that holds them all to one
-// wave.  A mesh of up to LISTS_TOGETHER patches has a SIMD for every set, so
-// there the second launch (5 us) would buy nothing.
-enum { ROWS_TO_96 = 1, ROWS_ABOVE_96 = 2, ROWS_ALL = 3 };
-constexpr int64_t LISTS_TOGETHER = 1024;
+// rows) take 22.5 ms in two launches, 38.2 in one that holds them all to one
+// wave.  Up to FEW sets of up to 96 rows have a SIMD each as it is: then the
+// second launch takes them beside the larger ones, and the first is empty (a
+// launch lasts as long as one set's chain of sums, some 20 us).  Either grid
+// is what the chip holds at once.
+constexpr int FEW = 1024;
 
-template <int NT, int MODE, int ROWS>
-__global__ __launch_bounds__(64, ROWS == ROWS_TO_96 ? 2 : 1) void k_exact_fit(FitArgs a)
+template <int NT, int MODE, bool ALL>
+__global__ __launch_bounds__(64, ALL ? 1 : 2) void k_exact_fit(FitArgs a)
 {
-  constexpr int SM = exact_lds(NT, ROWS == ROWS_TO_96 ? 96 : 192);
+  constexpr int SM = exact_lds(NT, ALL ? 192 : 96);
   __shared__ double sm[SM];
   static_assert(NSMALL == 3 && NBUCKET == 7, "the buckets below");
-  if constexpr (ROWS & ROWS_TO_96) {
+  int n64, n96;
+  fit_list<MODE>(a, 3, &n64);
+  fit_list<MODE>(a, 4, &n96);
+  if ((n64 + n96 <= FEW) == ALL) {
     exact_fit<NT, 64, 64, MODE>(a, 3, sm);
     exact_fit<NT, 96, 64, MODE>(a, 4, sm);
   }
-  if constexpr (ROWS & ROWS_ABOVE_96) {
+  if constexpr (ALL) {
     exact_fit<NT, 128, 64, MODE>(a, 5, sm);
     exact_fit<NT, 192, 64, MODE>(a, 6, sm);
   }
@@ -895,13 +899,8 @@ template <int NT, int MODE>
 int fit_lists(const FitArgs& a, hipStream_t s)
 {
   const int64_t most = std::min<int64_t>(a.shape.exact_blocks, a.npatch);
-  if (a.npatch <= LISTS_TOGETHER) {
-    k_exact_fit<NT, MODE, ROWS_ALL><<<(unsigned)most, 64, 0, s>>>(a);
-  } else {
-    // (few sets have more than 96 rows: a wave for every SIMD)
-    k_exact_fit<NT, MODE, ROWS_TO_96><<<(unsigned)most, 64, 0, s>>>(a);
-    k_exact_fit<NT, MODE, ROWS_ABOVE_96><<<(unsigned)std::min<int64_t>(most, 1024), 64, 0, s>>>(a);
-  }
+  if (a.npatch > FEW) k_exact_fit<NT, MODE, false><<<(unsigned)std::min<int64_t>(most, 2048), 64, 0, s>>>(a);
+  k_exact_fit<NT, MODE, true><<<(unsigned)std::min<int64_t>(most, 1024), 64, 0, s>>>(a);
   return hipGetLastError() == hipSuccess ? 0 : sprg_fail(SPRG_EHIP, "exact fit launch failed");
 }
 

@@ -357,8 +357,8 @@ __device__ __forceinline__ void sum8(double* v)
 // thread per set takes as long as its tets' chain of loads and sums, however
 // few the sets (35 us for some hundred; 12 here).  Up to SETS_GROUPED queued
 // sets, a wave of them for every SIMD; with more the threads fill the chip by
-// themselves and do not repeat the factorisation (349 us at 452,700 queued
-// sets of mostly six tets; 714 by groups).
+// themselves and do not repeat the factorisation (349 us at the 452,700 queued
+// sets of an undistorted box, grown to 5-18 tets; 714 by groups).
 constexpr int64_t SETS_GROUPED = 65536;
 
 template <int NT, int NC, bool P2MAP>

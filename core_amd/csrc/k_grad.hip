@@ -23,9 +23,9 @@
 // A one-point rule has nothing to share: a lane per tet, 256 to a block,
 // loads its nodes itself, and the results leave the same way.
 // Measured (calls on an order-2 mesh and field, four points): vector fields
-// on 5.3M tets 0.73 -> 0.67 ms, the vector ALU 75% busy with the 560 FP64
+// on 5.3M tets 0.77 -> 0.69 ms, the vector ALU 75% busy with the 560 FP64
 // operations a point needs and the address unit 78%; matrix fields on 384k
-// tets 0.245 -> 0.120 ms, 2.9 TB/s of stores in the kernel (a thread per
+// tets 0.245 -> 0.131 ms, 2.9 TB/s of stores in the kernel (a thread per
 // point with run-time orders and 27 strided stores before).
 #include "device.h"
 #include "spr_math.h"
@@ -41,7 +41,7 @@ constexpr int grad_points(int ipo) { return ipo <= 1 ? 1 : ipo == 2 ? 4 : 5; }
 constexpr int grad_tets(int ipo) { return ipo <= 1 ? 256 : 64; }  // per block
 constexpr int grad_threads(int ipo) { return grad_tets(ipo) * grad_points(ipo); }
 // waves per SIMD asked for: matrix fields' 27 sums take 144 VGPRs, three
-// waves; four, with ten of them spilled, take 120 us instead of 125
+// waves; four, with ten of them spilled, take 131 us a call instead of 134
 constexpr int grad_waves(int ipo, int nc) { return ipo == 2 && nc == 9 ? 4 : 1; }
 
 template <int MO, int FO, int IPO, int NCIN>

@@ -1,7 +1,7 @@
 """Sets that grow above 32 rows in the exact form and refits of more than 32
-rows in the fast forms (csrc/k_exact.hip, k_exact_fit): up to 1,024 patches one
-launch takes every list, above it one takes the sets of up to 96 rows and one
-the larger.  All values are the oracle's, bit for bit.
+rows in the fast forms (csrc/k_exact.hip, k_exact_fit): up to 1,024 sets of at
+most 96 rows are fitted beside the larger ones in one launch (the only one up to
+1,024 patches), more of them by a launch of their own.  All values are the oracle's, bit for bit.
 """
 import numpy as np
 import pytest
