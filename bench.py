@@ -348,8 +348,8 @@ def main():
                            "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                            "frac": fit_flops(T, V, E) / (fit_ms / 1e3) / 1e12 / FP64_PEAK_TFLOPS,
                            "flops": fit_flops(T, V, E),
-                           "note": "the same launch priced by its algorithmic FP64 flops, the bound it "
-                                   "is held by (its HBM traffic moves at a fraction of peak)"}
+                           "note": "the same launch priced by its algorithmic FP64 flops (what holds it "
+                                   "is its vector caches, an access nearly every cycle)"}
                           if args.form == "fp64f" else None),
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic_of(args.form),

@@ -1323,7 +1323,7 @@ extern "C" int sprg_patch_sets(sprg_mesh* m, int ip_order, int64_t* set_off, int
 // that mostly wait on their own latency, so this many recorded graphs run side
 // by side, each on a stream of its own (as many as a process has hardware
 // queues; more would share them).  256 jittered boxes of 1,296 to 384,000
-// tets: a replay takes 36 ms against 93 ms as one chain (fp64f).
+// tets: a replay takes 31 ms against 93 ms as one chain (fp64f).
 constexpr int BATCH_LANES = 4;
 // a pipeline's fixed time in tets of throughput (about 0.2 ms at 1.5e9 tets/s)
 constexpr int64_t BATCH_LAUNCH_TETS = 300000;
